@@ -147,88 +147,103 @@ hipError_t launch_bin(const BinArgs& a, hipStream_t s) {
 }
 
 // ============================================================== potential
-// Per-Z constants, host side.  vatom (U.cu:160-193):
-//   V(r) = sum_i A_i exp2(-B_i r) / r + sum_i C_i exp2(-D_i r^2)
-//   A = 150.4121417 a, B = 2 pi sqrt(b) log2 e, C = 266.5157269 c d^-1.5,
-//   D = pi^2 / d log2 e
-// vzatom2 (U.cu:119-152):
-//   Vz(r) = sum_i A'_i K0(B'_i r) + sum_i C'_i exp2(-D_i r^2)
-//   A' = 300.8242834 a, B' = 2 pi sqrt(b), C' = 150.4121417 c / d
-void kirkland_transform(const float* fp, float* zt) {
-  const double pi = 3.141592654, l2e = 1.4426950408889634;
-  for (int z = 0; z < 103; ++z) {
-    const float* p = fp + z * 12;
-    float* o = zt + z * 24;
-    for (int i = 0; i < 3; ++i) {
-      double a = p[2 * i], b = p[2 * i + 1], c = p[6 + 2 * i], d = p[6 + 2 * i + 1];
-      o[2 * i] = (float)(150.4121417 * a);
-      o[2 * i + 1] = (float)(2.0 * pi * std::sqrt(b) * l2e);
-      o[6 + 2 * i] = (float)(266.5157269 * c * std::pow(d, -1.5));
-      o[6 + 2 * i + 1] = (float)(pi * pi / d * l2e);
-      o[12 + 2 * i] = (float)(300.8242834 * a);
-      o[12 + 2 * i + 1] = (float)(2.0 * pi * std::sqrt(b));
-      o[18 + 2 * i] = (float)(150.4121417 * c / d);
-      o[18 + 2 * i + 1] = (float)(pi * pi / d * l2e);
-    }
-  }
-}
+// Radial tables.  The potential of an atom depends on the squared distance
+// alone: vatom (U.cu:160-193)
+//   V(r) = sum_i A_i exp(-B_i r) / r + sum_i C_i exp(-D_i r^2)
+//   A = 150.4121417 a, B = 2 pi sqrt(b), C = 266.5157269 c d^-1.5, D = pi^2 / d
+// and vzatom2 (U.cu:119-152)
+//   Vz(r) = sum_i A'_i K0(B_i r) + sum_i C'_i exp(-D_i r^2)
+//   A' = 300.8242834 a, C' = 150.4121417 c / d,
+// both constant for r <= 0.25 A and cut off at r^2 = 5 A^2.  Evaluated
+// directly a sample costs six exponentials, a square root and a reciprocal
+// at a quarter of the FP32 rate each (57 issue slots; the potential kernels
+// were bound by them).  Each species gets instead a piecewise cubic in
+// x = r^2, fitted in FP64: 32 intervals per octave of [1/16, 5), so the
+// interval is the top bits of x and the local coordinate the rest, and one
+// interval of zeros from 5 on, which is where the cutoff lands (5 is an
+// interval's edge, so r^2 < 5 is decided exactly).  Over all 103 species the
+// cubic is within 5.2e-7 relative of the FP64 value (1.0e-7 rms), the direct
+// FP32 form within 1.3e-6; 16 intervals per octave would leave 7e-6.
+constexpr int VT_OCT = 32, VT_SHIFT = 18;            // intervals per octave; 23 - log2(32) mantissa bits left
+constexpr int VT_N = 6 * VT_OCT + VT_OCT / 4 + 1;    // [1/16, 4), [4, 5), zeros
+constexpr int VT_FIRST = 0x3D800000 >> VT_SHIFT;     // 1/16
+constexpr float VT_LO = 0.0625f, VT_HI = 5.0f;
 
-// The innermost function of the potential kernels: one square root, six
-// base-2 exponentials and a reciprocal per sample, taken as the hardware
-// instructions (about 1 ulp each).  The library forms of sqrtf, exp2f and the
-// division are correctly rounded over the whole range, denormals included,
-// at 82 instructions per sample against about 30 here; their difference is
-// ~1e-7 of the potential.  Exponentials below 2^-126 flush to zero: terms of
-// that size are below the FP32 resolution of the O(1)..O(1e3) V sums.
-__device__ __forceinline__ float vatom_dev(const float* c, float r2) {
-  float r = __builtin_amdgcn_sqrtf(r2);
-  r = fmaxf(r, 0.25f);
-  const float rr = r * r;
-  const float sl = c[0] * __builtin_amdgcn_exp2f(-c[1] * r) + c[2] * __builtin_amdgcn_exp2f(-c[3] * r) +
-                   c[4] * __builtin_amdgcn_exp2f(-c[5] * r);
-  const float sg = c[6] * __builtin_amdgcn_exp2f(-c[7] * rr) + c[8] * __builtin_amdgcn_exp2f(-c[9] * rr) +
-                   c[10] * __builtin_amdgcn_exp2f(-c[11] * rr);
-  return sl * __builtin_amdgcn_rcpf(r) + sg;
-}
-
-// Abramowitz & Stegun 9.8.1-9.8.6 in FP32 (the forms of U.cu:41-111)
-__device__ __forceinline__ float bessi0_dev(float x) {
-  const float ax = fabsf(x);
-  if (ax <= 3.75f) {
-    float t = x / 3.75f;
+// Abramowitz & Stegun 9.8.1-9.8.6 (the forms of U.cu:41-111)
+__device__ double bessk0_f64(double x) {
+  if (x <= 2.0) {
+    double t = x / 3.75, u = x * 0.5;
     t = t * t;
-    return 1.0f + t * (3.5156229f + t * (3.0899424f + t * (1.2067492f + t * (0.2659732f + t * (0.0360768f + t * 0.0045813f)))));
+    u = u * u;
+    const double i0 = 1.0 + t * (3.5156229 + t * (3.0899424 + t * (1.2067492 + t * (0.2659732 + t * (0.0360768 +
+                      t * 0.0045813)))));
+    return -log(x * 0.5) * i0 - 0.57721566 + u * (0.42278420 + u * (0.23069756 + u * (0.03488590 + u * (0.00262698 +
+           u * (0.00010750 + u * 0.00000740)))));
   }
-  const float t = 3.75f / ax;
-  const float s = 0.39894228f + t * (0.01328592f + t * (0.00225319f + t * (-0.00157565f + t * (0.00916281f +
-                  t * (-0.02057706f + t * (0.02635537f + t * (-0.01647633f + t * 0.00392377f)))))));
-  return expf(ax) * s / sqrtf(ax);
+  const double u = 2.0 / x;
+  return exp(-x) / sqrt(x) * (1.25331414 + u * (-0.07832358 + u * (0.02189568 + u * (-0.01062446 + u * (0.00587872 +
+         u * (-0.00251540 + u * 0.00053208))))));
 }
 
-__device__ __forceinline__ float bessk0_dev(float x) {
-  const float ax = fabsf(x);
-  if (ax > 0.f && ax <= 2.0f) {
-    float x2 = ax * 0.5f;
-    x2 = x2 * x2;
-    const float s = -0.57721566f + x2 * (0.42278420f + x2 * (0.23069756f + x2 * (0.03488590f + x2 * (0.00262698f +
-                    x2 * (0.00010750f + x2 * 0.00000740f)))));
-    return -logf(ax * 0.5f) * bessi0_dev(x) + s;
-  } else if (ax > 2.0f) {
-    const float x2 = 2.0f / ax;
-    const float s = 1.25331414f + x2 * (-0.07832358f + x2 * (0.02189568f + x2 * (-0.01062446f + x2 * (0.00587872f +
-                    x2 * (-0.00251540f + x2 * 0.00053208f)))));
-    return expf(-ax) * s / sqrtf(ax);
+// one thread per interval; blockIdx.y: species, blockIdx.z: 0 vatom, 1 vzatom
+__global__ void k_vatom_table(const float* fp, float4* tab) {
+  const int k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= VT_N) return;
+  const int zi = blockIdx.y, proj = blockIdx.z;
+  float4* o = tab + ((long long)proj * gridDim.y + zi) * VT_N + k;
+  if (k == VT_N - 1) {
+    *o = make_float4(0.f, 0.f, 0.f, 0.f);
+    return;
   }
-  return 1.0e20f;
+  const float* p = fp + zi * 12;
+  const double pi = 3.141592654;
+  double A[3], B[3], C[3], D[3];
+  for (int i = 0; i < 3; ++i) {
+    const double a = p[2 * i], b = p[2 * i + 1], c = p[6 + 2 * i], d = p[6 + 2 * i + 1];
+    A[i] = (proj ? 300.8242834 : 150.4121417) * a;
+    B[i] = 2.0 * pi * sqrt(b);
+    C[i] = proj ? 150.4121417 * c / d : 266.5157269 * c / (d * sqrt(d));
+    D[i] = pi * pi / d;
+  }
+  const double x0 = ldexp(1.0 + (double)(k % VT_OCT) / VT_OCT, k / VT_OCT - 4);
+  const double w = ldexp(1.0 / VT_OCT, k / VT_OCT - 4);
+  // cubic through the four Chebyshev nodes (Newton's divided differences)
+  const double n[4] = {0.038060233744356624, 0.30865828381745514, 0.69134171618254486, 0.96193976625564338};
+  double f[4];
+  for (int j = 0; j < 4; ++j) {
+    const double x = x0 + w * n[j], r = sqrt(x);
+    double v = 0.0;
+    for (int i = 0; i < 3; ++i)
+      v += (proj ? A[i] * bessk0_f64(B[i] * r) : A[i] * exp(-B[i] * r) / r) + C[i] * exp(-D[i] * x);
+    f[j] = v;
+  }
+  for (int l = 1; l < 4; ++l)
+    for (int j = 3; j >= l; --j) f[j] = (f[j] - f[j - 1]) / (n[j] - n[j - l]);
+  // Newton form to powers of the node coordinate, then of t = x - x0
+  double c0 = f[3], c1 = 0.0, c2 = 0.0, c3 = 0.0;
+  for (int j = 2; j >= 0; --j) {
+    c3 = c2 - n[j] * c3;
+    c2 = c1 - n[j] * c2;
+    c1 = c0 - n[j] * c1;
+    c0 = f[j] - n[j] * c0;
+  }
+  *o = make_float4((float)c0, (float)(c1 / w), (float)(c2 / (w * w)), (float)(c3 / (w * w * w)));
 }
 
-__device__ __forceinline__ float vzatom_dev(const float* c, float r2) {
-  float r = sqrtf(r2);
-  r = fmaxf(r, 0.25f);
-  const float rr = r * r;
-  const float sl = c[12] * bessk0_dev(c[13] * r) + c[14] * bessk0_dev(c[15] * r) + c[16] * bessk0_dev(c[17] * r);
-  const float sg = c[18] * exp2f(-c[19] * rr) + c[20] * exp2f(-c[21] * rr) + c[22] * exp2f(-c[23] * rr);
-  return sl + sg;
+size_t vatom_table_size() { return (size_t)2 * 103 * VT_N; }
+
+hipError_t launch_vatom_table(const float* fparams, float4* tab, hipStream_t s) {
+  hipLaunchKernelGGL(k_vatom_table, dim3(nblk(VT_N, 64), 103, 2), dim3(64), 0, s, fparams, tab);
+  return hipGetLastError();
+}
+
+// the table's value at r2; base: the species' first entry less VT_FIRST
+template <class T> __device__ __forceinline__ float vt_at(T tab, int base, float r2) {
+  const float x = __builtin_amdgcn_fmed3f(r2, VT_LO, VT_HI);
+  const unsigned b = __float_as_uint(x);
+  const float4 c = tab[base + (int)(b >> VT_SHIFT)];
+  const float t = x - __uint_as_float(b & ~((1u << VT_SHIFT) - 1u));
+  return fmaf(t, fmaf(t, fmaf(t, c.w, c.z), c.y), c.x);
 }
 
 // FP32 distance decisions of the reference kernels (U.cu:637-640, 784, 931):
@@ -270,13 +285,16 @@ template <> struct PotTile<1> { static constexpr int X = 32, Y = 8; };
 template <> struct PotTile<2> { static constexpr int X = 64, Y = 4; };
 template <> struct PotTile<3> { static constexpr int X = 8, Y = 32; };
 constexpr int kPotTiles = 4;
-constexpr int ACAP = 1024;  // atoms staged in LDS per chunk
+constexpr int ACAP = 512;   // atoms staged in LDS per chunk
+constexpr int kTabLds = 4;  // species whose tables fit the LDS stage
 
-// binnedAtomPKernel3 (U.cu:582-653), binnedAtomPKernelConventional3
-// (U.cu:730-795) and binnedAtomPKernelFD (U.cu:883-946).  One workgroup
-// owns a 16x16 pixel tile of one slice; the atoms of every CSR bin within
-// sqrt(5) A of the tile (slab window per mode) are staged through LDS in
-// chunks, then each thread sums its pixel's contributions.
+// what a launch sums per atom: the samples of a slice (modes 0 and 3), the
+// projected potential (mode 1) or one plane (mode 2)
+enum PotKind { POT_SAMPLES = 0, POT_PROJECTED = 1, POT_PLANE = 2 };
+static inline __host__ __device__ constexpr int pot_kind(int mode) {
+  return mode == 1 ? POT_PROJECTED : mode == 2 ? POT_PLANE : POT_SAMPLES;
+}
+
 // the potential arguments as device code reads them from a table in memory
 // (pointers in the global address space, same layout)
 struct PotArgsG {
@@ -284,19 +302,49 @@ struct PotArgsG {
 };
 static_assert(sizeof(PotArgsG) == sizeof(PotArgs), "layouts differ");
 
-// pixel tile (tx, ty) of TX x TY pixels (TX TY = 256 threads) of slice
-// `slice` (relative to first_slice)
-template <int TX, int TY, class A>
-__device__ __forceinline__ void potential_tile(const A& a, int tx, int ty, int slice) {
-  static_assert(TX * TY == 256, "one thread per pixel of a 256-thread workgroup");
-  __shared__ float zt[103 * 24];
-  __shared__ float sx[ACAP], sy[ACAP], sz[ACAP];
-  __shared__ int sZ[ACAP];
-  __shared__ int rs[64], rl[65];
-  __shared__ float zsm[21];  // the slice's z samples (modes 0 and 3), index m
-  const int tid = threadIdx.x;
-  for (int i = tid; i < 103 * 24; i += 256) zt[i] = a.ztab[i];
-  const int ix = tx * TX + (tid % TX), iy = ty * TY + (tid / TX);
+__device__ __forceinline__ float readlane_f(float v, int l) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
+}
+
+// binnedAtomPKernel3 (U.cu:582-653), binnedAtomPKernelConventional3
+// (U.cu:730-795), binnedAtomPKernelFD (U.cu:883-946) and binnedAtomPKernelRS
+// (U.cu:656-727): pixel tile (tx, ty) of TX x TY pixels of slice `slice`
+// (relative to first_slice), one thread per pixel and, with SPLIT 4, four
+// waves per 8 x 8 pixels that share the atoms between them.
+//
+// The bin rows of every slab of the window are gathered in one go (one scan
+// over all of them, one round of atom loads): a workgroup waits for three
+// dependent loads in all, not for three per slab.  Then each wave works on
+// an 8 x 8 pixel patch of its own: its lanes test 64 atoms at a time against
+// the patch and find the samples each can reach, and only those atoms and
+// samples are summed, with the atom in scalar registers.  Lanes out of an
+// atom's reach read the table's zero interval, so there is no divergence.
+// Bound by VALU issue at large grids (13 instructions and a 16-byte LDS read
+// per sample), by those three loads and the launch at small ones.  Per slice,
+// before (slab after slab, transcendentals, a divergent loop per pixel) and
+// now: Si 1024^2 of 0.074 A 114.6 -> 39.9 us, SrTiO3 512^2 of 0.078 A 51.0 ->
+// 19.2, Si 256^2 of 0.085 A 27.9 -> 9.1, 64^2 of 0.2 A 27.2 -> 6.8; one plane
+// of Si at 256^2 16.0 -> 5.6.
+template <int TX, int TY, int SPLIT, int KIND, class A>
+__device__ __forceinline__ void potential_tile(const A& a, int tx, int ty, int slice, float4* tabs) {
+  static_assert(TX * TY * SPLIT == 256, "256-thread workgroups");
+  __shared__ float4 sa[ACAP];      // x, y, z, table base (as int)
+  __shared__ int si[ACAP];
+  __shared__ int wsum[4];
+  __shared__ float red[SPLIT > 1 ? 256 : 1];
+  const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // the wave's patch: 8 x 8 pixels, 16 x 4 in the 64 x 4 tile
+  constexpr int PW = TY % 8 == 0 ? 8 : 16, PH = 64 / PW;
+  const int pt = SPLIT > 1 ? 0 : wv;
+  const int wx = tx * TX + (pt % (TX / PW)) * PW, wy = ty * TY + (pt / (TX / PW)) * PH;
+  const int ix = wx + lane % PW, iy = wy + lane / PW;
+  constexpr int kPart = KIND == POT_PROJECTED ? 103 * VT_N : 0;
+  const bool in_lds = KIND != POT_PLANE && a.nspec > 0;
+  if (in_lds)
+    for (int q = tid; q < a.nspec * VT_N; q += 256) {
+      const int sp = q / VT_N;
+      tabs[q] = a.vtab[kPart + (a.spec[sp] - 1) * VT_N + (q - sp * VT_N)];
+    }
   float zf, h;
   {
 #pragma clang fp contract(off)
@@ -306,7 +354,7 @@ __device__ __forceinline__ void potential_tile(const A& a, int tx, int ty, int s
     zf = (a.mode >= 2) ? a.zplane : h - a.dz * (float)(a.first_slice + slice - phys);
   }
   int k0, k1;
-  if (a.mode == 1) {
+  if constexpr (KIND == POT_PROJECTED) {
     k0 = (int)floorf(h - zf);
     k1 = (int)floorf(h - zf + a.dz) - 1;
   } else {
@@ -324,103 +372,130 @@ __device__ __forceinline__ void potential_tile(const A& a, int tx, int ty, int s
   k1 = min(k1, a.nslab - 1);
   const float offx = a.mode == 2 ? 0.f : a.offx, offy = a.mode == 2 ? 0.f : a.offy;
   const float px = pix_pos(ix, a.ps, offx), py = pix_pos(iy, a.ps, offy);
+  const float bx0 = pix_pos(wx, a.ps, offx), bx1 = pix_pos(wx + PW - 1, a.ps, offx);
+  const float by0 = pix_pos(wy, a.ps, offy), by1 = pix_pos(wy + PH - 1, a.ps, offy);
   // bin window of the tile: every bin that may hold an atom within sqrt(5)
-  const float wx = (a.MaxX - a.MinX) / 50.f, wy = (a.MaxY - a.MinY) / 50.f, reach = 2.2360680f;
+  const float bwx = (a.MaxX - a.MinX) / 50.f, bwy = (a.MaxY - a.MinY) / 50.f, reach = 2.2360680f;
   const float tx0 = offx + (float)(tx * TX) * a.ps, tx1 = offx + (float)(tx * TX + TX - 1) * a.ps;
   const float ty0 = offy + (float)(ty * TY) * a.ps, ty1 = offy + (float)(ty * TY + TY - 1) * a.ps;
-  const int i0 = max(0, (int)floorf((tx0 - reach) / wx) - 1), i1 = min(49, (int)floorf((tx1 + reach) / wx) + 1);
-  const int j0 = max(0, (int)floorf((ty0 - reach) / wy) - 1), j1 = min(49, (int)floorf((ty1 + reach) / wy) + 1);
-  const float h20 = a.dz / 20.0f;
-  // the sample positions depend on the slice only: computed once per
-  // workgroup (each an FP32 division, as the reference takes it) instead of
-  // once per atom and pixel
-  if (tid >= 1 && tid <= 20) zsm[tid] = a.mode == 3 ? (tid <= 10 ? sample_z_rs(zf, tid) : 0.f) : sample_z(zf, tid, a.dz);
+  const int i0 = max(0, (int)floorf((tx0 - reach) / bwx) - 1), i1 = min(49, (int)floorf((tx1 + reach) / bwx) + 1);
+  const int j0 = max(0, (int)floorf((ty0 - reach) / bwy) - 1), j1 = min(49, (int)floorf((ty1 + reach) / bwy) + 1);
+  const int nj = j1 - j0 + 1;
+  const int runs = (i0 <= i1 && nj > 0 && k0 <= k1) ? nj * (k1 - k0 + 1) : 0;
+  // lane m holds sample position m; the lanes past the last sample are out
+  // of every atom's reach
+  const int nsamp = a.mode == 3 ? 10 : 20;
+  const float hs = a.mode == 3 ? 0.1f : a.dz / 20.0f, us = 1.0f / hs;
+  float zl = 3.0e18f;
+  if constexpr (KIND == POT_SAMPLES)
+    if (lane >= 1 && lane <= nsamp) zl = a.mode == 3 ? sample_z_rs(zf, lane) : sample_z(zf, lane, a.dz);
+  // the patch test may err on the side of keeping an atom: FP32 rounding of
+  // positions a thousand angstroms away is 1e-3 A^2 in r^2
+  constexpr float kReach2 = 5.05f;
   float sum = 0.f;
-  __syncthreads();
-  for (int k = k0; k <= k1; ++k) {
-    for (int jb = j0; jb <= j1; jb += 64) {
-      const int nr = min(64, j1 - jb + 1);
-      if (i0 > i1) break;
-      if (tid < 64) {
-        // the first wave loads the window's bin-row runs and scans their
-        // lengths (inclusive, shuffles across the 64 lanes)
-        int len = 0;
-        if (tid < nr) {
-          const int bb = k * 2500 + (jb + tid) * 50;
-          const int r0 = a.start[bb + i0];
-          rs[tid] = r0;
-          len = a.start[bb + i1 + 1] - r0;
+  int seen = 0;  // atoms of the patch so far (SPLIT: atom n goes to wave n % SPLIT)
+  for (int rb = 0; rb < runs; rb += 256) {
+    int len = 0, r0 = 0;
+    if (rb + tid < runs) {
+      const int k = (rb + tid) / nj, j = (rb + tid) - k * nj;
+      const int bb = (k0 + k) * 2500 + (j0 + j) * 50;
+      r0 = a.start[bb + i0];
+      len = a.start[bb + i1 + 1] - r0;
+    }
+    int incl = len;
+    for (int d = 1; d < 64; d <<= 1) {
+      const int v = __shfl_up(incl, d, 64);
+      if (lane >= d) incl += v;
+    }
+    if (lane == 63) wsum[wv] = incl;
+    __syncthreads();
+    int off = incl - len, tot = 0;
+    for (int w = 0; w < 4; ++w) {
+      const int v = wsum[w];
+      off += w < wv ? v : 0;
+      tot += v;
+    }
+    for (int c0 = 0; c0 < tot; c0 += ACAP) {
+      const int cn = min(ACAP, tot - c0);
+      for (int j = max(0, c0 - off); j < len && off + j < c0 + cn; ++j) si[off + j - c0] = r0 + j;
+      __syncthreads();
+      for (int q = tid; q < cn; q += 256) {
+        const int src = si[q], Z = a.bZ[src];
+        int base = (Z - 1) * VT_N + kPart;
+        if (in_lds) {
+          base = 0;
+          for (int sp = 1; sp < a.nspec; ++sp) base = Z == a.spec[sp] ? sp * VT_N : base;
         }
-        for (int d = 1; d < 64; d <<= 1) {
-          const int v = __shfl_up(len, d, 64);
-          if (tid >= d) len += v;
-        }
-        if (tid < nr) rl[tid + 1] = len;
-        if (tid == 0) rl[0] = 0;
+        sa[q] = make_float4(a.bx[src], a.by[src], a.bz[src], __int_as_float(base - VT_FIRST));
       }
       __syncthreads();
-      const int tot = rl[nr];
-      for (int c0 = 0; c0 < tot; c0 += ACAP) {
-        const int cn = min(ACAP, tot - c0);
-        for (int q = tid; q < cn; q += 256) {
-          const int g = c0 + q;
-          // the run holding g: the largest r with rl[r] <= g (rl ascending)
-          int lo = 0, hi = nr - 1;
-          while (lo < hi) {
-            const int mid = (lo + hi + 1) >> 1;
-            if (rl[mid] <= g) lo = mid;
-            else hi = mid - 1;
+      auto atoms = [&](auto tab) {
+        for (int b0 = 0; b0 < cn; b0 += 64) {
+          float4 at = make_float4(0.f, 0.f, 0.f, 0.f);
+          bool hit = false;
+          int mlo = 1, mhi = 0;
+          if (b0 + lane < cn) {
+            at = sa[b0 + lane];
+            const float ex = fmaxf(fmaxf(bx0 - at.x, at.x - bx1), 0.f);
+            const float ey = fmaxf(fmaxf(by0 - at.y, at.y - by1), 0.f);
+            float room = kReach2 - (ex * ex + ey * ey);
+            hit = room > 0.f;
+            if constexpr (KIND == POT_SAMPLES) {
+              // samples with |zf - m hs - z| within the patch's reach, one
+              // more on each side
+              const float hz = __builtin_amdgcn_sqrtf(fmaxf(room, 0.f)), zc = zf - at.z;
+              mlo = max(1, (int)fmaxf(floorf((zc - hz) * us), -1.f) - 1);
+              mhi = min(nsamp, (int)fminf(ceilf((zc + hz) * us), 64.f) + 1);
+              hit = hit && mlo <= mhi;
+            } else if constexpr (KIND == POT_PLANE) {
+              room -= (zf - at.z) * (zf - at.z);
+              hit = room > 0.f;
+            }
           }
-          const int r = lo;
-          const int src = rs[r] + (g - rl[r]);
-          sx[q] = a.bx[src];
-          sy[q] = a.by[src];
-          sz[q] = a.bz[src];
-          sZ[q] = a.bZ[src];
-        }
-        __syncthreads();
-        for (int l = 0; l < cn; ++l) {
-          const float rxy = dist2_xy(px, py, sx[l], sy[l]);
-          if (rxy >= 5.0f) continue;
-          const float* c = zt + (sZ[l] - 1) * 24;
-          if (a.mode == 0) {
-            const float zr = sz[l];
-            // samples m with |zf - m dz / 20 - zr| < sqrt(5 - rxy), widened by
-            // one sample on each side; inside that range each sample takes
-            // the exact FP32 cutoff test, so the set summed is the 20-sample
-            // loop's (the samples outside fail it by more than rounding, and
-            // by far more than the hardware square root's last bit)
-            const float hz = __builtin_amdgcn_sqrtf(5.0f - rxy), u = 20.0f / a.dz;
-            const int mlo = max(1, (int)floorf((zf - zr - hz) * u) - 1);
-            const int mhi = min(20, (int)ceilf((zf - zr + hz) * u) + 1);
-            // the atom's coefficients in registers for all its samples
-            float cr[12];
+          unsigned long long mask = __ballot(hit);
+          while (mask) {
+            const int l = __builtin_ctzll(mask);
+            mask &= mask - 1;
+            if (SPLIT > 1 && (seen++ % SPLIT) != wv) continue;
+            const float ax = readlane_f(at.x, l), ay = readlane_f(at.y, l), az = readlane_f(at.z, l);
+            const int base = __builtin_amdgcn_readlane(__float_as_int(at.w), l);
+            const float rxy = dist2_xy(px, py, ax, ay);
+            if constexpr (KIND == POT_PROJECTED) {
+              sum += vt_at(tab, base, rxy);
+            } else if constexpr (KIND == POT_PLANE) {
+              sum += vt_at(tab, base, dist2_z(rxy, zf, az));
+            } else {
+              const int m0 = __builtin_amdgcn_readlane(mlo, l), m1 = __builtin_amdgcn_readlane(mhi, l);
+              const float dl = zl - az;
+              float s = 0.f;
+              // four samples at a time (their table reads in flight
+              // together); a sample past m1 adds an exact zero
+              for (int m = m0; m <= m1; m += 4) {
+                float v[4];
 #pragma unroll
-            for (int i = 0; i < 12; ++i) cr[i] = c[i];
-            for (int m = mlo; m <= mhi; ++m) {
-              const float r2 = dist2_z(rxy, zsm[m], zr);
-              if (r2 < 5.0f) sum += h20 * vatom_dev(cr, r2);
-            }
-          } else if (a.mode == 1) {
-            sum += vzatom_dev(c, rxy);
-          } else if (a.mode == 3) {  // real-space slab of 1 A, 10 samples
-            const float zr = sz[l];
-            float cr[12];
+                for (int u = 0; u < 4; ++u) {
+                  const float dd = readlane_f(dl, m + u);
+                  v[u] = vt_at(tab, base, fmaf(dd, dd, rxy));
+                }
 #pragma unroll
-            for (int i = 0; i < 12; ++i) cr[i] = c[i];
-            for (int m = 1; m <= 10; ++m) {
-              const float r2 = dist2_z(rxy, zsm[m], zr);
-              if (r2 < 5.0f) sum += 0.1f * vatom_dev(cr, r2);
+                for (int u = 0; u < 4; ++u) s += v[u];
+              }
+              sum = fmaf(hs, s, sum);
             }
-          } else {
-            const float r2 = dist2_z(rxy, zf, sz[l]);
-            if (r2 < 5.0f) sum += vatom_dev(c, r2);
           }
         }
-        __syncthreads();
-      }
-      __syncthreads();  // rs / rl are rewritten by the next window row
+      };
+      if (in_lds) atoms((const float4*)tabs);
+      else atoms(a.vtab);
+      __syncthreads();  // si / sa are rewritten by the next chunk
     }
+    __syncthreads();  // wsum is rewritten by the next runs
+  }
+  if constexpr (SPLIT > 1) {
+    red[tid] = sum;
+    __syncthreads();
+    if (wv != 0) return;
+    sum = ((red[lane] + red[64 + lane]) + red[128 + lane]) + red[192 + lane];
   }
   if (ix >= a.nx || iy >= a.ny) return;
   const long long o = (long long)slice * a.out_sstride + (long long)iy * a.nx + ix;
@@ -435,15 +510,25 @@ __device__ __forceinline__ void potential_tile(const A& a, int tx, int ty, int s
   }
 }
 
-template <int V>
+template <int V, int KIND>
 __global__ void __launch_bounds__(256) k_potential(PotArgs a) {
-  potential_tile<PotTile<V>::X, PotTile<V>::Y>(a, blockIdx.x, blockIdx.y, blockIdx.z);
+  extern __shared__ float4 pot_tabs[];
+  potential_tile<PotTile<V>::X, PotTile<V>::Y, 1, KIND>(a, blockIdx.x, blockIdx.y, blockIdx.z, pot_tabs);
+}
+
+// small launches: 64 pixels per workgroup, its four waves sharing the atoms
+template <int KIND>
+__global__ void __launch_bounds__(256) k_potential_split(PotArgs a) {
+  extern __shared__ float4 pot_tabs[];
+  potential_tile<8, 8, 4, KIND>(a, blockIdx.x, blockIdx.y, blockIdx.z, pot_tabs);
 }
 
 // slice `first` of njobs jobs in one launch: workgroup id -> (job, tile)
 // through the block offsets blk0[0..njobs] (ascending)
+template <int KIND>
 __global__ void __launch_bounds__(256) k_potential_group(const PotArgs* tab, const long long* blk0, int njobs,
                                                          int first) {
+  extern __shared__ float4 pot_tabs[];
   const long long id = blockIdx.x;
   int lo = 0, hi = njobs - 1;
   while (lo < hi) {
@@ -455,22 +540,45 @@ __global__ void __launch_bounds__(256) k_potential_group(const PotArgs* tab, con
   a.first_slice = first;
   const int tx = nblk(a.nx, PT);
   const long long local = id - blk0[lo];
-  potential_tile<PT, PT>(a, (int)(local % tx), (int)(local / tx), 0);
+  potential_tile<PT, PT, 1, KIND>(a, (int)(local % tx), (int)(local / tx), 0, pot_tabs);
 }
 
-template <int V> static hipError_t potential_v(const PotArgs& a, hipStream_t s) {
+// dynamic LDS of a launch: the tables of its species (the one read per atom
+// of a plane comes from the caches)
+template <int KIND> static size_t pot_lds(const PotArgs& a) {
+  return KIND == POT_PLANE ? 0 : a.nspec * VT_N * sizeof(float4);
+}
+
+template <int V, int KIND> static hipError_t potential_v(const PotArgs& a, hipStream_t s) {
   dim3 grid(nblk(a.nx, PotTile<V>::X), nblk(a.ny, PotTile<V>::Y), a.nslices);
-  hipLaunchKernelGGL(k_potential<V>, grid, dim3(256), 0, s, a);
+  hipLaunchKernelGGL((k_potential<V, KIND>), grid, dim3(256), pot_lds<KIND>(a), s, a);
   return hipGetLastError();
+}
+
+template <int KIND> static hipError_t potential_k(const PotArgs& a, hipStream_t s) {
+  // one wave per 8 x 8 pixels leaves SIMDs (1024 on the chip) with fewer than
+  // four waves each below 4096 patches: four waves then share a patch
+  const long long patches = (long long)nblk(a.nx, 8) * nblk(a.ny, 8) * a.nslices;
+  if (patches < 4096) {
+    hipLaunchKernelGGL(k_potential_split<KIND>, dim3(nblk(a.nx, 8), nblk(a.ny, 8), a.nslices), dim3(256),
+                       pot_lds<KIND>(a), s, a);
+    return hipGetLastError();
+  }
+  switch (a.tile) {
+    case 1: return potential_v<1, KIND>(a, s);
+    case 2: return potential_v<2, KIND>(a, s);
+    case 3: return potential_v<3, KIND>(a, s);
+    default: return potential_v<0, KIND>(a, s);
+  }
 }
 
 hipError_t launch_potential(const PotArgs& a, hipStream_t s) {
   if (a.nslices <= 0) return hipSuccess;
-  switch (a.tile) {
-    case 1: return potential_v<1>(a, s);
-    case 2: return potential_v<2>(a, s);
-    case 3: return potential_v<3>(a, s);
-    default: return potential_v<0>(a, s);
+  if (!a.vtab || a.nspec < 0 || a.nspec > kTabLds) return hipErrorInvalidValue;
+  switch (pot_kind(a.mode)) {
+    case POT_PROJECTED: return potential_k<POT_PROJECTED>(a, s);
+    case POT_PLANE: return potential_k<POT_PLANE>(a, s);
+    default: return potential_k<POT_SAMPLES>(a, s);
   }
 }
 
@@ -479,10 +587,13 @@ int potential_tile_variants() { return kPotTiles; }
 int potential_tiles(int nx, int ny) { return nblk(nx, PT) * nblk(ny, PT); }
 
 hipError_t launch_potential_group(const PotArgs* tab, const long long* blk0, int njobs, long long nblocks, int first,
-                                  hipStream_t s) {
+                                  int mode, hipStream_t s) {
   if (njobs <= 0 || nblocks <= 0) return hipSuccess;
-  if (nblocks > 0x7fffffffLL) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_potential_group, dim3((unsigned)nblocks), dim3(256), 0, s, tab, blk0, njobs, first);
+  if (nblocks > 0x7fffffffLL || mode < 0 || mode > 1) return hipErrorInvalidValue;
+  const size_t lds = kTabLds * VT_N * sizeof(float4);
+  const dim3 grid((unsigned)nblocks), block(256);
+  if (mode == 1) hipLaunchKernelGGL(k_potential_group<POT_PROJECTED>, grid, block, lds, s, tab, blk0, njobs, first);
+  else hipLaunchKernelGGL(k_potential_group<POT_SAMPLES>, grid, block, lds, s, tab, blk0, njobs, first);
   return hipGetLastError();
 }
 

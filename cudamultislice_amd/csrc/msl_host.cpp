@@ -175,38 +175,43 @@ void ensure_prop(msl_sim* s, float dz) {
   s->prop_dz = dz;
 }
 
-// generic transform of nbatch waves in place, then the scale
-void gen_fft2(msl_sim* s, float2* w, int nbatch, bool inverse, float scale) {
-  s->gscr.ensure((size_t)nbatch * s->npix());
-  HIPC(launch_gen_fft2(w, s->gscr.p, s->resX, s->resY, nbatch, inverse ? 1 : 0, s->twx.p, s->twy.p, s->stream));
-  if (scale != 1.0f)
-    HIPC(launch_gen_kmul(w, s->resX, s->resY, nbatch, CM_SCALE, nullptr, nullptr, nullptr, nullptr, 0.f, scale,
-                         s->stream));
+// generic rows: dst = (src t) transformed along x (t optional; dst2 an
+// optional second copy)
+void gen_row(msl_sim* s, const float2* src, float2* dst, int nbatch, bool inverse, const float2* t = nullptr,
+             float2* dst2 = nullptr) {
+  GenRowArgs a{};
+  a.src = src; a.dst = dst; a.dst2 = dst2; a.t = t;
+  a.nx = s->resX; a.ny = s->resY; a.nbatch = nbatch; a.inverse = inverse ? 1 : 0;
+  a.len = s->glx;
+  HIPC(launch_gen_row(a, s->stream));
 }
-// w *= (k-space multiplier mul) * scale, one wave (generic grids)
-void gen_kmul(msl_sim* s, float2* w, int mul, float scale) {
-  HIPC(launch_gen_kmul(w, s->resX, s->resY, 1, mul, s->kx.p, s->ky.p, s->px.p, s->py.p, s->kmax, scale, s->stream));
+// generic columns, in place: COL_FWD, COL_INV or COL_FWD_MUL_INV with the
+// k-space factor mul times scale
+void gen_col(msl_sim* s, float2* w, int nbatch, int mode, int mul, double scale) {
+  GenColArgs a{};
+  a.src = w; a.dst = w;
+  a.nx = s->resX; a.ny = s->resY; a.nbatch = nbatch; a.mode = mode; a.mul = mul;
+  a.kx = s->kx.p; a.ky = s->ky.p; a.px = s->px.p; a.py = s->py.p; a.kmax = s->kmax; a.scale = scale;
+  a.len = s->gly;
+  HIPC(launch_gen_col(a, s->stream));
 }
-void copy_wave(msl_sim* s, float2* dst, const float2* src) {
-  if (dst != src)
-    HIPC(hipMemcpyAsync(dst, src, s->npix() * sizeof(float2), hipMemcpyDeviceToDevice, s->stream));
-}
-
 // in-place unnormalised 2D transforms of nbatch waves
-void fft2(msl_sim* s, float2* w, int nbatch, bool inverse, float scale = 1.0f) {
+void fft2(msl_sim* s, float2* w, int nbatch, bool inverse, double scale = 1.0) {
   if (s->generic) {
-    gen_fft2(s, w, nbatch, inverse, scale);
+    if (!inverse) gen_row(s, w, w, nbatch, false);
+    gen_col(s, w, nbatch, inverse ? COL_INV : COL_FWD, CM_SCALE, scale);
+    if (inverse) gen_row(s, w, w, nbatch, true);
     return;
   }
   const long long bs = (long long)s->npix();
   if (!inverse) {
     row(s, ROW_FWD, RM_NONE, row_args(s, w, w, nbatch, bs));
     ColArgs c = col_args(s, w, w, nbatch, bs);
-    c.scale = scale;
+    c.scale = (float)scale;
     col(s, COL_FWD, CM_SCALE, c);
   } else {
     ColArgs c = col_args(s, w, w, nbatch, bs);
-    c.scale = scale;
+    c.scale = (float)scale;
     col(s, COL_INV, CM_SCALE, c);
     row(s, ROW_INV, RM_NONE, row_args(s, w, w, nbatch, bs));
   }
@@ -216,10 +221,9 @@ void fft2(msl_sim* s, float2* w, int nbatch, bool inverse, float scale = 1.0f) {
 void propagate(msl_sim* s, float2* src, float2* dst, float dz) {
   ensure_prop(s, dz);
   if (s->generic) {
-    copy_wave(s, dst, src);
-    gen_fft2(s, dst, 1, false, 1.0f);
-    gen_kmul(s, dst, CM_PROP, s->nf * s->nf);
-    gen_fft2(s, dst, 1, true, 1.0f);
+    gen_row(s, src, dst, 1, false);
+    gen_col(s, dst, 1, COL_FWD_MUL_INV, CM_PROP, s->nfd * s->nfd);
+    gen_row(s, dst, dst, 1, true);
     return;
   }
   const long long bs = (long long)s->npix();
@@ -230,13 +234,17 @@ void propagate(msl_sim* s, float2* src, float2* dst, float dz) {
   row(s, ROW_INV, RM_NONE, row_args(s, dst, dst, 1, bs));
 }
 
-void ensure_ztab(msl_sim* s) {
-  if (s->ztab.p) return;
-  std::vector<float> zt(103 * 24);
-  kirkland_transform(s->fparams.data(), zt.data());
-  s->ztab.ensure(zt.size());
-  HIPC(hipMemcpyAsync(s->ztab.p, zt.data(), zt.size() * sizeof(float), hipMemcpyHostToDevice, s->stream));
+void ensure_vtab(msl_sim* s) {
+  if (s->vtab.p) return;
+  DBuf<float> fp;
+  fp.ensure(s->fparams.size());
+  DBuf<float4> tab;
+  tab.ensure(vatom_table_size());
+  HIPC(hipMemcpyAsync(fp.p, s->fparams.data(), s->fparams.size() * sizeof(float), hipMemcpyHostToDevice, s->stream));
+  HIPC(launch_vatom_table(fp.p, tab.p, s->stream));
   HIPC(hipStreamSynchronize(s->stream));
+  std::swap(s->vtab.p, tab.p);
+  std::swap(s->vtab.n, tab.n);
 }
 
 // LoadAtomFile extents, U.cu:1323-1355
@@ -257,6 +265,15 @@ void set_atoms(msl_sim* s, std::vector<int>&& Z, std::vector<float>&& x, std::ve
   s->MaxY = y[my] + 2; s->MinY = y[ny] - 2;
   s->MaxZ = z[mz] + 2; s->MinZ = z[nz] - 2;
   s->Z = std::move(Z); s->x = std::move(x); s->y = std::move(y); s->z = std::move(z);
+  s->nspec = 0;
+  bool seen[104] = {false};
+  for (int v : s->Z) seen[v] = true;
+  for (int v = 1; v <= 103; ++v)
+    if (seen[v]) {
+      if (s->nspec < 4) s->spec[s->nspec] = v;
+      ++s->nspec;
+    }
+  if (s->nspec > 4) s->nspec = 0;
   s->have_atoms = true;
   s->binned = false;
   s->tds_config = 0;
@@ -360,6 +377,7 @@ void precalc(msl_sim* s) {
   // compat=physical: 2/3 of the Nyquist frequency
   if (s->compat & MSL_COMPAT_PHYSICAL) s->kmax = (2.0f / 3.0f) * std::min(s->hkx[imidx], s->hky[imidy]);
   s->nf = 1.0f / std::sqrt((float)(rx * ry));
+  s->nfd = s->generic ? 1.0 / std::sqrt((double)rx * ry) : (double)s->nf;
   // band pruning is exact when every column N/4 <= x < 3N/4 fails the
   // propagator's |k| < kmax test for any ky (then so does the band limit's)
   s->prune_tiles = band_tiles_lo(rx);
@@ -372,11 +390,31 @@ void precalc(msl_sim* s) {
   HIPC(hipMemcpyAsync(s->ky.p, s->hky.data(), ry * sizeof(float), hipMemcpyHostToDevice, s->stream));
   s->prow.ensure(rx);
   HIPC(make_prop_rows(s->kx.p, s->ky.p, rx, ry, s->kmax, s->prow.p, s->stream));
-  auto tx = twiddles(rx), ty = twiddles(ry);
-  s->twx.ensure(rx);
-  s->twy.ensure(ry);
-  HIPC(hipMemcpyAsync(s->twx.p, tx.data(), rx * sizeof(float2), hipMemcpyHostToDevice, s->stream));
-  HIPC(hipMemcpyAsync(s->twy.p, ty.data(), ry * sizeof(float2), hipMemcpyHostToDevice, s->stream));
+  auto upload = [&](auto& d, const auto& v) {
+    d.ensure(v.size());
+    if (!v.empty()) HIPC(hipMemcpyAsync(d.p, v.data(), v.size() * sizeof(v[0]), hipMemcpyHostToDevice, s->stream));
+  };
+  std::vector<float2> tx, ty;
+  std::vector<double2> wx, cx, fx, wy, cy, fy;
+  if (s->generic && s->glx.n == rx && s->gly.n == ry) {
+    // the tables depend on the sides alone
+  } else if (s->generic) {
+    gen_tables(rx, wx, cx, fx);
+    gen_tables(ry, wy, cy, fy);
+    upload(s->gtwx, wx);
+    upload(s->gchx, cx);
+    upload(s->gfix, fx);
+    upload(s->gtwy, wy);
+    upload(s->gchy, cy);
+    upload(s->gfiy, fy);
+    s->glx = GenLen{rx, (int)wx.size(), s->gtwx.p, cx.empty() ? nullptr : s->gchx.p, cx.empty() ? nullptr : s->gfix.p};
+    s->gly = GenLen{ry, (int)wy.size(), s->gtwy.p, cy.empty() ? nullptr : s->gchy.p, cy.empty() ? nullptr : s->gfiy.p};
+  } else {
+    tx = twiddles(rx);
+    ty = twiddles(ry);
+    upload(s->twx, tx);
+    upload(s->twy, ty);
+  }
   HIPC(hipStreamSynchronize(s->stream));
   s->prop_dz = std::nanf("");
   s->have_freqs = true;
@@ -398,10 +436,12 @@ void potential(msl_sim* s, int mode, int first, int nslices, float dz, float zpl
 PotArgs pot_args(msl_sim* s, int mode, int first, int nslices, float dz, float zplane, int out_kind, void* out,
                  long long sstride) {
   require(s->binned, MSL_ERR_STATE, "UploadBinnedAtoms first");
-  ensure_ztab(s);
+  ensure_vtab(s);
   PotArgs p{};
   p.bx = s->bx.p; p.by = s->by.p; p.bz = s->bz.p; p.bZ = s->bZ.p; p.start = s->start.p; p.nslab = s->nslab;
-  p.ztab = s->ztab.p;
+  p.vtab = s->vtab.p;
+  p.nspec = s->nspec;
+  std::copy(s->spec, s->spec + 4, p.spec);
   p.MaxX = s->MaxX; p.MinX = s->MinX; p.MaxY = s->MaxY; p.MinY = s->MinY; p.MaxZ = s->MaxZ; p.MinZ = s->MinZ;
   p.nx = s->resX; p.ny = s->resY; p.ps = s->ps; p.offx = s->offx; p.offy = s->offy;
   p.dz = dz; p.first_slice = first; p.nslices = nslices; p.zplane = zplane;
@@ -486,8 +526,8 @@ struct KTimer {
 float adf_of(msl_sim* s, const float2* w, float inner, float outer) {
   const long long bs = (long long)s->npix();
   if (s->generic) {
-    copy_wave(s, s->B.p, w);
-    gen_fft2(s, s->B.p, 1, false, 1.0f);
+    gen_row(s, w, s->B.p, 1, false);
+    gen_col(s, s->B.p, 1, COL_FWD, CM_SCALE, 1.0f);
     s->gpart.ensure(gen_annulus_blocks(bs));
     HIPC(launch_gen_annulus(s->B.p, s->resX, s->resY, s->kx.p, s->ky.p, inner * 1e-3f / s->wavel,
                             outer * 1e-3f / s->wavel, s->nf * s->nf, s->gpart.p, s->red.p + 2048, s->stream));
@@ -706,7 +746,7 @@ msl_status msl_get_parameterisation(msl_sim* s, const char* path) {
   } else {
     s->fparams.assign(kFparams, kFparams + 103 * 12);
   }
-  s->ztab.release();
+  s->vtab.release();
   s->have_params = true;
   API_END(s)
 }
@@ -807,11 +847,9 @@ msl_status msl_multislice_step_conv(msl_sim* s, int it) {
   ensure_prop(s, s->conventionaldz);
   const float2* src = (it == 1) ? s->PsiMinus.p : s->Psi.p;
   if (s->generic) {
-    HIPC(launch_gen_cmul(src, s->V.p, s->PsiPlus.p, bs, s->stream));
-    gen_fft2(s, s->PsiPlus.p, 1, false, 1.0f);
-    gen_kmul(s, s->PsiPlus.p, CM_PROP, s->nf * s->nf);
-    gen_fft2(s, s->PsiPlus.p, 1, true, 1.0f);
-    copy_wave(s, s->Psi.p, s->PsiPlus.p);
+    gen_row(s, src, s->PsiPlus.p, 1, false, s->V.p);
+    gen_col(s, s->PsiPlus.p, 1, COL_FWD_MUL_INV, CM_PROP, s->nfd * s->nfd);
+    gen_row(s, s->PsiPlus.p, s->PsiPlus.p, 1, true, nullptr, s->Psi.p);
   } else {
     const bool prune = s->prune_tiles > 0;
     RowArgs r = row_args(s, src, s->PsiPlus.p, 1, bs);
@@ -843,18 +881,16 @@ msl_status msl_multislice_step(msl_sim* s, int it) {
   }
   potential(s, 2, 0, 1, 1.0f, zc, 1, s->V.p, bs);
   if (s->generic) {
-    gen_fft2(s, s->V.p, 1, false, 1.0f);
-    gen_kmul(s, s->V.p, CM_BAND, s->nf * s->nf);
-    gen_fft2(s, s->V.p, 1, true, 1.0f);
-    copy_wave(s, s->G.p, s->Psi.p);
-    gen_fft2(s, s->G.p, 1, false, 1.0f);
-    gen_kmul(s, s->G.p, CM_GRAD, s->nf * s->nf);
-    gen_fft2(s, s->G.p, 1, true, 1.0f);
+    auto filter = [&](const float2* src, float2* dst, int mul) {
+      gen_row(s, src, dst, 1, false);
+      gen_col(s, dst, 1, COL_FWD_MUL_INV, mul, s->nfd * s->nfd);
+      gen_row(s, dst, dst, 1, true);
+    };
+    filter(s->V.p, s->V.p, CM_BAND);
+    filter(s->Psi.p, s->G.p, CM_GRAD);
     HIPC(launch_fd_update(s->G.p, s->PsiMinus.p, s->PsiPlus.p, s->Psi.p, s->V.p, bs, bs, s->sigma2, s->wavel,
                           s->dzFD, s->stream));
-    gen_fft2(s, s->PsiPlus.p, 1, false, 1.0f);
-    gen_kmul(s, s->PsiPlus.p, CM_BAND, s->nf * s->nf);
-    gen_fft2(s, s->PsiPlus.p, 1, true, 1.0f);
+    filter(s->PsiPlus.p, s->PsiPlus.p, CM_BAND);
     std::swap(s->PsiMinus.p, s->Psi.p);
     std::swap(s->Psi.p, s->PsiPlus.p);
   } else {
@@ -990,7 +1026,7 @@ namespace {
 void ctf_images(msl_sim* s, int ndf, const float* dfs, float* d_out, const float* css = nullptr) {
   const long long n = (long long)s->npix();
   HIPC(hipMemcpyAsync(s->B.p, s->Psi.p, n * sizeof(float2), hipMemcpyDeviceToDevice, s->stream));
-  fft2(s, s->B.p, 1, false, s->nf);
+  fft2(s, s->B.p, 1, false, s->nfd);
   DBuf<float2> K;
   DBuf<float> dd, dc;
   K.ensure((size_t)ndf * n);
@@ -1005,7 +1041,7 @@ void ctf_images(msl_sim* s, int ndf, const float* dfs, float* d_out, const float
   c.dfs = dd.p; c.css = css ? dc.p : nullptr; c.Cs = s->Cs; c.A1 = s->A1; c.A1phi = s->A1phi; c.A2 = s->A2; c.A2phi = s->A2phi; c.obj = s->obj;
   c.wavel = s->wavel; c.beta = s->beta / 1000.f; c.delta = s->delta; c.scale = 1.0f;
   HIPC(launch_ctf(c, s->stream));
-  fft2(s, K.p, ndf, true, s->nf);
+  fft2(s, K.p, ndf, true, s->nfd);
   HIPC(launch_intensity(K.p, d_out, n * ndf, 1.0f, s->stream));
   HIPC(hipStreamSynchronize(s->stream));
 }
@@ -1032,7 +1068,7 @@ void detector_image(msl_sim* s, float dose) {
   HIPC(launch_shot_noise(W, s->detimg.p, n, s->nf, dose, s->detector_seed, s->stream));
   fft2(s, s->detimg.p, 1, false);
   HIPC(launch_detector_filter(s->detimg.p, s->resX, s->resY, s->ntf_tab.p, binning, 0, s->nf, s->stream));
-  fft2(s, s->detimg.p, 1, true, 64.f * s->nf);
+  fft2(s, s->detimg.p, 1, true, 64.0 * s->nfd);
   s->have_detimg = true;
 }
 }  // namespace
@@ -1432,7 +1468,7 @@ extern "C" msl_status msl_stem_batched(msl_sim* s, const msl_stem_batch_desc* d)
   B = std::max(1, std::min(std::min(B, d->nprobe), 65535));  // grid.y limit of the column pass
   const int C = col_tile(ny), ntiles = nx / C;
   alloc_waves(s);
-  ensure_ztab(s);
+  ensure_vtab(s);
   ensure_prop(s, d->dz);
   DBuf<float2> tall, W;
   DBuf<float> partial, adf;

@@ -72,13 +72,14 @@ struct msl_sim {
   // structure (U.cuh:88-99, 127-132)
   std::vector<int> Z;
   std::vector<float> x, y, z;
+  int nspec = 0, spec[4] = {0, 0, 0, 0};  // species when at most four (PotArgs::nspec)
   float MaxX = 0, MinX = 0, MaxY = 0, MinY = 0, MaxZ = 0, MinZ = 0;
   bool have_atoms = false;
 
   // parameterisation
   std::vector<float> fparams = std::vector<float>(kFparams, kFparams + 103 * 12);
   bool have_params = false;
-  mslh::DBuf<float> ztab;
+  mslh::DBuf<float4> vtab;  // radial potential tables of the parameters
 
   // binned atoms on the device
   mslh::DBuf<float> in_x, in_y, in_z, bx, by, bz;
@@ -100,6 +101,10 @@ struct msl_sim {
   int numberOfSlices = 0, loadblocksx = 0, loadblocksy = 0, loadslicesz = 0;
   bool have_calc = false, have_freqs = false;
   float kmax = 0, nf = 0;
+  // 1 / sqrt(resX resY) as the generic transforms apply it (64 bits: the FP32
+  // value squared is off by up to 1.2e-7 where resX resY is no power of four,
+  // at every slice); nf itself elsewhere
+  double nfd = 0;
   int prune_tiles = 0;  // > 0: columns N/4 <= x < 3N/4 are outside the propagator band
   bool zb_rows = false;  // rows N/4 <= y < 3N/4 are outside the propagator band (every column)
   std::vector<float> hkx, hky;
@@ -111,10 +116,12 @@ struct msl_sim {
 
   // waves
   mslh::DBuf<float2> PsiMinus, Psi, PsiPlus, V, G, B;
-  // sides not powers of two: the generic transforms (k_generic.hip) and
-  // their scratch; the batched, serving and differentiable paths refuse
+  // sides not both powers of two: the generic transforms (k_generic.hip),
+  // whose tables follow the sides; the batched, serving and differentiable
+  // paths refuse
   bool generic = false;
-  mslh::DBuf<float2> gscr;
+  msl::GenLen glx{}, gly{};
+  mslh::DBuf<double2> gtwx, gchx, gfix, gtwy, gchy, gfiy;
   mslh::DBuf<float> gpart;
   bool have_waves = false, fd_ready = false;
   mslh::DBuf<float> tds, image, red;
@@ -155,7 +162,7 @@ void row(msl_sim* s, int mode, int mul, const RowArgs& a);
 void col(msl_sim* s, int mode, int mul, const ColArgs& a);
 // separable Fresnel factors for slice thickness dz (px, py)
 void ensure_prop(msl_sim* s, float dz);
-void ensure_ztab(msl_sim* s);
+void ensure_vtab(msl_sim* s);
 void set_atoms(msl_sim* s, std::vector<int>&& Z, std::vector<float>&& x, std::vector<float>&& y,
                std::vector<float>&& z);
 void bin_atoms(msl_sim* s, const float* dx, const float* dy, const float* dz);

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <vector>
 
 namespace msl {
 
@@ -107,16 +108,38 @@ void set_pass_variant(int kind, int n, int v);
 int num_pass_variants(int kind);
 hipError_t launch_row_v(int mode, int mul, const RowArgs& a, hipStream_t s, int var);
 hipError_t launch_col_v(int mode, int mul, const ColArgs& a, hipStream_t s, int var);
-// grids whose sides are not powers of two (k_generic.hip): unnormalised 2D
-// FFT of nbatch [ny][nx] waves in place (scratch of the same size; twx / twy
-// the tables exp(-2 pi i k / n)), k-space multipliers (ColMul, one wave
-// layout, scale included), elementwise product, and the annular |F|^2 sum
-// (partial: gen_annulus_blocks floats) into out[0]
-hipError_t launch_gen_fft2(float2* data, float2* scratch, int nx, int ny, int nbatch, int inverse,
-                           const float2* twx, const float2* twy, hipStream_t s);
-hipError_t launch_gen_kmul(float2* w, int nx, int ny, int nbatch, int mul, const float* kx, const float* ky,
-                           const float2* px, const float2* py, float kmax, float scale, hipStream_t s);
-hipError_t launch_gen_cmul(const float2* src, const float2* t, float2* dst, long long n, hipStream_t s);
+// grids whose sides are not both powers of two (k_generic.hip): row and
+// column transforms of any length from 1 to 8192, unnormalised, and the
+// annular |F|^2 sum (partial: gen_annulus_blocks floats) into out[0]
+struct GenLen {
+  int n, M;             // length and the transforms' length (gen_fft_length)
+  // tables of gen_tables: M twiddles exp(-2 pi i k / M); n and M entries,
+  // null when M == n
+  const double2 *tw, *chirp, *filt;
+};
+struct GenRowArgs {
+  const float2* src;
+  float2* dst;
+  float2* dst2;     // optional second copy of the result
+  const float2* t;  // optional [ny][nx] factor of every wave, before the transform
+  int nx, ny, nbatch, inverse;
+  GenLen len;  // of nx
+};
+struct GenColArgs {
+  const float2* src;
+  float2* dst;
+  int nx, ny, nbatch;
+  int mode, mul;  // COL_FWD, COL_INV or COL_FWD_MUL_INV, and the factor after the first transform
+  const float *kx, *ky;
+  const float2 *px, *py;
+  float kmax;
+  double scale;
+  GenLen len;  // of ny
+};
+int gen_fft_length(int n);
+void gen_tables(int n, std::vector<double2>& tw, std::vector<double2>& chirp, std::vector<double2>& filt);
+hipError_t launch_gen_row(const GenRowArgs& a, hipStream_t s);
+hipError_t launch_gen_col(const GenColArgs& a, hipStream_t s);
 int gen_annulus_blocks(long long np);
 hipError_t launch_gen_annulus(const float2* F, int nx, int ny, const float* kx, const float* ky, float kin,
                               float kout, float scale, float* partial, float* out, hipStream_t s);
@@ -181,7 +204,9 @@ hipError_t launch_bin(const BinArgs& a, hipStream_t s);
   const int G* bZ;                                                                                       \
   const int G* start;                                                                                    \
   int nslab;                                                                                             \
-  const float G* ztab;       /* per-Z transformed Kirkland constants (103 x 12) */                       \
+  const float4 G* vtab;      /* radial tables (launch_vatom_table) */                                    \
+  int nspec;                 /* species of the atoms when at most 4 (staged in LDS), else 0 */           \
+  int spec[4];               /* their atomic numbers */                                                  \
   float MaxX, MinX, MaxY, MinY, MaxZ, MinZ;                                                              \
   int nx, ny;                                                                                            \
   float ps, offx, offy;                                                                                  \
@@ -203,12 +228,14 @@ struct PotArgs {
 hipError_t launch_potential(const PotArgs& a, hipStream_t s);
 // one slice (first_slice = first, nslices 1) of several jobs in one launch:
 // tab[j] (device) holds job j's arguments, blk0[0..njobs] (device) the first
-// workgroup of each job, job j owning potential_tiles(nx, ny) workgroups
+// workgroup of each job, job j owning potential_tiles(nx, ny) workgroups; mode (0 or 1) is every job's
 int potential_tiles(int nx, int ny);
 int potential_tile_variants();
 hipError_t launch_potential_group(const PotArgs* tab, const long long* blk0, int njobs, long long nblocks, int first,
-                                  hipStream_t s);
-void kirkland_transform(const float* fparams, float* ztab);  // host: 103x12 -> per-Z constants
+                                  int mode, hipStream_t s);
+// radial tables of every species from the 103 x 12 parameters (device)
+size_t vatom_table_size();  // float4 entries
+hipError_t launch_vatom_table(const float* fparams, float4* tab, hipStream_t s);
 
 // Probe in k-space (U.cu:354-383) for nprobe positions: batch b gets
 // (posx[b], posy[b]); or posx == nullptr for the single position (px0, py0).

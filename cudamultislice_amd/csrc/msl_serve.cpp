@@ -275,7 +275,7 @@ class Runner {
     for (int i = 1; i <= ns; ++i) {
       int ja = 0;
       while (ja < nj && jobs_[jorder[ja].second].d->nslices >= i) ++ja;
-      HIPC(launch_potential_group(dptab.p, dpblk.p, ja, pblk[ja], i, st()));
+      HIPC(launch_potential_group(dptab.p, dpblk.p, ja, pblk[ja], i, p_.potential_mode, st()));
       HIPC(launch_row_group(ROW_INV_MUL_FWD, RM_T, rg[i - 1], drg.p + (i - 1), st()));
       HIPC(launch_col_group(COL_FWD_MUL_INV, CM_PROP, cg[i - 1], dcg.p + (i - 1), st()));
       st_.launches += 3;
@@ -710,7 +710,7 @@ msl_status msl_server_run(msl_server* srv, const msl_serve_params* prm, const ms
       s->have_micro = true;
       calc_vars(s, prm->ps, 0.f, d.n, d.n, s->MaxZ - s->MinZ, 0.f, 0.f, J.stem);
       precalc(s);
-      ensure_ztab(s);
+      ensure_vtab(s);
       if (d.method == MSL_METHOD_FD)
         require(std::isfinite(s->dzFD) && s->dzFD > 0, MSL_ERR_RANGE,
                 "job " + std::to_string(i) + ": no stable finite-difference step");
