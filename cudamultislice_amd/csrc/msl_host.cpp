@@ -452,18 +452,17 @@ PotArgs pot_args(msl_sim* s, int mode, int first, int nslices, float dz, float z
   return p;
 }
 
-// host argmax / argmin of |psi| with first-occurrence ties (cublasIsamax /
-// Isamin semantics, U.cu:2261-2262)
-void extrema(const std::vector<float2>& w, float& mx, float& mn) {
-  size_t imx = 0, imn = 0;
-  float vmx = -1, vmn = 3.4e38f;
-  for (size_t i = 0; i < w.size(); ++i) {
-    const float a = std::sqrt(w[i].x * w[i].x + w[i].y * w[i].y);
-    if (a > vmx) { vmx = a; imx = i; }
-    if (a < vmn) { vmn = a; imn = i; }
-  }
-  mx = std::sqrt(w[imx].x * w[imx].x + w[imx].y * w[imx].y);
-  mn = std::sqrt(w[imn].x * w[imn].x + w[imn].y * w[imn].y);
+// |psi| at the argmax / argmin of a wave (cublasIsamax / Isamin semantics,
+// U.cu:2261-2262; where no value is a number, that of the first element)
+void extrema(msl_sim* s, const float2* w, float* out, float& mx, float& mn) {
+  s->stats.ensure(stat_scratch_doubles());
+  HIPC(launch_stats(w, (long long)s->npix(), 0, s->resX, 0, 0, s->stats.p, s->stream));
+  double v[3];
+  HIPC(hipMemcpyAsync(v, s->stats.p, sizeof(v), hipMemcpyDeviceToHost, s->stream));
+  if (out) HIPC(hipMemcpyAsync(out, w, s->npix() * sizeof(float2), hipMemcpyDeviceToHost, s->stream));
+  HIPC(hipStreamSynchronize(s->stream));
+  mx = (float)(v[0] >= 0 ? v[0] : v[2]);
+  mn = (float)(v[0] >= 0 ? v[1] : v[2]);
 }
 
 // STEM probe of U.cu:2672-2705 for one position: k-space synthesis,
@@ -942,11 +941,7 @@ msl_status msl_get_slices(const msl_sim* s, int conventional, int* out) {
 msl_status msl_get_exit_wave(msl_sim* s, float* out) {
   API_BEGIN(s)
   require(s->have_waves, MSL_ERR_STATE, "no wave");
-  std::vector<float2> ew(s->npix());
-  HIPC(hipMemcpyAsync(ew.data(), s->Psi.p, ew.size() * sizeof(float2), hipMemcpyDeviceToHost, s->stream));
-  HIPC(hipStreamSynchronize(s->stream));
-  extrema(ew, s->maxposEW, s->minposEW);
-  if (out) std::memcpy(out, ew.data(), ew.size() * sizeof(float2));
+  extrema(s, s->Psi.p, out, s->maxposEW, s->minposEW);
   API_END(s)
 }
 
@@ -956,17 +951,8 @@ msl_status msl_get_stem_exit_wave(msl_sim* s, float* out) {
   require(s->have_waves, MSL_ERR_STATE, "no wave");
   HIPC(hipMemcpyAsync(s->B.p, s->Psi.p, s->npix() * sizeof(float2), hipMemcpyDeviceToDevice, s->stream));
   fft2(s, s->B.p, 1, false);
-  std::vector<float2> F(s->npix()), ew(s->npix());
-  HIPC(hipMemcpyAsync(F.data(), s->B.p, F.size() * sizeof(float2), hipMemcpyDeviceToHost, s->stream));
-  HIPC(hipStreamSynchronize(s->stream));
-  const int nx = s->resX, ny = s->resY;
-  for (int y = 0; y < ny; ++y)
-    for (int x = 0; x < nx; ++x) {
-      const int x2 = x >= nx / 2 ? x - nx / 2 : x + nx / 2, y2 = y >= ny / 2 ? y - ny / 2 : y + ny / 2;
-      ew[(size_t)y * nx + x] = F[(size_t)y2 * nx + x2];
-    }
-  extrema(ew, s->maxposEW, s->minposEW);
-  if (out) std::memcpy(out, ew.data(), ew.size() * sizeof(float2));
+  HIPC(launch_centre(s->B.p, s->V.p, s->resX, s->resY, s->stream));
+  extrema(s, s->V.p, out, s->maxposEW, s->minposEW);
   API_END(s)
 }
 
@@ -1080,35 +1066,20 @@ msl_status msl_simulate_image(msl_sim* s, float dose) {
   const float df = s->df;
   ctf_images(s, 1, &df, s->image.p);
   s->have_detimg = false;
-  std::vector<float> im(s->npix());
-  if (s->detector) {
-    detector_image(s, dose);
-    std::vector<float2> z(s->npix());
-    d2h(s, z.data(), s->detimg.p, z.size() * sizeof(float2));
-    for (size_t i = 0; i < z.size(); ++i) im[i] = std::sqrt(z[i].x * z[i].x + z[i].y * z[i].y);
-  } else {
-    d2h(s, im.data(), s->image.p, im.size() * sizeof(float));
-  }
-  // display range and contrast (U.cu:2430-2491) on the CTF intensity:
-  // standard deviation over the top-left min(512, N) square
-  size_t imx = 0, imn = 0;
-  for (size_t i = 0; i < im.size(); ++i) {
-    if (std::fabs(im[i]) > std::fabs(im[imx])) imx = i;
-    if (std::fabs(im[i]) < std::fabs(im[imn])) imn = i;
-  }
-  s->maxposIm = std::fabs(im[imx]);
-  s->minposIm = std::fabs(im[imn]);
-  const int w = std::min(512, s->resX), h = std::min(512, s->resY);
-  double mean = 0, var = 0;
-  for (int y = 0; y < h; ++y)
-    for (int x = 0; x < w; ++x) mean += std::fabs(im[(size_t)y * s->resX + x]);
-  mean /= (double)w * h;
-  for (int y = 0; y < h; ++y)
-    for (int x = 0; x < w; ++x) {
-      const double d = std::fabs(im[(size_t)y * s->resX + x]) - mean;
-      var += d * d;
-    }
-  s->imagecontrast = (float)std::sqrt(var / ((double)w * h));
+  if (s->detector) detector_image(s, dose);
+  // display range and contrast (U.cu:2430-2491) on the modulus of the
+  // detector image, or the CTF intensity: standard deviation over the top-left
+  // min(512, N) square
+  s->stats.ensure(stat_scratch_doubles());
+  HIPC(launch_stats(s->detector ? (const void*)s->detimg.p : s->image.p, (long long)s->npix(), s->detector ? 0 : 1,
+                    s->resX, std::min(512, s->resX), std::min(512, s->resY), s->stats.p, s->stream));
+  double v[5];
+  d2h(s, v, s->stats.p, sizeof(v));
+  // (comparisons with a first value that is no number are never true)
+  const bool nan0 = std::isnan(v[2]);
+  s->maxposIm = (float)(nan0 ? v[2] : v[0]);
+  s->minposIm = (float)(nan0 ? v[2] : v[1]);
+  s->imagecontrast = (float)std::sqrt(v[4]);
   s->have_image = true;
   API_END(s)
 }

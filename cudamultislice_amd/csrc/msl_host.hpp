@@ -125,6 +125,7 @@ struct msl_sim {
   mslh::DBuf<float> gpart;
   bool have_waves = false, fd_ready = false;
   mslh::DBuf<float> tds, image, red;
+  mslh::DBuf<double> stats;  // readback statistics (launch_stats)
   // stochastic detector model (SimulateImage, U.cu:2345-2428)
   bool detector = false;
   uint64_t detector_seed = 0x4D534CULL;

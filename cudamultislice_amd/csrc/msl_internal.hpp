@@ -301,6 +301,14 @@ hipError_t launch_tds_accum(const float2* F, float* tds, int nx, int ny, hipStre
 // intensity != 0: tds += scale |F|^2 (compat=physical) instead of |F|
 hipError_t launch_tds_accum_mode(const float2* F, float* tds, int nx, int ny, int intensity, float scale,
                                  hipStream_t s);
+// extrema of n values, and mean and variance of the w x h corner (rows of nx;
+// w h = 0: extrema only), of |complex| (kind 0) or |real| (kind 1) values:
+// scratch[0..4] = max, min (numbers only: -1 and infinity if there is none),
+// value of element 0, mean, variance
+size_t stat_scratch_doubles();
+hipError_t launch_stats(const void* src, long long n, int kind, int nx, int w, int h, double* scratch, hipStream_t s);
+// out = in shifted by half the grid (fftshift)
+hipError_t launch_centre(const float2* in, float2* out, int nx, int ny, hipStream_t s);
 // sum over nbatch maps of n floats in fixed order: out (+)= sum_b in[b]
 hipError_t launch_sum_maps(const float* in, int nbatch, long long n, float* out, int accumulate, hipStream_t s);
 
