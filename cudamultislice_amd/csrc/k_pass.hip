@@ -15,7 +15,6 @@
 #include <algorithm>
 #include <cmath>
 #include <type_traits>
-#include <vector>
 
 #include "msl_fft.hpp"
 #include "msl_internal.hpp"
@@ -81,6 +80,7 @@ static int lg2(int n) {
 // loops over waves won once they existed: rows variant 4 (0.447-0.469 vs
 // 0.525-0.531 ms per 32 waves for variant 1), columns variant 5 (0.376-0.378
 // vs 0.440-0.447 ms for variant 0); at 256 variants 1 and 0 stay fastest.
+#ifndef MSL_PASS_LEN
 static int g_row_var[12] = {0, 0, 0, 0, 1, 1, 1, 1, 1, 4, 4, 4};
 static int g_col_var[12] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 7, 0, 5};
 
@@ -90,6 +90,7 @@ void set_pass_variant(int kind, int n, int v) {
   else g_col_var[lg2(n)] = v;
 }
 int num_pass_variants(int kind) { return kind == 0 ? 5 : 8; }
+#endif
 
 template <int N> struct ColTile0 { static constexpr int C = (N >= 2048) ? 4 : (N >= 1024 ? 8 : 16); };
 
@@ -117,6 +118,7 @@ template <int N, int CV> struct ColCfg {
   static constexpr int MIN_WAVES = (CV == 3 && N / T <= 8) ? 6 : 1;
 };
 
+#ifndef MSL_PASS_LEN
 int col_tile(int ny) {
   switch (ny) {
     case 16: return ColTile0<16>::C;
@@ -139,6 +141,7 @@ int band_tiles_lo(int nx) {
   if (C <= 0 || (nx / 4) % C != 0 || nx / 4 < C) return 0;
   return nx / 4 / C;
 }
+#endif
 
 // Workgroups are dispatched round-robin over the XCDs, each with its own L2.
 // A column tile narrower than 16 columns reads part of each 128-byte line;
@@ -436,40 +439,36 @@ __device__ __forceinline__ bool in_prop_band(float kxv, float kyv, float kmax) {
   return sqrtf(kxv * kxv + kyv * kyv) < kmax;
 }
 
+#ifndef MSL_PASS_LEN
 // Per column x the rows inside the propagator band are r <= rows[x].x and
-// r >= rows[x].y: |ky| grows from row 0 up to N/2 and from row N-1 down to
-// N/2+1, and the FP32 test above is monotone in |ky|.  bad[x] != 0 flags a
-// column where that shape does not hold.
-__global__ void k_prop_rows(const float* kx, const float* ky, int nx, int ny, float kmax, int2* rows, int* bad) {
-  const int x = blockIdx.x * blockDim.x + threadIdx.x;
-  if (x >= nx) return;
+// r >= rows[x].y: |ky| grows from row 0 up to N/2 and falls from there to row
+// N-1 (every k-grid of the engine, by construction), and the FP32 test above
+// is monotone in |ky|, so the rows that fail it are one run.  One wave per
+// column (a thread per column, walking its rows, took 51 us at 256 and 166 us
+// at 1024, a quarter of a small run's set-up; this takes 3-4 us).
+__global__ void __launch_bounds__(64) k_prop_rows(const float* kx, const float* ky, int nx, int ny, float kmax,
+                                                  int2* rows) {
+  const int x = blockIdx.x, lane = threadIdx.x;
   const float kxv = kx[x];
-  int hi = -1;
-  while (hi + 1 < ny && in_prop_band(kxv, ky[hi + 1], kmax)) ++hi;
-  int lo = ny;
-  while (lo - 1 > hi && in_prop_band(kxv, ky[lo - 1], kmax)) --lo;
-  int stray = 0;
-  for (int r = hi + 1; r < lo; ++r) stray |= in_prop_band(kxv, ky[r], kmax) ? 1 : 0;
-  rows[x] = make_int2(hi, lo);
-  bad[x] = stray;
+  int first = ny, last = -1;  // failing rows
+  for (int r = lane; r < ny; r += 64)
+    if (!in_prop_band(kxv, ky[r], kmax)) {
+      first = min(first, r);
+      last = max(last, r);
+    }
+  for (int d = 32; d > 0; d >>= 1) {
+    first = min(first, __shfl_xor(first, d, 64));
+    last = max(last, __shfl_xor(last, d, 64));
+  }
+  if (lane == 0) rows[x] = first < ny ? make_int2(first - 1, last + 1) : make_int2(ny - 1, ny);
 }
 
-hipError_t make_prop_rows(const float* kx, const float* ky, int nx, int ny, float kmax, int2* rows, hipStream_t s) {
+hipError_t launch_prop_rows(const float* kx, const float* ky, int nx, int ny, float kmax, int2* rows, hipStream_t s) {
   if (nx <= 0 || ny <= 0 || !kx || !ky || !rows) return hipErrorInvalidValue;
-  int* bad = nullptr;
-  hipError_t e = hipMalloc(&bad, nx * sizeof(int));
-  if (e != hipSuccess) return e;
-  std::vector<int> h(nx, 1);
-  hipLaunchKernelGGL(k_prop_rows, dim3((nx + 63) / 64), dim3(64), 0, s, kx, ky, nx, ny, kmax, rows, bad);
-  e = hipGetLastError();
-  if (e == hipSuccess) e = hipMemcpyAsync(h.data(), bad, nx * sizeof(int), hipMemcpyDeviceToHost, s);
-  if (e == hipSuccess) e = hipStreamSynchronize(s);
-  (void)hipFree(bad);
-  if (e != hipSuccess) return e;
-  for (int x = 0; x < nx; ++x)
-    if (h[x]) return hipErrorInvalidValue;
-  return hipSuccess;
+  hipLaunchKernelGGL(k_prop_rows, dim3(nx), dim3(64), 0, s, kx, ky, nx, ny, kmax, rows);
+  return hipGetLastError();
 }
+#endif
 
 template <int MUL, class A>
 __device__ __forceinline__ float2 kmul(const A& a, int x, int r, float kxv, float kyv, int2 pr) {
@@ -688,6 +687,7 @@ __global__ void __launch_bounds__((ColCfg<N, ColPL<N>::CV>::THREADS), 4) k_col_p
   }
 }
 
+#ifndef MSL_PASS_LEN
 // ------------------------------------------------------------------ grouped (uneven sizes)
 // One launch covers the waves of several grid sizes, one segment per size
 // (256 .. 2048): the workgroups of all segments are concatenated and each runs
@@ -880,6 +880,7 @@ hipError_t launch_col_group(int mode, int mul, const PassGroup<ColArgs>& h, cons
 #undef MSL_CG
   return hipGetLastError();
 }
+#endif
 
 // ------------------------------------------------------------------ dispatch
 template <int N, int RV>
@@ -1053,18 +1054,36 @@ static hipError_t col_n(int mode, int mul, const ColArgs& a, hipStream_t s, int 
   return col_nv<N, 0>(mode, mul, a, s);
 }
 
+// The kernels of each length are a translation unit of their own (this file
+// with MSL_PASS_LEN), so that they compile in parallel.
+#define MSL_PASS_LENGTHS(F) F(16) F(32) F(64) F(128) F(256) F(512) F(1024) F(2048)
+#define MSL_PASS_DECL(n)                                                                   \
+  hipError_t row_len_##n(int mode, int mul, const RowArgs& a, hipStream_t s, int var);     \
+  hipError_t col_len_##n(int mode, int mul, const ColArgs& a, hipStream_t s, int var);
+MSL_PASS_LENGTHS(MSL_PASS_DECL)
+#ifdef MSL_PASS_LEN
+#define MSL_PASS_DEF2(n)                                                                   \
+  hipError_t row_len_##n(int mode, int mul, const RowArgs& a, hipStream_t s, int var) {    \
+    return row_n<n>(mode, mul, a, s, var);                                                 \
+  }                                                                                        \
+  hipError_t col_len_##n(int mode, int mul, const ColArgs& a, hipStream_t s, int var) {    \
+    return col_n<n>(mode, mul, a, s, var);                                                 \
+  }
+#define MSL_PASS_DEF(n) MSL_PASS_DEF2(n)
+MSL_PASS_DEF(MSL_PASS_LEN)
+#else
 hipError_t launch_row_v(int mode, int mul, const RowArgs& a, hipStream_t s, int var) {
   // the kernels walk rows in steps of ny: a grid needs at least one row
   if (a.ny <= 0 || a.nbatch < 0) return hipErrorInvalidValue;
   switch (a.nx) {
-    case 16: return row_n<16>(mode, mul, a, s, var);
-    case 32: return row_n<32>(mode, mul, a, s, var);
-    case 64: return row_n<64>(mode, mul, a, s, var);
-    case 128: return row_n<128>(mode, mul, a, s, var);
-    case 256: return row_n<256>(mode, mul, a, s, var);
-    case 512: return row_n<512>(mode, mul, a, s, var);
-    case 1024: return row_n<1024>(mode, mul, a, s, var);
-    case 2048: return row_n<2048>(mode, mul, a, s, var);
+    case 16: return row_len_16(mode, mul, a, s, var);
+    case 32: return row_len_32(mode, mul, a, s, var);
+    case 64: return row_len_64(mode, mul, a, s, var);
+    case 128: return row_len_128(mode, mul, a, s, var);
+    case 256: return row_len_256(mode, mul, a, s, var);
+    case 512: return row_len_512(mode, mul, a, s, var);
+    case 1024: return row_len_1024(mode, mul, a, s, var);
+    case 2048: return row_len_2048(mode, mul, a, s, var);
   }
   return hipErrorInvalidValue;
 }
@@ -1105,14 +1124,14 @@ hipError_t launch_col_v(int mode, int mul, const ColArgs& a, hipStream_t s, int 
     else if (mul == CM_PROPCONJ) mul = CM_PROPCONJ_ZB;
   }
   switch (a.ny) {
-    case 16: return col_n<16>(mode, mul, a, s, var);
-    case 32: return col_n<32>(mode, mul, a, s, var);
-    case 64: return col_n<64>(mode, mul, a, s, var);
-    case 128: return col_n<128>(mode, mul, a, s, var);
-    case 256: return col_n<256>(mode, mul, a, s, var);
-    case 512: return col_n<512>(mode, mul, a, s, var);
-    case 1024: return col_n<1024>(mode, mul, a, s, var);
-    case 2048: return col_n<2048>(mode, mul, a, s, var);
+    case 16: return col_len_16(mode, mul, a, s, var);
+    case 32: return col_len_32(mode, mul, a, s, var);
+    case 64: return col_len_64(mode, mul, a, s, var);
+    case 128: return col_len_128(mode, mul, a, s, var);
+    case 256: return col_len_256(mode, mul, a, s, var);
+    case 512: return col_len_512(mode, mul, a, s, var);
+    case 1024: return col_len_1024(mode, mul, a, s, var);
+    case 2048: return col_len_2048(mode, mul, a, s, var);
   }
   return hipErrorInvalidValue;
 }
@@ -1123,5 +1142,7 @@ hipError_t launch_row(int mode, int mul, const RowArgs& a, hipStream_t s) {
 hipError_t launch_col(int mode, int mul, const ColArgs& a, hipStream_t s) {
   return launch_col_v(mode, mul, a, s, g_col_var[lg2(a.ny)]);
 }
+
+#endif
 
 }  // namespace msl

@@ -213,7 +213,8 @@ msl_status msl_diff_create(msl_diff** out, int device, int nx, int ny, float ps,
     up(d->kx, d->hkx); up(d->ky, d->hky); up(d->twx, tw(nx)); up(d->twy, tw(ny));
     up(d->px, pr(d->hkx)); up(d->py, pr(d->hky));
     d->prow.alloc(nx);
-    HC(make_prop_rows(d->kx.p, d->ky.p, nx, ny, d->kmax, d->prow.p, nullptr));
+    HC(launch_prop_rows(d->kx.p, d->ky.p, nx, ny, d->kmax, d->prow.p, nullptr));
+    HC(hipStreamSynchronize(nullptr));
     const size_t wave = (size_t)nprobe * nx * ny;
     d->W.alloc(wave);
     d->G.alloc(wave);

@@ -284,37 +284,36 @@ void set_atoms(msl_sim* s, std::vector<int>&& Z, std::vector<float>&& x, std::ve
 void bin_atoms(msl_sim* s, const float* dx, const float* dy, const float* dz) {
   require(s->have_atoms, MSL_ERR_STATE, "no atoms loaded");
   const int n = (int)s->x.size();
-  std::vector<float> X(n), Y(n), Zp(n);
+  // x, y, z and Z in one upload
+  std::vector<float> up(4 * (size_t)n);
   for (int i = 0; i < n; ++i) {
-    X[i] = s->x[i] + (dx ? dx[i] : 0.0f);
-    Y[i] = s->y[i] + (dy ? dy[i] : 0.0f);
-    Zp[i] = s->z[i] + (dz ? dz[i] : 0.0f);
+    up[i] = s->x[i] + (dx ? dx[i] : 0.0f);
+    up[n + i] = s->y[i] + (dy ? dy[i] : 0.0f);
+    up[2 * (size_t)n + i] = s->z[i] + (dz ? dz[i] : 0.0f);
   }
+  std::memcpy(up.data() + 3 * (size_t)n, s->Z.data(), n * sizeof(int));
   int nslab = (int)std::ceil((s->MaxZ - s->MinZ) / 1.0f);
   nslab += (nslab == 0);
   const int nb = nslab * 2500;
-  s->in_x.ensure(n); s->in_y.ensure(n); s->in_z.ensure(n); s->in_Z.ensure(n);
+  s->in.ensure(up.size());
   s->bx.ensure(n); s->by.ensure(n); s->bz.ensure(n); s->bZ.ensure(n);
   s->key.ensure(n); s->perm.ensure(n);
-  s->count.ensure(nb + 1); s->fill.ensure(nb); s->start.ensure(nb + 1); s->bad.ensure(1);
+  s->zeroed.ensure(2 * (size_t)nb + 2); s->start.ensure(nb + 1);
   s->scan_tmp.ensure((nb + 1 + 1023) / 1024 + 1);
   hipStream_t st = s->stream;
-  HIPC(hipMemcpyAsync(s->in_x.p, X.data(), n * sizeof(float), hipMemcpyHostToDevice, st));
-  HIPC(hipMemcpyAsync(s->in_y.p, Y.data(), n * sizeof(float), hipMemcpyHostToDevice, st));
-  HIPC(hipMemcpyAsync(s->in_z.p, Zp.data(), n * sizeof(float), hipMemcpyHostToDevice, st));
-  HIPC(hipMemcpyAsync(s->in_Z.p, s->Z.data(), n * sizeof(int), hipMemcpyHostToDevice, st));
-  HIPC(hipMemsetAsync(s->count.p, 0, (nb + 1) * sizeof(int), st));
-  HIPC(hipMemsetAsync(s->fill.p, 0, nb * sizeof(int), st));
-  HIPC(hipMemsetAsync(s->bad.p, 0, sizeof(int), st));
+  HIPC(hipMemcpyAsync(s->in.p, up.data(), up.size() * sizeof(float), hipMemcpyHostToDevice, st));
+  HIPC(hipMemsetAsync(s->zeroed.p, 0, (2 * (size_t)nb + 2) * sizeof(int), st));
+  int* flag = s->zeroed.p + 2 * (size_t)nb + 1;
   BinArgs a{};
-  a.x = s->in_x.p; a.y = s->in_y.p; a.z = s->in_z.p; a.Z = s->in_Z.p; a.n = n;
+  a.x = s->in.p; a.y = s->in.p + n; a.z = s->in.p + 2 * (size_t)n;
+  a.Z = reinterpret_cast<const int*>(s->in.p + 3 * (size_t)n); a.n = n;
   a.MaxX = s->MaxX; a.MinX = s->MinX; a.MaxY = s->MaxY; a.MinY = s->MinY; a.MaxZ = s->MaxZ; a.MinZ = s->MinZ;
   a.nslab = nslab;
-  a.key = s->key.p; a.count = s->count.p; a.start = s->start.p; a.fill = s->fill.p; a.perm = s->perm.p;
-  a.bx = s->bx.p; a.by = s->by.p; a.bz = s->bz.p; a.bZ = s->bZ.p; a.bad = s->bad.p; a.scan_tmp = s->scan_tmp.p;
+  a.key = s->key.p; a.count = s->zeroed.p; a.fill = s->zeroed.p + nb + 1; a.start = s->start.p; a.perm = s->perm.p;
+  a.bx = s->bx.p; a.by = s->by.p; a.bz = s->bz.p; a.bZ = s->bZ.p; a.bad = flag; a.scan_tmp = s->scan_tmp.p;
   HIPC(launch_bin(a, st));
   int bad = 0;
-  HIPC(hipMemcpyAsync(&bad, s->bad.p, sizeof(int), hipMemcpyDeviceToHost, st));
+  HIPC(hipMemcpyAsync(&bad, flag, sizeof(int), hipMemcpyDeviceToHost, st));
   HIPC(hipStreamSynchronize(st));
   require(!bad, MSL_ERR_RANGE, "an atom lies outside the 50x50 bin grid (displacement larger than the 2 A margin?)");
   s->nslab = nslab;
@@ -384,17 +383,10 @@ void precalc(msl_sim* s) {
   for (int x = rx / 4; x < 3 * rx / 4 && s->prune_tiles > 0; ++x)
     if (std::sqrt(s->hkx[x] * s->hkx[x] + 0.0f) < s->kmax) s->prune_tiles = 0;
   s->zb_rows = prop_rows_quarter(s->hky.data(), ry, s->kmax);
-  s->kx.ensure(rx);
-  s->ky.ensure(ry);
-  HIPC(hipMemcpyAsync(s->kx.p, s->hkx.data(), rx * sizeof(float), hipMemcpyHostToDevice, s->stream));
-  HIPC(hipMemcpyAsync(s->ky.p, s->hky.data(), ry * sizeof(float), hipMemcpyHostToDevice, s->stream));
-  s->prow.ensure(rx);
-  HIPC(make_prop_rows(s->kx.p, s->ky.p, rx, ry, s->kmax, s->prow.p, s->stream));
   auto upload = [&](auto& d, const auto& v) {
     d.ensure(v.size());
     if (!v.empty()) HIPC(hipMemcpyAsync(d.p, v.data(), v.size() * sizeof(v[0]), hipMemcpyHostToDevice, s->stream));
   };
-  std::vector<float2> tx, ty;
   std::vector<double2> wx, cx, fx, wy, cy, fy;
   if (s->generic && s->glx.n == rx && s->gly.n == ry) {
     // the tables depend on the sides alone
@@ -409,12 +401,25 @@ void precalc(msl_sim* s) {
     upload(s->gfiy, fy);
     s->glx = GenLen{rx, (int)wx.size(), s->gtwx.p, cx.empty() ? nullptr : s->gchx.p, cx.empty() ? nullptr : s->gfix.p};
     s->gly = GenLen{ry, (int)wy.size(), s->gtwy.p, cy.empty() ? nullptr : s->gchy.p, cy.empty() ? nullptr : s->gfiy.p};
-  } else {
-    tx = twiddles(rx);
-    ty = twiddles(ry);
-    upload(s->twx, tx);
-    upload(s->twy, ty);
   }
+  // k-grids, and the twiddles of the power-of-two passes
+  std::vector<float> kt(s->hkx);
+  kt.insert(kt.end(), s->hky.begin(), s->hky.end());
+  kt.resize(kt.size() + kt.size() % 2);
+  const size_t o = kt.size();
+  if (!s->generic) {
+    const auto tx = twiddles(rx), ty = twiddles(ry);
+    kt.resize(o + 2 * (size_t)(rx + ry));
+    std::memcpy(kt.data() + o, tx.data(), rx * sizeof(float2));
+    std::memcpy(kt.data() + o + 2 * (size_t)rx, ty.data(), ry * sizeof(float2));
+  }
+  upload(s->ktab, kt);
+  s->kx.p = s->ktab.p;
+  s->ky.p = s->ktab.p + rx;
+  s->twx.p = s->generic ? nullptr : reinterpret_cast<float2*>(s->ktab.p + o);
+  s->twy.p = s->generic ? nullptr : reinterpret_cast<float2*>(s->ktab.p + o) + rx;
+  s->prow.ensure(rx);
+  HIPC(launch_prop_rows(s->kx.p, s->ky.p, rx, ry, s->kmax, s->prow.p, s->stream));
   HIPC(hipStreamSynchronize(s->stream));
   s->prop_dz = std::nanf("");
   s->have_freqs = true;

@@ -53,6 +53,11 @@ template <class T> struct DBuf {
   }
 };
 
+// a pointer into another buffer
+template <class T> struct Ptr {
+  T* p = nullptr;
+};
+
 }  // namespace mslh
 
 // ------------------------------------------------------------------ handle
@@ -82,8 +87,8 @@ struct msl_sim {
   mslh::DBuf<float4> vtab;  // radial potential tables of the parameters
 
   // binned atoms on the device
-  mslh::DBuf<float> in_x, in_y, in_z, bx, by, bz;
-  mslh::DBuf<int> in_Z, bZ, key, count, start, fill, perm, bad, scan_tmp;
+  mslh::DBuf<float> in, bx, by, bz;   // in: x, y, z and Z as uploaded
+  mslh::DBuf<int> bZ, key, zeroed, start, perm, scan_tmp;  // zeroed: counts, fills and the range flag
   int nslab = 0, nbinned = 0;
   bool binned = false;
   uint64_t tds_seed = 0x4D534CULL;
@@ -108,8 +113,12 @@ struct msl_sim {
   int prune_tiles = 0;  // > 0: columns N/4 <= x < 3N/4 are outside the propagator band
   bool zb_rows = false;  // rows N/4 <= y < 3N/4 are outside the propagator band (every column)
   std::vector<float> hkx, hky;
-  mslh::DBuf<float> kx, ky;
-  mslh::DBuf<float2> twx, twy, px, py;
+  // the k-grids and twiddles of both axes, one upload; kx, ky, twx, twy point
+  // into it
+  mslh::DBuf<float> ktab;
+  mslh::Ptr<float> kx, ky;
+  mslh::Ptr<float2> twx, twy;
+  mslh::DBuf<float2> px, py;
   mslh::DBuf<int2> prow;  // rows of each column inside |k| < kmax
   float prop_dz = std::nanf("");
   float conventionaldz = 1.0f;

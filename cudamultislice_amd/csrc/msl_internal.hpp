@@ -73,7 +73,7 @@ enum ColMul { CM_SCALE = 0, CM_PROP = 1, CM_BAND = 2, CM_GRAD = 3, CM_PROPCONJ =
   const float2 G* px;        /* separable propagator factors exp(-i pi lambda dz k^2) */                 \
   const float2 G* py;                                                                                    \
   /* CM_PROP / CM_PROPCONJ: column x is inside |k| < kmax at rows r <= prop_rows[x].x and */            \
-  /* r >= prop_rows[x].y (make_prop_rows) */                                                             \
+  /* r >= prop_rows[x].y (launch_prop_rows) */                                                           \
   const int2 G* prop_rows;                                                                               \
   float kmax;                                                                                            \
   float scale;                                                                                           \
@@ -93,9 +93,8 @@ struct ColArgs {
 };
 
 // rows of each column inside the propagator band |k| < kmax (nx entries,
-// device), built on s and waited for; hipErrorInvalidValue if some column's
-// band is not a run from each end of ky
-hipError_t make_prop_rows(const float* kx, const float* ky, int nx, int ny, float kmax, int2* rows, hipStream_t s);
+// device), queued on s
+hipError_t launch_prop_rows(const float* kx, const float* ky, int nx, int ny, float kmax, int2* rows, hipStream_t s);
 int col_tile(int ny);  // columns per column-pass workgroup (detector layout)
 // true when rows ny/4 .. 3ny/4 - 1 fail the propagator test |k| < kmax for
 // every column: the row ny/4 fails it at kx = 0 (the FP32 test of

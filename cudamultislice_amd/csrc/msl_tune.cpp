@@ -52,7 +52,7 @@ struct Bench {
     if ((e = hipMemcpyAsync(pxy.p, p.data(), n * 8, hipMemcpyHostToDevice, s)) != hipSuccess) return e;
     if ((e = hipMemcpyAsync(tw.p, w.data(), n * 8, hipMemcpyHostToDevice, s)) != hipSuccess) return e;
     if ((e = launch_hash_fill(t.as<float2>(), (long long)n * n, 7u, 1, s)) != hipSuccess) return e;
-    if ((e = make_prop_rows(k.as<float>(), k.as<float>(), n, n, kmax, rows.as<int2>(), s)) != hipSuccess) return e;
+    if ((e = launch_prop_rows(k.as<float>(), k.as<float>(), n, n, kmax, rows.as<int2>(), s)) != hipSuccess) return e;
     return hipStreamSynchronize(s);
   }
   hipError_t fill(float2* w, int nw, hipStream_t s) { return launch_hash_fill(w, (long long)nw * n * n, 11u, 0, s); }
