@@ -179,6 +179,31 @@ template <int N, int RV> struct RowCfg {
 // T_SLOTS (row loop only): each wave reads the transmission of its own slot
 // (RowArgs::t_index or b / t_group) instead of one shared by the launch
 enum { PRUNE_IN = 1, PRUNE_OUT = 2, STORE_AUX = 4, T_SLOTS = 8 };
+// a workgroup's N table entries, requested when this is made and written to
+// LDS (and waited for by the workgroup) by store()
+template <int N, int NT> struct TwStage {
+  static constexpr int PER = (N + NT - 1) / NT;
+  float2 r[PER];
+  __device__ __forceinline__ explicit TwStage(const float2* tab) {
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+      const int i = threadIdx.x + k * NT;
+      if (PER * NT == N || i < N) r[k] = tab[i];
+    }
+  }
+  __device__ __forceinline__ void put(float2* lds) const {
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+      const int i = threadIdx.x + k * NT;
+      if (PER * NT == N || i < N) lds[i] = r[k];
+    }
+  }
+  __device__ __forceinline__ void store(float2* lds) const {
+    put(lds);
+    __syncthreads();
+  }
+};
+
 template <int E> struct BandBlocks {
   static constexpr int LO = E / 4 > 0 ? E / 4 : 1;
   static __host__ __device__ constexpr bool active(int c) { return c < LO || c >= E - LO; }
@@ -189,8 +214,11 @@ template <int E> struct BandBlocks {
 // per launch, arguments in kernel registers) and k_row_group (several
 // lengths per launch, arguments read from a table in device memory) both
 // expand this one body.
-template <int N, int MODE, int MUL, int FL, int RV, class A>
-__device__ __forceinline__ void row_block(const A& a, long long blk, float2* lds, const float2* stw) {
+// staged() runs once the loads of the row are under way: k_row fills and
+// waits for the twiddles there, so a workgroup waits for one round of loads
+// before its first transform, not for two.
+template <int N, int MODE, int MUL, int FL, int RV, class A, class F>
+__device__ __forceinline__ void row_block(const A& a, long long blk, float2* lds, const float2* stw, F staged) {
   using Cfg = RowCfg<N, RV>;
   using P = typename Cfg::P;
   using S = typename std::conditional<Cfg::WAVE, WaveSync, BlockSync>::type;
@@ -222,6 +250,22 @@ __device__ __forceinline__ void row_block(const A& a, long long blk, float2* lds
     for (int c = 0; c < E; ++c)
       if (!(FL & PRUNE_IN) || BandBlocks<E>::active(c)) v[c] = row[t + c * T];
   }
+  // the transmission with them where the registers leave the occupancy that
+  // the LDS allows (up to 256), and where no transform comes first
+  constexpr bool EARLY_T = MUL == RM_T && (MODE == ROW_FWD || (MODE == ROW_INV_MUL_FWD && N <= 256));
+  float2 te[EARLY_T ? E : 1];
+  auto load_t = [&](float2* w) {
+    // slot of wave b0 on the scalar unit; per thread only past a wave edge
+    long long slot = a.t_index ? (long long)a.t_index[b0] : b0 / a.t_group;
+    if (db != 0) slot = a.t_index ? (long long)a.t_index[b] : (long long)(b / a.t_group);
+    const float2* tr = a.t + slot * a.t_bstride + (long long)y * N;
+#pragma unroll
+    for (int c = 0; c < E; ++c) w[c] = tr[t + c * T];
+  };
+  if constexpr (EARLY_T) {
+    if (ok) load_t(te);
+  }
+  staged();
   const LL L{lds + ln * LS, 1};
   constexpr bool ZIN = (FL & PRUNE_IN) != 0 && E % 4 == 0 && P::R1 % 4 == 0;  // first transform's input
   if constexpr (MODE == ROW_INV || MODE == ROW_INV_MUL_FWD || MODE == ROW_INV_FD_FWD)
@@ -278,12 +322,11 @@ __device__ __forceinline__ void row_block(const A& a, long long blk, float2* lds
     }
   } else if constexpr (MUL == RM_T) {
     if (ok) {
-      // slot of wave b0 on the scalar unit; per thread only past a wave edge
-      long long slot = a.t_index ? (long long)a.t_index[b0] : b0 / a.t_group;
-      if (db != 0) slot = a.t_index ? (long long)a.t_index[b] : (long long)(b / a.t_group);
-      const float2* tr = a.t + slot * a.t_bstride + (long long)y * N;
+      float2 tl[EARLY_T ? 1 : E];
+      if constexpr (!EARLY_T) load_t(tl);
+      const float2* tr = EARLY_T ? te : tl;
 #pragma unroll
-      for (int c = 0; c < E; ++c) v[c] = cscale(cmul(v[c], tr[t + c * T]), a.scale);
+      for (int c = 0; c < E; ++c) v[c] = cscale(cmul(v[c], tr[c]), a.scale);
     }
   } else {
     if (a.scale != 1.0f) {
@@ -324,8 +367,8 @@ template <int N, int MODE, int MUL, int FL, int RV>
 __global__ void __launch_bounds__((RowCfg<N, RV>::LINES * RowCfg<N, RV>::T)) k_row(RowArgs a) {
   __shared__ float2 lds[RowCfg<N, RV>::LINES * RowCfg<N, RV>::LS];
   __shared__ float2 stw[N];  // twiddles staged in LDS: no global loads inside the transforms
-  for (int i = threadIdx.x; i < N; i += RowCfg<N, RV>::LINES * RowCfg<N, RV>::T) stw[i] = a.tw[i];
-  __syncthreads();
+  constexpr int NT = RowCfg<N, RV>::LINES * RowCfg<N, RV>::T;
+  const TwStage<N, NT> tws(a.tw);
   long long blk = blockIdx.x;
   // wave-interleaved, XCD-aware order where a shared slice outgrows the L2
   // (measured slower than the plain order at 1024 and below, where the slice
@@ -333,7 +376,7 @@ __global__ void __launch_bounds__((RowCfg<N, RV>::LINES * RowCfg<N, RV>::T)) k_r
   if constexpr (N >= 2048 && MUL != RM_NONE)
     if (N % RowCfg<N, RV>::LINES == 0 && a.ny == N)
       blk = row_order(blockIdx.x, gridDim.x, a.nbatch, N / RowCfg<N, RV>::LINES);
-  row_block<N, MODE, MUL, FL, RV>(a, blk, lds, stw);
+  row_block<N, MODE, MUL, FL, RV>(a, blk, lds, stw, [&] { tws.store(stw); });
 }
 
 // Variant 4, for IFFT_x -> t -> FFT_x: a workgroup owns row y of LINES x
@@ -497,35 +540,37 @@ template <int MODE> struct ColModeTraits {
   static constexpr bool INV = MODE == COL_INV || MODE == COL_FWD_MUL_INV || MODE == COL_MUL_INV;
 };
 
-// FFT / multiply / IFFT of one column held canonically by T threads
-template <class P, int N, int MODE, int MUL, class S, class LL, class A>
+template <int MODE, int MUL> constexpr bool needs_rows() {
+  return ColModeTraits<MODE>::MULT &&
+         (MUL == CM_PROP || MUL == CM_PROPCONJ || MUL == CM_PROP_ZB || MUL == CM_PROPCONJ_ZB);
+}
+
+// FFT / multiply / IFFT of one column held canonically by T threads; pr and
+// pxv are the column's band rows and propagator factor, py the rows' factors
+template <class P, int N, int MODE, int MUL, class S, class LL, class A, class PY>
 __device__ __forceinline__ void col_body(float2 (&v)[N / P::T], int t, int x, const A& a, const LL& L,
-                                         const float2* tw) {
+                                         const float2* tw, int2 pr, float2 pxv, const PY py) {
   using Tr = ColModeTraits<MODE>;
   constexpr int T = P::T, E = N / T;
   if constexpr (Tr::FWD) fft_line<P, N, -1, S>(v, t, tw, L);
   // frequencies are read only by modes that need them (scale-only passes may
   // run without k-grids)
   constexpr bool NEEDK = (Tr::MULT && (MUL == CM_BAND || MUL == CM_GRAD || MUL == CM_BANDGRAD));
-  constexpr bool NEEDROWS =
-      (Tr::MULT && (MUL == CM_PROP || MUL == CM_PROPCONJ || MUL == CM_PROP_ZB || MUL == CM_PROPCONJ_ZB));
+  constexpr bool NEEDROWS = needs_rows<MODE, MUL>();
   constexpr bool CONJ = MUL == CM_PROPCONJ || MUL == CM_PROPCONJ_ZB;
   // the propagator zeroes rows N/4 .. 3N/4 - 1 (canonical blocks E/4 .. 3E/4 - 1)
   constexpr bool ZB = (MUL == CM_PROP_ZB || MUL == CM_PROPCONJ_ZB) && E % 4 == 0 && P::R1 % 4 == 0;
   float kxv = 0.f;
   if constexpr (NEEDK) kxv = a.kx[x];
-  int2 pr = make_int2(0, 0);
-  if constexpr (NEEDROWS) pr = a.prop_rows[x];
   if constexpr (NEEDROWS) {
     // propagator inside |k| < kmax (rows per column from k_prop_rows): the
     // factor is loaded for every row and zeroed by a multiplier, so the
     // compiler issues the loads together instead of one branch (and one
     // memory round trip) per element
-    const float2 pxv = a.px[x];
 #pragma unroll
     for (int c = 0; c < E; ++c) {
       const int r = t + c * T;
-      float2 p = cmul(pxv, a.py[r]);
+      float2 p = cmul(pxv, py[r]);
       if constexpr (CONJ) p.y = -p.y;
       const float m = (r <= pr.x || r >= pr.y) ? a.scale : 0.f;
       v[c] = cmul(v[c], cscale(p, m));
@@ -549,8 +594,10 @@ __device__ __forceinline__ void col_body(float2 (&v)[N / P::T], int t, int x, co
 // (col, t) holds rows t + c T of column col; workgroup barriers
 // launched tile bx (of nbx per wave) of wave b; lds holds Cfg::LDS elements,
 // stw the twiddles of length N
-template <int N, int MODE, int MUL, class Cfg, class A>
-__device__ __forceinline__ void col_block(const A& a, int bx, int b, int nbx, float2* lds, const float2* stw) {
+// (staged() as in row_block; py the propagator's row factors)
+template <int N, int MODE, int MUL, class Cfg, class A, class PY, class F>
+__device__ __forceinline__ void col_block(const A& a, int bx, int b, int nbx, float2* lds, const float2* stw,
+                                          const PY py, F staged) {
   constexpr int T = Cfg::T, E = N / T, C = Cfg::C;
   const int col = Cfg::WAVECOL ? threadIdx.x / T : threadIdx.x % C;
   const int t = Cfg::WAVECOL ? threadIdx.x % T : threadIdx.x / C;
@@ -569,13 +616,20 @@ __device__ __forceinline__ void col_block(const A& a, int bx, int b, int nbx, fl
 #pragma unroll
     for (int c = 0; c < E; ++c) v[c] = src[o0 + (unsigned)c * step];
   }
+  int2 pr = make_int2(0, 0);
+  float2 pxv = make_float2(0.f, 0.f);
+  if constexpr (needs_rows<MODE, MUL>()) {
+    pr = a.prop_rows[x];
+    pxv = a.px[x];
+  }
+  staged();
   using LL = LdsLine<Cfg::SH>;
   const LL L = Cfg::INTERLEAVED ? LL{lds + col, C} : LL{lds + col * Cfg::LSC, 1};
   if constexpr (Cfg::DUAL) {
     const DualLine<LL> D{L, LL{lds + N * C + col, C}};
-    col_body<typename Cfg::P, N, MODE, MUL, S>(v, t, x, a, D, stw);
+    col_body<typename Cfg::P, N, MODE, MUL, S>(v, t, x, a, D, stw, pr, pxv, py);
   } else {
-    col_body<typename Cfg::P, N, MODE, MUL, S>(v, t, x, a, L, stw);
+    col_body<typename Cfg::P, N, MODE, MUL, S>(v, t, x, a, L, stw, pr, pxv, py);
   }
   if constexpr (MODE == COL_FWD_DETECT) {
     const float kxv = a.kx[x];
@@ -614,11 +668,19 @@ __global__ void __launch_bounds__((ColCfg<N, CV>::THREADS), (ColCfg<N, CV>::MIN_
   using Cfg = ColCfg<N, CV>;
   __shared__ float2 lds[Cfg::LDS];
   __shared__ float2 stw[N];  // twiddles staged in LDS
-  for (int i = threadIdx.x; i < N; i += Cfg::THREADS) stw[i] = a.tw[i];
-  __syncthreads();
+  // and the propagator's row factors: read between the transforms, where a
+  // load from memory would stall the workgroup
+  constexpr bool ROWS = needs_rows<MODE, MUL>();
+  __shared__ float2 spy[ROWS ? N : 1];
+  const TwStage<N, Cfg::THREADS> tws(a.tw);
+  const TwStage<ROWS ? N : 1, Cfg::THREADS> pys(ROWS ? a.py : a.tw);
   // logical (tile, wave) of this workgroup, XCD-aware
   const long long gid = xcd_remap((long long)blockIdx.y * gridDim.x + blockIdx.x, (long long)gridDim.x * gridDim.y);
-  col_block<N, MODE, MUL, Cfg>(a, (int)(gid % gridDim.x), (int)(gid / gridDim.x), (int)gridDim.x, lds, stw);
+  col_block<N, MODE, MUL, Cfg>(a, (int)(gid % gridDim.x), (int)(gid / gridDim.x), (int)gridDim.x, lds, stw,
+                               (const float2*)spy, [&] {
+                                 if constexpr (ROWS) pys.put(spy);
+                                 tws.store(stw);
+                               });
 }
 
 // ------------------------------------------------------------------ columns looping over waves
@@ -738,12 +800,12 @@ __global__ void __launch_bounds__(256) k_row_group(const PassGroup<RowArgs>* g, 
   for (int i = threadIdx.x; i < n; i += 256) stw[i] = a.tw[i];
   __syncthreads();
   switch (n) {
-    case 256: row_block<256, MODE, MUL, FL, GroupRow<256>::RV>(a, blk, lds, stw); break;
-    case 512: row_block<512, MODE, MUL, FL, GroupRow<512>::RV>(a, blk, lds, stw); break;
-    case 1024: row_block<1024, MODE, MUL, FL, GroupRow<1024>::RV>(a, blk, lds, stw); break;
+    case 256: row_block<256, MODE, MUL, FL, GroupRow<256>::RV>(a, blk, lds, stw, [] {}); break;
+    case 512: row_block<512, MODE, MUL, FL, GroupRow<512>::RV>(a, blk, lds, stw, [] {}); break;
+    case 1024: row_block<1024, MODE, MUL, FL, GroupRow<1024>::RV>(a, blk, lds, stw, [] {}); break;
     default: {
       constexpr int ybs = 2048 / RowCfg<2048, GroupRow<2048>::RV>::LINES;
-      row_block<2048, MODE, MUL, FL, GroupRow<2048>::RV>(a, row_interleave(blk, a.nbatch, ybs), lds, stw);
+      row_block<2048, MODE, MUL, FL, GroupRow<2048>::RV>(a, row_interleave(blk, a.nbatch, ybs), lds, stw, [] {});
       break;
     }
   }
@@ -765,10 +827,10 @@ __global__ void __launch_bounds__(512) k_col_group(const PassGroup<ColArgs>* g, 
   for (int i = threadIdx.x; i < n; i += 512) stw[i] = a.tw[i];
   __syncthreads();
   switch (n) {
-    case 256: col_block<256, MODE, MUL, GroupCol<256>>(a, bx, b, nbx, lds, stw); break;
-    case 512: col_block<512, MODE, MUL, GroupCol<512>>(a, bx, b, nbx, lds, stw); break;
-    case 1024: col_block<1024, MODE, MUL, GroupCol<1024>>(a, bx, b, nbx, lds, stw); break;
-    default: col_block<2048, MODE, MUL, GroupCol<2048>>(a, bx, b, nbx, lds, stw); break;
+    case 256: col_block<256, MODE, MUL, GroupCol<256>>(a, bx, b, nbx, lds, stw, a.py, [] {}); break;
+    case 512: col_block<512, MODE, MUL, GroupCol<512>>(a, bx, b, nbx, lds, stw, a.py, [] {}); break;
+    case 1024: col_block<1024, MODE, MUL, GroupCol<1024>>(a, bx, b, nbx, lds, stw, a.py, [] {}); break;
+    default: col_block<2048, MODE, MUL, GroupCol<2048>>(a, bx, b, nbx, lds, stw, a.py, [] {}); break;
   }
 }
 
