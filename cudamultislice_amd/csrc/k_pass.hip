@@ -72,22 +72,62 @@ static int lg2(int n) {
 // 256 waves); rows of 512 and 1024 then went to variant 4 (one workgroup per
 // row looping over waves; 512: 0.58 vs 0.69 ms per 1024 waves for 2, 1024:
 // 0.78 vs 0.85 ms per 256 waves for 3; 1.131 vs 1.080e6 probe-slice/s on the
-// 512^2 STEM workload).  Columns: 512 half-width tiles on the alternative plan (0.48
-// vs 0.51 ms per 1024 waves for half-width tiles on the default plan, 1 %
-// more probe-slices per second on the 512^2 STEM workload); 256, 1024 and
-// 2048 variant 0 (1024: 0.54 vs 0.62 ms per 256 waves for the half-width
-// tiles once the inverse skipped the propagator's zero rows).  At 2048 the
+// 512^2 STEM workload).  Columns: 512 half-width tiles (with the row factors
+// in LDS 72.1 us per 256 waves against 73.1 on the alternative plan, which
+// was ahead before); 256, 1024 and 2048 variant 0 (1024: 0.54 vs 0.62 ms per
+// 256 waves for the half-width tiles once the inverse skipped the
+// propagator's zero rows).  At 2048 the
 // loops over waves won once they existed: rows variant 4 (0.447-0.469 vs
 // 0.525-0.531 ms per 32 waves for variant 1), columns variant 5 (0.376-0.378
 // vs 0.440-0.447 ms for variant 0); at 256 variants 1 and 0 stay fastest.
 #ifndef MSL_PASS_LEN
-static int g_row_var[12] = {0, 0, 0, 0, 1, 1, 1, 1, 1, 4, 4, 4};
-static int g_col_var[12] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 7, 0, 5};
+static const int kRowDefault[12] = {0, 0, 0, 0, 1, 1, 1, 1, 1, 4, 4, 4};
+static const int kColDefault[12] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 3, 0, 5};
+// variants chosen by msl_set_pass_variant or the tuner (-1: by the rules below)
+static int g_row_var[12] = {-1, -1, -1, -1, -1, -1, -1, -1, -1, -1, -1, -1};
+static int g_col_var[12] = {-1, -1, -1, -1, -1, -1, -1, -1, -1, -1, -1, -1};
 
-int pass_variant(int kind, int n) { return kind == 0 ? g_row_var[lg2(n)] : g_col_var[lg2(n)]; }
+int pass_variant(int kind, int n) {
+  const int l = lg2(n), v = kind == 0 ? g_row_var[l] : g_col_var[l];
+  return v >= 0 ? v : kind == 0 ? kRowDefault[l] : kColDefault[l];
+}
 void set_pass_variant(int kind, int n, int v) {
   if (kind == 0) g_row_var[lg2(n)] = v;
   else g_col_var[lg2(n)] = v;
+}
+
+// The variant of a launch of `lines` rows.  Below some thousand rows the
+// chip is not full and the shortest chain of a line wins (more threads per
+// line, or fewer lines per workgroup); above, the layouts of the defaults.
+// Between variants of one plan (0, 1, 3; at 1024 and 2048 also 4) a line's
+// bits are the same, so the choice may follow the batch; a change of plan
+// (2; 4 at 512) is for callers whose batch never varies (RowArgs::alone), so
+// that a wave's result does not depend on how a run is cut into batches.
+// Us per launch of IFFT -> t -> FFT at 1 / 4 / 16 waves of n x n (variant:time):
+//   128  1: 4.4 / 4.5 / 4.6, 2: 3.7 / 3.8 / 3.8 (from 37 waves on 1)
+//   256  1: 4.7 / 4.8 / 5.3, 2: 3.8 / 3.9 / 5.3
+//   512  1: 4.2 at 1 wave (2: 5.8); at 24 waves 3: 15.7, 4: 18.2; at 64 3: 40.2, 4: 38.1
+//  1024  1: 6.5 at 1 wave (3: 7.9); at 8 waves 3: 23.9, 4: 25.4; at 16 3: 44.5, 4: 42.6
+static int auto_row(int n, long long lines, bool alone) {
+  switch (n) {
+    case 128:
+    case 256: return alone && lines <= 3072 ? 2 : 1;
+    case 512: return !alone || lines > 20480 ? 4 : lines <= 1024 ? 1 : 3;
+    case 1024: return lines <= 2048 ? 1 : lines <= 12288 ? 3 : 4;
+  }
+  return kRowDefault[lg2(n)];
+}
+
+// The variant of a launch of `cols` columns: half-width tiles (twice the
+// workgroups, the same bits as 0) while the full ones leave CUs idle, and at
+// 512 always.  Us per launch of the propagation pass, variants 0 and 3:
+//   64   3.3, 2.9 at 16 waves of n x n
+//  256   5.2, 4.4 at 1 wave; 5.5, 4.9 at 16; 8.1, 8.2 at 64
+//  512   8.1, 5.3 at 1; 16.3, 11.0 at 24; 128, 72.1 at 256 (variant 7: 6.2, 11.7, 73.1)
+//  1024  8.5, 7.8 at 1; 16.1, 19.1 at 8
+static int auto_col(int n, long long cols) {
+  const int half = n == 64 ? 4096 : n == 256 ? 8192 : n == 1024 ? 1024 : 0;
+  return cols <= half ? 3 : kColDefault[lg2(n)];
 }
 int num_pass_variants(int kind) { return kind == 0 ? 5 : 8; }
 #endif
@@ -1199,10 +1239,12 @@ hipError_t launch_col_v(int mode, int mul, const ColArgs& a, hipStream_t s, int 
 }
 
 hipError_t launch_row(int mode, int mul, const RowArgs& a, hipStream_t s) {
-  return launch_row_v(mode, mul, a, s, g_row_var[lg2(a.nx)]);
+  const int v = fft_size_supported(a.nx) ? g_row_var[lg2(a.nx)] : 0;
+  return launch_row_v(mode, mul, a, s, v >= 0 ? v : auto_row(a.nx, (long long)a.nbatch * a.ny, a.alone != 0));
 }
 hipError_t launch_col(int mode, int mul, const ColArgs& a, hipStream_t s) {
-  return launch_col_v(mode, mul, a, s, g_col_var[lg2(a.ny)]);
+  const int v = fft_size_supported(a.ny) ? g_col_var[lg2(a.ny)] : 0;
+  return launch_col_v(mode, mul, a, s, v >= 0 ? v : auto_col(a.ny, (long long)a.nbatch * a.nx));
 }
 
 #endif

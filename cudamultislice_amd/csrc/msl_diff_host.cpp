@@ -80,6 +80,7 @@ RowArgs rargs(msl_diff* d, const float2* src, float2* dst, bool pin = false, boo
   a.src = src; a.dst = dst; a.src_bstride = a.dst_bstride = d->np();
   a.nx = d->nx; a.ny = d->ny; a.nbatch = d->B; a.t_group = d->B; a.t_bstride = 0; a.scale = 1.f;
   a.tw = d->twx.p; a.sigma = d->sigma;
+  a.alone = 1;
   return a;
 }
 ColArgs cargs(msl_diff* d, const float2* src, float2* dst, float scale) {

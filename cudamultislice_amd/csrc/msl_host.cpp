@@ -152,6 +152,11 @@ ColArgs col_args(msl_sim* s, const float2* src, float2* dst, int nbatch, long lo
 }
 
 void row(msl_sim* s, int mode, int mul, const RowArgs& a) { HIPC(launch_row(mode, mul, a, s->stream)); }
+// the one wave of the handle's own steps
+void row1(msl_sim* s, int mode, int mul, RowArgs a) {
+  a.alone = 1;
+  row(s, mode, mul, a);
+}
 void col(msl_sim* s, int mode, int mul, const ColArgs& a) { HIPC(launch_col(mode, mul, a, s->stream)); }
 
 // separable Fresnel factors exp(-i pi dz lambda k^2) per axis (CreatePropsKernel,
@@ -227,11 +232,11 @@ void propagate(msl_sim* s, float2* src, float2* dst, float dz) {
     return;
   }
   const long long bs = (long long)s->npix();
-  row(s, ROW_FWD, RM_NONE, row_args(s, src, dst, 1, bs));
+  row1(s, ROW_FWD, RM_NONE, row_args(s, src, dst, 1, bs));
   ColArgs c = col_args(s, dst, dst, 1, bs);
   c.scale = s->nf * s->nf;
   col(s, COL_FWD_MUL_INV, CM_PROP, c);
-  row(s, ROW_INV, RM_NONE, row_args(s, dst, dst, 1, bs));
+  row1(s, ROW_INV, RM_NONE, row_args(s, dst, dst, 1, bs));
 }
 
 void ensure_vtab(msl_sim* s) {
@@ -537,7 +542,7 @@ float adf_of(msl_sim* s, const float2* w, float inner, float outer) {
                             outer * 1e-3f / s->wavel, s->nf * s->nf, s->gpart.p, s->red.p + 2048, s->stream));
     return download_scalar(s, s->red.p + 2048);
   }
-  row(s, ROW_FWD, RM_NONE, row_args(s, w, s->B.p, 1, bs));
+  row1(s, ROW_FWD, RM_NONE, row_args(s, w, s->B.p, 1, bs));
   ColArgs c = col_args(s, s->B.p, nullptr, 1, bs);
   c.kin = inner * 1e-3f / s->wavel;
   c.kout = outer * 1e-3f / s->wavel;
@@ -554,25 +559,25 @@ float adf_of(msl_sim* s, const float2* w, float inner, float outer) {
 void fd_step_passes(msl_sim* s) {
   const long long bs = (long long)s->npix();
   // band-limit V: FFT, |k| <= kmax, IFFT, * nf^2
-  row(s, ROW_FWD, RM_NONE, row_args(s, s->V.p, s->B.p, 1, bs));
+  row1(s, ROW_FWD, RM_NONE, row_args(s, s->V.p, s->B.p, 1, bs));
   ColArgs c = col_args(s, s->B.p, s->B.p, 1, bs);
   c.scale = s->nf * s->nf;
   col(s, COL_FWD_MUL_INV, CM_BAND, c);
-  row(s, ROW_INV, RM_NONE, row_args(s, s->B.p, s->V.p, 1, bs));
+  row1(s, ROW_INV, RM_NONE, row_args(s, s->B.p, s->V.p, 1, bs));
   // spectral Laplacian: FFT, * nf (-4 pi^2 k^2), IFFT, * nf
-  row(s, ROW_FWD, RM_NONE, row_args(s, s->Psi.p, s->G.p, 1, bs));
+  row1(s, ROW_FWD, RM_NONE, row_args(s, s->Psi.p, s->G.p, 1, bs));
   c = col_args(s, s->G.p, s->G.p, 1, bs);
   c.scale = s->nf * s->nf;
   col(s, COL_FWD_MUL_INV, CM_GRAD, c);
-  row(s, ROW_INV, RM_NONE, row_args(s, s->G.p, s->G.p, 1, bs));
+  row1(s, ROW_INV, RM_NONE, row_args(s, s->G.p, s->G.p, 1, bs));
   HIPC(launch_fd_update(s->G.p, s->PsiMinus.p, s->PsiPlus.p, s->Psi.p, s->V.p, bs, bs, s->sigma2, s->wavel, s->dzFD,
                         s->stream));
   // band-limit psi+
-  row(s, ROW_FWD, RM_NONE, row_args(s, s->PsiPlus.p, s->B.p, 1, bs));
+  row1(s, ROW_FWD, RM_NONE, row_args(s, s->PsiPlus.p, s->B.p, 1, bs));
   c = col_args(s, s->B.p, s->B.p, 1, bs);
   c.scale = s->nf * s->nf;
   col(s, COL_FWD_MUL_INV, CM_BAND, c);
-  row(s, ROW_INV, RM_NONE, row_args(s, s->B.p, s->PsiPlus.p, 1, bs));
+  row1(s, ROW_INV, RM_NONE, row_args(s, s->B.p, s->PsiPlus.p, 1, bs));
   // rotate: psi- <- psi, psi <- psi+
   std::swap(s->PsiMinus.p, s->Psi.p);
   std::swap(s->Psi.p, s->PsiPlus.p);
@@ -859,14 +864,14 @@ msl_status msl_multislice_step_conv(msl_sim* s, int it) {
     RowArgs r = row_args(s, src, s->PsiPlus.p, 1, bs);
     r.t = s->V.p;
     r.prune_out = prune;
-    row(s, ROW_FWD, RM_T, r);
+    row1(s, ROW_FWD, RM_T, r);
     ColArgs c = col_args(s, s->PsiPlus.p, s->PsiPlus.p, 1, bs);
     c.scale = s->nf * s->nf;
     c.tiles_lo = s->prune_tiles;
     col(s, COL_FWD_MUL_INV, CM_PROP, c);
     RowArgs ri = row_args(s, s->PsiPlus.p, s->Psi.p, 1, bs);
     ri.prune_in = prune;
-    row(s, ROW_INV, RM_NONE, ri);
+    row1(s, ROW_INV, RM_NONE, ri);
   }
   API_END(s)
 }

@@ -46,7 +46,8 @@ enum RowMul { RM_NONE = 0, RM_T = 1, RM_SEED = 2 };
   const float2 G* fd_pm;                                                                                 \
   const float2 G* fd_p0;                                                                                 \
   float fd_dz, fd_wavel;                                                                                 \
-  const float G* seed;       /* RM_SEED: real factor per element, src indexing */
+  const float G* seed;       /* RM_SEED: real factor per element, src indexing */                        \
+  int alone;                 /* 1: the caller's batch never varies (variant rules, launch_row) */
 struct RowArgs {
   MSL_ROW_ARGS()
 };
