@@ -218,7 +218,8 @@ template <int N, int RV> struct RowCfg {
 // (the adjoint reuses it instead of transforming again).
 // T_SLOTS (row loop only): each wave reads the transmission of its own slot
 // (RowArgs::t_index or b / t_group) instead of one shared by the launch
-enum { PRUNE_IN = 1, PRUNE_OUT = 2, STORE_AUX = 4, T_SLOTS = 8 };
+// V_REAL (ROW_INV_FD_FWD): the potential comes in real space
+enum { PRUNE_IN = 1, PRUNE_OUT = 2, STORE_AUX = 4, T_SLOTS = 8, V_REAL = 16 };
 // a workgroup's N table entries, requested when this is made and written to
 // LDS (and waited for by the workgroup) by store()
 template <int N, int NT> struct TwStage {
@@ -308,6 +309,26 @@ __device__ __forceinline__ void row_block(const A& a, long long blk, float2* lds
   staged();
   const LL L{lds + ln * LS, 1};
   constexpr bool ZIN = (FL & PRUNE_IN) != 0 && E % 4 == 0 && P::R1 % 4 == 0;  // first transform's input
+  // finite differences: the band-limited potential of the row, from its
+  // (kx, y) spectrum (in-band columns where the step is pruned)
+  float vr[MODE == ROW_INV_FD_FWD ? E : 1];
+  if constexpr (MODE == ROW_INV_FD_FWD) {
+    constexpr bool VZ = (FL & PRUNE_OUT) != 0 && E % 4 == 0 && P::R1 % 4 == 0;
+    const long long slot = a.t_index ? (long long)a.t_index[b] : (long long)(b / a.t_group);
+    const float2* tr = a.t + slot * a.t_bstride + (long long)y * N;
+    if constexpr ((FL & V_REAL) != 0) {
+#pragma unroll
+      for (int c = 0; c < E; ++c) vr[c] = tr[t + c * T].x;
+    } else {
+      float2 w[E];
+#pragma unroll
+      for (int c = 0; c < E; ++c)
+        w[c] = (!(FL & PRUNE_OUT) || BandBlocks<E>::active(c)) ? tr[t + c * T] : make_float2(0.f, 0.f);
+      fft_line<P, N, +1, S, LL, VZ>(w, t, stw, L);
+#pragma unroll
+      for (int c = 0; c < E; ++c) vr[c] = w[c].x;
+    }
+  }
   if constexpr (MODE == ROW_INV || MODE == ROW_INV_MUL_FWD || MODE == ROW_INV_FD_FWD)
     fft_line<P, N, +1, S, LL, ZIN>(v, t, stw, L);
   if constexpr ((FL & STORE_AUX) != 0) {
@@ -322,8 +343,6 @@ __device__ __forceinline__ void row_block(const A& a, long long blk, float2* lds
     // finiteDifferenceKernel, U.cu:995-1023: v holds the Laplacian G of psi
     if (ok) {
       const long long o = roff(a.dst_bstride);
-      const long long slot = a.t_index ? (long long)a.t_index[b] : (long long)(b / a.t_group);
-      const float2* vr = a.t + slot * a.t_bstride + (long long)y * N;
       const float dz = a.fd_dz, wavel = a.fd_wavel;
       const float al = 2.f * 3.14159f * dz / wavel;
       const float den = 1.f + al * al;
@@ -335,17 +354,15 @@ __device__ __forceinline__ void row_block(const A& a, long long blk, float2* lds
 #pragma unroll
       for (int c0 = 0; c0 < E; c0 += Q) {
         float2 pm[Q], p0[Q];
-        float vv[Q];
 #pragma unroll
         for (int q = 0; q < Q; ++q) {
           pm[q] = a.fd_pm[o + t + (c0 + q) * T];
           p0[q] = a.fd_p0[o + t + (c0 + q) * T];
-          vv[q] = vr[t + (c0 + q) * T].x;
         }
 #pragma unroll
         for (int q = 0; q < Q; ++q) {
           const float2 p = p0[q], g = v[c0 + q];
-          const float w = dz * dz * 4.f * 3.14159f * a.sigma * vv[q] / wavel;
+          const float w = dz * dz * 4.f * 3.14159f * a.sigma * vr[c0 + q] / wavel;
           const float2 u = make_float2(2.f * p.x - dz * dz * g.x - w * p.x, 2.f * p.y - dz * dz * g.y - w * p.y);
           v[c0 + q] = csub(cmul(rcp, u), cmul(ratio, pm[q]));
         }
@@ -553,30 +570,27 @@ hipError_t launch_prop_rows(const float* kx, const float* ky, int nx, int ny, fl
 }
 #endif
 
-template <int MUL, class A>
-__device__ __forceinline__ float2 kmul(const A& a, int x, int r, float kxv, float kyv, int2 pr) {
-  if constexpr (MUL == CM_SCALE) {
-    return make_float2(a.scale, 0.f);
-  } else if constexpr (MUL == CM_PROP || MUL == CM_PROPCONJ || MUL == CM_PROP_ZB || MUL == CM_PROPCONJ_ZB) {
-    // not reached: col_body applies the propagator itself
-    return make_float2(0.f, 0.f);
-  } else if constexpr (MUL == CM_BAND) {
+// real factor of the passes that filter by |k| (kx, ky in 1/A, scale included)
+template <int MUL, class A> __device__ __forceinline__ float kmul(const A& a, float kxv, float kyv) {
+  if constexpr (MUL == CM_BAND || MUL == CM_BAND_ZB) {
     // BandLimitKernel, U.cu:1037-1040: keeps |k| <= kmax
     const float k = sqrtf(kxv * kxv + kyv * kyv);
-    return make_float2(k <= a.kmax ? a.scale : 0.f, 0.f);
+    return k <= a.kmax ? a.scale : 0.f;
   } else if constexpr (MUL == CM_BANDGRAD) {
     // BandLimitKernel then gradKernel (U.cu:1037-1040, 959-960) as one factor
     const float k = sqrtf(kxv * kxv + kyv * kyv);
     const float gr = -4.f * 3.14159f * 3.14159f * (kxv * kxv + kyv * kyv);
-    return make_float2(k <= a.kmax ? a.scale * gr : 0.f, 0.f);
-  } else {  // CM_GRAD: gradKernel, U.cu:959-960
-    return make_float2(a.scale * -4.f * 3.14159f * 3.14159f * (kxv * kxv + kyv * kyv), 0.f);
+    return k <= a.kmax ? a.scale * gr : 0.f;
+  } else if constexpr (MUL == CM_GRAD) {  // gradKernel, U.cu:959-960
+    return a.scale * -4.f * 3.14159f * 3.14159f * (kxv * kxv + kyv * kyv);
+  } else {
+    return a.scale;
   }
 }
 
 template <int MODE> struct ColModeTraits {
-  static constexpr bool FWD = MODE == COL_FWD || MODE == COL_FWD_MUL_INV || MODE == COL_FWD_MUL || MODE == COL_FWD_DETECT;
-  static constexpr bool MULT = MODE == COL_FWD_MUL_INV || MODE == COL_FWD_MUL || MODE == COL_FWD_DETECT || MODE == COL_MUL_INV;
+  static constexpr bool FWD = MODE == COL_FD || MODE == COL_FWD || MODE == COL_FWD_MUL_INV || MODE == COL_FWD_MUL || MODE == COL_FWD_DETECT;
+  static constexpr bool MULT = MODE == COL_FD || MODE == COL_FWD_MUL_INV || MODE == COL_FWD_MUL || MODE == COL_FWD_DETECT || MODE == COL_MUL_INV;
   static constexpr bool INV = MODE == COL_INV || MODE == COL_FWD_MUL_INV || MODE == COL_MUL_INV;
 };
 
@@ -585,23 +599,24 @@ template <int MODE, int MUL> constexpr bool needs_rows() {
          (MUL == CM_PROP || MUL == CM_PROPCONJ || MUL == CM_PROP_ZB || MUL == CM_PROPCONJ_ZB);
 }
 
+template <int MODE, int MUL> constexpr bool needs_k() {
+  return ColModeTraits<MODE>::MULT &&
+         (MUL == CM_BAND || MUL == CM_BAND_ZB || MUL == CM_GRAD || MUL == CM_BANDGRAD);
+}
+
 // FFT / multiply / IFFT of one column held canonically by T threads; pr and
-// pxv are the column's band rows and propagator factor, py the rows' factors
-template <class P, int N, int MODE, int MUL, class S, class LL, class A, class PY>
+// pxv are the column's band rows and propagator factor, kxv its frequency, py
+// the rows' propagator factors and ky their frequencies
+template <class P, int N, int MODE, int MUL, class S, class LL, class A, class PY, class KY>
 __device__ __forceinline__ void col_body(float2 (&v)[N / P::T], int t, int x, const A& a, const LL& L,
-                                         const float2* tw, int2 pr, float2 pxv, const PY py) {
+                                         const float2* tw, int2 pr, float2 pxv, const PY py, float kxv, const KY ky) {
   using Tr = ColModeTraits<MODE>;
   constexpr int T = P::T, E = N / T;
   if constexpr (Tr::FWD) fft_line<P, N, -1, S>(v, t, tw, L);
-  // frequencies are read only by modes that need them (scale-only passes may
-  // run without k-grids)
-  constexpr bool NEEDK = (Tr::MULT && (MUL == CM_BAND || MUL == CM_GRAD || MUL == CM_BANDGRAD));
   constexpr bool NEEDROWS = needs_rows<MODE, MUL>();
   constexpr bool CONJ = MUL == CM_PROPCONJ || MUL == CM_PROPCONJ_ZB;
   // the propagator zeroes rows N/4 .. 3N/4 - 1 (canonical blocks E/4 .. 3E/4 - 1)
   constexpr bool ZB = (MUL == CM_PROP_ZB || MUL == CM_PROPCONJ_ZB) && E % 4 == 0 && P::R1 % 4 == 0;
-  float kxv = 0.f;
-  if constexpr (NEEDK) kxv = a.kx[x];
   if constexpr (NEEDROWS) {
     // propagator inside |k| < kmax (rows per column from k_prop_rows): the
     // factor is loaded for every row and zeroed by a multiplier, so the
@@ -617,12 +632,7 @@ __device__ __forceinline__ void col_body(float2 (&v)[N / P::T], int t, int x, co
     }
   } else if constexpr (Tr::MULT) {
 #pragma unroll
-    for (int c = 0; c < E; ++c) {
-      const int r = t + c * T;
-      float kyv = 0.f;
-      if constexpr (NEEDK) kyv = a.ky[r];
-      v[c] = cmul(v[c], kmul<MUL>(a, x, r, kxv, kyv, pr));
-    }
+    for (int c = 0; c < E; ++c) v[c] = cscale(v[c], kmul<MUL>(a, kxv, needs_k<MODE, MUL>() ? ky[t + c * T] : 0.f));
   } else if (a.scale != 1.0f) {
 #pragma unroll
     for (int c = 0; c < E; ++c) v[c] = cscale(v[c], a.scale);
@@ -634,10 +644,11 @@ __device__ __forceinline__ void col_body(float2 (&v)[N / P::T], int t, int x, co
 // (col, t) holds rows t + c T of column col; workgroup barriers
 // launched tile bx (of nbx per wave) of wave b; lds holds Cfg::LDS elements,
 // stw the twiddles of length N
-// (staged() as in row_block; py the propagator's row factors)
-template <int N, int MODE, int MUL, class Cfg, class A, class PY, class F>
+// (staged() as in row_block; py the propagator's row factors, ky the rows'
+// frequencies)
+template <int N, int MODE, int MUL, class Cfg, class A, class PY, class KY, class F>
 __device__ __forceinline__ void col_block(const A& a, int bx, int b, int nbx, float2* lds, const float2* stw,
-                                          const PY py, F staged) {
+                                          const PY py, const KY ky, F staged) {
   constexpr int T = Cfg::T, E = N / T, C = Cfg::C;
   const int col = Cfg::WAVECOL ? threadIdx.x / T : threadIdx.x % C;
   const int t = Cfg::WAVECOL ? threadIdx.x % T : threadIdx.x / C;
@@ -662,14 +673,39 @@ __device__ __forceinline__ void col_block(const A& a, int bx, int b, int nbx, fl
     pr = a.prop_rows[x];
     pxv = a.px[x];
   }
+  float kxv = 0.f;
+  if constexpr (needs_k<MODE, MUL>()) kxv = a.kx[x];
   staged();
   using LL = LdsLine<Cfg::SH>;
   const LL L = Cfg::INTERLEAVED ? LL{lds + col, C} : LL{lds + col * Cfg::LSC, 1};
   if constexpr (Cfg::DUAL) {
     const DualLine<LL> D{L, LL{lds + N * C + col, C}};
-    col_body<typename Cfg::P, N, MODE, MUL, S>(v, t, x, a, D, stw, pr, pxv, py);
+    col_body<typename Cfg::P, N, MODE, MUL, S>(v, t, x, a, D, stw, pr, pxv, py, kxv, ky);
   } else {
-    col_body<typename Cfg::P, N, MODE, MUL, S>(v, t, x, a, L, stw, pr, pxv, py);
+    if constexpr (MODE == COL_FD) {
+      // the finite-difference step's two filters of one spectrum: band limit
+      // into dst, band limit and Laplacian into dst2
+      using P = typename Cfg::P;
+      constexpr bool ZB = MUL == CM_BAND_ZB && E % 4 == 0 && P::R1 % 4 == 0;
+      fft_line<P, N, -1, S>(v, t, stw, L);
+      float2 w[E];
+#pragma unroll
+      for (int c = 0; c < E; ++c) {
+        const float kyv = ky[t + c * T];
+        w[c] = cscale(v[c], kmul<CM_BANDGRAD>(a, kxv, kyv));
+        v[c] = cscale(v[c], kmul<CM_BAND>(a, kxv, kyv));
+      }
+      fft_line<P, N, +1, S, LL, ZB>(w, t, stw, L);
+      {
+        float2* dst = a.dst2 + (long long)b * a.dst_bstride;
+        const unsigned o0 = (unsigned)t * (unsigned)nx + (unsigned)x, step = (unsigned)T * (unsigned)nx;
+#pragma unroll
+        for (int c = 0; c < E; ++c) dst[o0 + (unsigned)c * step] = w[c];
+      }
+      fft_line<P, N, +1, S, LL, ZB>(v, t, stw, L);
+    } else {
+      col_body<typename Cfg::P, N, MODE, MUL, S>(v, t, x, a, L, stw, pr, pxv, py, kxv, ky);
+    }
   }
   if constexpr (MODE == COL_FWD_DETECT) {
     const float kxv = a.kx[x];
@@ -710,14 +746,17 @@ __global__ void __launch_bounds__((ColCfg<N, CV>::THREADS), (ColCfg<N, CV>::MIN_
   __shared__ float2 stw[N];  // twiddles staged in LDS
   // and the propagator's row factors: read between the transforms, where a
   // load from memory would stall the workgroup
-  constexpr bool ROWS = needs_rows<MODE, MUL>();
+  constexpr bool ROWS = needs_rows<MODE, MUL>(), FREQ = needs_k<MODE, MUL>();
   __shared__ float2 spy[ROWS ? N : 1];
+  __shared__ float sky[FREQ ? N : 1];
   const TwStage<N, Cfg::THREADS> tws(a.tw);
   const TwStage<ROWS ? N : 1, Cfg::THREADS> pys(ROWS ? a.py : a.tw);
+  if constexpr (FREQ)
+    for (int i = threadIdx.x; i < N; i += Cfg::THREADS) sky[i] = a.ky[i];
   // logical (tile, wave) of this workgroup, XCD-aware
   const long long gid = xcd_remap((long long)blockIdx.y * gridDim.x + blockIdx.x, (long long)gridDim.x * gridDim.y);
   col_block<N, MODE, MUL, Cfg>(a, (int)(gid % gridDim.x), (int)(gid / gridDim.x), (int)gridDim.x, lds, stw,
-                               (const float2*)spy, [&] {
+                               (const float2*)spy, (const float*)sky, [&] {
                                  if constexpr (ROWS) pys.put(spy);
                                  tws.store(stw);
                                });
@@ -867,10 +906,10 @@ __global__ void __launch_bounds__(512) k_col_group(const PassGroup<ColArgs>* g, 
   for (int i = threadIdx.x; i < n; i += 512) stw[i] = a.tw[i];
   __syncthreads();
   switch (n) {
-    case 256: col_block<256, MODE, MUL, GroupCol<256>>(a, bx, b, nbx, lds, stw, a.py, [] {}); break;
-    case 512: col_block<512, MODE, MUL, GroupCol<512>>(a, bx, b, nbx, lds, stw, a.py, [] {}); break;
-    case 1024: col_block<1024, MODE, MUL, GroupCol<1024>>(a, bx, b, nbx, lds, stw, a.py, [] {}); break;
-    default: col_block<2048, MODE, MUL, GroupCol<2048>>(a, bx, b, nbx, lds, stw, a.py, [] {}); break;
+    case 256: col_block<256, MODE, MUL, GroupCol<256>>(a, bx, b, nbx, lds, stw, a.py, a.ky, [] {}); break;
+    case 512: col_block<512, MODE, MUL, GroupCol<512>>(a, bx, b, nbx, lds, stw, a.py, a.ky, [] {}); break;
+    case 1024: col_block<1024, MODE, MUL, GroupCol<1024>>(a, bx, b, nbx, lds, stw, a.py, a.ky, [] {}); break;
+    default: col_block<2048, MODE, MUL, GroupCol<2048>>(a, bx, b, nbx, lds, stw, a.py, a.ky, [] {}); break;
   }
 }
 
@@ -991,7 +1030,8 @@ static hipError_t row_nv(int mode, int mul, const RowArgs& a, hipStream_t s) {
   const long long nlines = (long long)a.nbatch * a.ny;
   if (nlines <= 0) return hipSuccess;
   dim3 grid((unsigned)((nlines + LINES - 1) / LINES)), block(LINES * T);
-  const int fl = (a.prune_in ? PRUNE_IN : 0) | (a.prune_out ? PRUNE_OUT : 0) | (a.aux ? STORE_AUX : 0);
+  const int fl = (a.prune_in ? PRUNE_IN : 0) | (a.prune_out ? PRUNE_OUT : 0) | (a.aux ? STORE_AUX : 0) |
+                 (a.fd_vreal ? V_REAL : 0);
   if (a.aux && mode != ROW_INV_MUL_FWD) return hipErrorInvalidValue;
   if (mode == ROW_INV_FD_FWD && (!a.fd_pm || !a.fd_p0 || !a.t)) return hipErrorInvalidValue;
   if (mul == RM_SEED && (mode != ROW_FWD || !a.seed)) return hipErrorInvalidValue;
@@ -1013,6 +1053,9 @@ static hipError_t row_nv(int mode, int mul, const RowArgs& a, hipStream_t s) {
     MSL_ROW(ROW_INV_MUL_FWD, RM_T, PRUNE_IN | PRUNE_OUT | STORE_AUX);
   else if (mode == ROW_INV_FD_FWD && mul == RM_T && fl == (PRUNE_IN | PRUNE_OUT))
     MSL_ROW(ROW_INV_FD_FWD, RM_T, PRUNE_IN | PRUNE_OUT);
+  else if (mode == ROW_INV_FD_FWD && mul == RM_T && fl == (PRUNE_IN | PRUNE_OUT | V_REAL))
+    MSL_ROW(ROW_INV_FD_FWD, RM_T, PRUNE_IN | PRUNE_OUT | V_REAL);
+  else if (mode == ROW_INV_FD_FWD && mul == RM_T && fl == PRUNE_OUT) MSL_ROW(ROW_INV_FD_FWD, RM_T, PRUNE_OUT);
   else if (mode == ROW_INV_FD_FWD && mul == RM_T && fl == 0) MSL_ROW(ROW_INV_FD_FWD, RM_T, 0);
   else return hipErrorInvalidValue;
 #undef MSL_ROW
@@ -1097,7 +1140,16 @@ static hipError_t col_nv(int mode, int mul, const ColArgs& a, hipStream_t s) {
     else if (mode == COL_FWD_MUL_INV && mul == CM_PROPCONJ_ZB) MSL_COL(COL_FWD_MUL_INV, CM_PROPCONJ_ZB);
     else if (mode == COL_FWD_MUL_INV && mul == CM_BAND) MSL_COL(COL_FWD_MUL_INV, CM_BAND);
     else if (mode == COL_FWD_MUL_INV && mul == CM_GRAD) MSL_COL(COL_FWD_MUL_INV, CM_GRAD);
-    else if (mode == COL_FWD_MUL_INV && mul == CM_BANDGRAD) MSL_COL(COL_FWD_MUL_INV, CM_BANDGRAD);
+    else if (mode == COL_FD) {
+      if constexpr (CV == 0 || CV == 3) {  // col_n sends it to no other
+        if (!a.dst2) return hipErrorInvalidValue;
+        if (mul == CM_BAND) MSL_COL(COL_FD, CM_BAND);
+        else if (mul == CM_BAND_ZB) MSL_COL(COL_FD, CM_BAND_ZB);
+        else return hipErrorInvalidValue;
+      } else {
+        return hipErrorInvalidValue;
+      }
+    }
     else if (mode == COL_FWD_MUL_INV && mul == CM_SCALE) MSL_COL(COL_FWD_MUL_INV, CM_SCALE);
     else if (mode == COL_FWD_MUL && mul == CM_PROP) MSL_COL(COL_FWD_MUL, CM_PROP);
     else if (mode == COL_FWD_MUL && mul == CM_SCALE) MSL_COL(COL_FWD_MUL, CM_SCALE);
@@ -1143,6 +1195,8 @@ static hipError_t col_n(int mode, int mul, const ColArgs& a, hipStream_t s, int 
     if (var == 4) return col_nv<N, 4>(mode, mul, a, s);
     return var == 2 ? col_nv<N, 2>(mode, mul, a, s) : col_nv<N, 0>(mode, mul, a, s);
   }
+  // the two filters of a finite-difference step: full or half-width tiles
+  if (mode == COL_FD) return var == 3 ? col_nv<N, 3>(mode, mul, a, s) : col_nv<N, 0>(mode, mul, a, s);
   if (var == 6) {
     if constexpr (ColCfg<N, 6>::WAVECOL) return col_nv<N, 6>(mode, mul, a, s);
     else return col_nv<N, 0>(mode, mul, a, s);
@@ -1201,6 +1255,12 @@ bool prop_rows_quarter(const float* hky, int ny, float kmax) {
   return !(std::sqrt(kxv * kxv + kyv * kyv) < kmax);
 }
 
+bool band_rows_quarter(const float* hky, int ny, float kmax) {
+  if (ny < 4) return false;
+  const float kyv = hky[ny / 4], kxv = 0.0f;
+  return !(std::sqrt(kxv * kxv + kyv * kyv) <= kmax);
+}
+
 // Column launches put the waves on grid.y, at most 65535 per launch: longer
 // batches run as consecutive launches over slices of the batch (the detector
 // pass, whose partial sums are indexed by wave, is refused instead).
@@ -1215,6 +1275,7 @@ hipError_t launch_col_v(int mode, int mul, const ColArgs& a, hipStream_t s, int 
       c.nbatch = (int)std::min<long long>(kMaxGridY, a.nbatch - b0);
       c.src = a.src + b0 * a.src_bstride;
       c.dst = a.dst + b0 * a.dst_bstride;
+      if (a.dst2) c.dst2 = a.dst2 + b0 * a.dst_bstride;
       const hipError_t e = launch_col_v(mode, mul, c, s, var);
       if (e != hipSuccess) return e;
     }
@@ -1225,6 +1286,7 @@ hipError_t launch_col_v(int mode, int mul, const ColArgs& a, hipStream_t s, int 
     if (mul == CM_PROP) mul = CM_PROP_ZB;
     else if (mul == CM_PROPCONJ) mul = CM_PROPCONJ_ZB;
   }
+  if (mode == COL_FD && mul == CM_BAND && a.zb_rows) mul = CM_BAND_ZB;
   switch (a.ny) {
     case 16: return col_len_16(mode, mul, a, s, var);
     case 32: return col_len_32(mode, mul, a, s, var);

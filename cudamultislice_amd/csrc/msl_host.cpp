@@ -361,6 +361,7 @@ void calc_vars(msl_sim* s, float ps, float df, int rx, int ry, float sizeZ, floa
     s->loadblocksy = (int)std::ceil(std::sqrt(5.0f) / ((s->MaxY - s->MinY) / 50.f));
   }
   s->loadslicesz = (int)std::ceil(std::sqrt(5.0f) / 1.0f);
+  s->fd_lap = false;
   s->have_calc = true;
   s->have_freqs = false;
   s->have_waves = false;
@@ -388,6 +389,10 @@ void precalc(msl_sim* s) {
   for (int x = rx / 4; x < 3 * rx / 4 && s->prune_tiles > 0; ++x)
     if (std::sqrt(s->hkx[x] * s->hkx[x] + 0.0f) < s->kmax) s->prune_tiles = 0;
   s->zb_rows = prop_rows_quarter(s->hky.data(), ry, s->kmax);
+  s->fd_zb = band_rows_quarter(s->hky.data(), ry, s->kmax);
+  s->fd_prune = s->prune_tiles > 0;
+  for (int x = rx / 4; x < 3 * rx / 4 && s->fd_prune; ++x)
+    if (std::sqrt(s->hkx[x] * s->hkx[x] + 0.0f) <= s->kmax) s->fd_prune = false;
   auto upload = [&](auto& d, const auto& v) {
     d.ensure(v.size());
     if (!v.empty()) HIPC(hipMemcpyAsync(d.p, v.data(), v.size() * sizeof(v[0]), hipMemcpyHostToDevice, s->stream));
@@ -427,6 +432,7 @@ void precalc(msl_sim* s) {
   HIPC(launch_prop_rows(s->kx.p, s->ky.p, rx, ry, s->kmax, s->prow.p, s->stream));
   HIPC(hipStreamSynchronize(s->stream));
   s->prop_dz = std::nanf("");
+  s->fd_lap = false;
   s->have_freqs = true;
 }
 
@@ -435,6 +441,7 @@ void alloc_waves(msl_sim* s) {
   s->PsiMinus.ensure(n); s->Psi.ensure(n); s->PsiPlus.ensure(n);
   s->V.ensure(n); s->G.ensure(n); s->B.ensure(n);
   s->red.ensure(4096);
+  s->fd_lap = false;
 }
 
 void potential(msl_sim* s, int mode, int first, int nslices, float dz, float zplane, int out_kind, void* out,
@@ -554,30 +561,53 @@ float adf_of(msl_sim* s, const float2* w, float inner, float outer) {
   return download_scalar(s, s->red.p + 2048);
 }
 
-// the finite-difference step of U.cu:2050-2083 on the fused passes (grids of
-// powers of two): band limit of V, Laplacian of psi, update, band limit of psi+
+// The finite-difference step of U.cu:2050-2083 on grids of powers of two: band
+// limit of V, Laplacian of psi, update, band limit of psi+.  psi+ is band
+// limited from the spectrum that also gives its Laplacian, so a step makes
+// the next step's Laplacian on the way, and V's last transform and the update
+// sit in one row pass: five passes (V rows, V columns, step rows, both
+// filters' columns, psi+ rows) instead of nine and an update kernel, 45 ->
+// 26 us a step at 256^2, where the launches' latency bounds them.
 void fd_step_passes(msl_sim* s) {
   const long long bs = (long long)s->npix();
-  // band-limit V: FFT, |k| <= kmax, IFFT, * nf^2
-  row1(s, ROW_FWD, RM_NONE, row_args(s, s->V.p, s->B.p, 1, bs));
+  const int tiles = s->fd_prune ? s->prune_tiles : 0;
+  // band-limited V in the (kx, y) domain: FFT, |k| <= kmax, IFFT_y, * nf^2
+  RowArgs rv = row_args(s, s->V.p, s->B.p, 1, bs);
+  rv.prune_out = s->fd_prune;
+  row1(s, ROW_FWD, RM_NONE, rv);
   ColArgs c = col_args(s, s->B.p, s->B.p, 1, bs);
   c.scale = s->nf * s->nf;
+  c.tiles_lo = tiles;
   col(s, COL_FWD_MUL_INV, CM_BAND, c);
-  row1(s, ROW_INV, RM_NONE, row_args(s, s->B.p, s->V.p, 1, bs));
-  // spectral Laplacian: FFT, * nf (-4 pi^2 k^2), IFFT, * nf
-  row1(s, ROW_FWD, RM_NONE, row_args(s, s->Psi.p, s->G.p, 1, bs));
-  c = col_args(s, s->G.p, s->G.p, 1, bs);
+  // spectral Laplacian of psi: FFT, * nf (-4 pi^2 k^2), IFFT_y, * nf
+  const bool had_lap = s->fd_lap;
+  if (!had_lap) {
+    row1(s, ROW_FWD, RM_NONE, row_args(s, s->Psi.p, s->G.p, 1, bs));
+    c = col_args(s, s->G.p, s->G.p, 1, bs);
+    c.scale = s->nf * s->nf;
+    col(s, COL_FWD_MUL_INV, CM_GRAD, c);
+  }
+  s->fd_lap = false;
+  RowArgs r = row_args(s, s->G.p, s->V.p, 1, bs);
+  r.prune_in = s->fd_prune && had_lap;  // a wave from elsewhere may hold any frequency
+  r.prune_out = s->fd_prune;
+  r.t = s->B.p;
+  r.fd_pm = s->PsiMinus.p;
+  r.fd_p0 = s->Psi.p;
+  r.fd_dz = s->dzFD;
+  r.fd_wavel = s->wavel;
+  r.sigma = s->sigma2;
+  row1(s, ROW_INV_FD_FWD, RM_T, r);
+  c = col_args(s, s->V.p, s->V.p, 1, bs);
+  c.dst2 = s->G.p;
   c.scale = s->nf * s->nf;
-  col(s, COL_FWD_MUL_INV, CM_GRAD, c);
-  row1(s, ROW_INV, RM_NONE, row_args(s, s->G.p, s->G.p, 1, bs));
-  HIPC(launch_fd_update(s->G.p, s->PsiMinus.p, s->PsiPlus.p, s->Psi.p, s->V.p, bs, bs, s->sigma2, s->wavel, s->dzFD,
-                        s->stream));
-  // band-limit psi+
-  row1(s, ROW_FWD, RM_NONE, row_args(s, s->PsiPlus.p, s->B.p, 1, bs));
-  c = col_args(s, s->B.p, s->B.p, 1, bs);
-  c.scale = s->nf * s->nf;
-  col(s, COL_FWD_MUL_INV, CM_BAND, c);
-  row1(s, ROW_INV, RM_NONE, row_args(s, s->B.p, s->PsiPlus.p, 1, bs));
+  c.tiles_lo = tiles;
+  c.zb_rows = s->fd_zb ? 1 : 0;
+  col(s, COL_FD, CM_BAND, c);
+  RowArgs ri = row_args(s, s->V.p, s->PsiPlus.p, 1, bs);
+  ri.prune_in = s->fd_prune;
+  row1(s, ROW_INV, RM_NONE, ri);
+  s->fd_lap = true;
   // rotate: psi- <- psi, psi <- psi+
   std::swap(s->PsiMinus.p, s->Psi.p);
   std::swap(s->Psi.p, s->PsiPlus.p);
@@ -852,6 +882,7 @@ msl_status msl_multislice_step_conv(msl_sim* s, int it) {
   require(it >= 1, MSL_ERR_ARG, "iterations count from 1");
   require(s->cancel == 0, MSL_ERR_CANCELLED, "cancelled");
   const long long bs = (long long)s->npix();
+  s->fd_lap = false;
   potential(s, s->potmode, it, 1, s->conventionaldz, 0.f, 0, s->V.p, bs);
   ensure_prop(s, s->conventionaldz);
   const float2* src = (it == 1) ? s->PsiMinus.p : s->Psi.p;
@@ -923,6 +954,7 @@ msl_status msl_multislice_step_rs(msl_sim* s, int it) {
     const float d = 1.0f * (float)it;
     zc = h - d;
   }
+  s->fd_lap = false;
   potential(s, 3, 0, 1, 1.0f, zc, 1, s->V.p, n);
   float2 *a = s->PsiPlus.p, *b = s->G.p;
   for (int m = 1; m <= 10; ++m) {
@@ -1287,6 +1319,7 @@ msl_status msl_set_wave(msl_sim* s, int which, const float* in) {
   API_BEGIN(s)
   require(s->have_waves && in, MSL_ERR_STATE, "no waves");
   float2* d = which == 0 ? s->Psi.p : which == 1 ? s->PsiMinus.p : s->PsiPlus.p;
+  s->fd_lap = false;
   h2d(s, d, in, s->npix() * sizeof(float2));
   API_END(s)
 }

@@ -112,6 +112,12 @@ struct msl_sim {
   double nfd = 0;
   int prune_tiles = 0;  // > 0: columns N/4 <= x < 3N/4 are outside the propagator band
   bool zb_rows = false;  // rows N/4 <= y < 3N/4 are outside the propagator band (every column)
+  // the same two of the finite differences' band limit |k| <= kmax
+  bool fd_prune = false, fd_zb = false;
+  // G holds the Laplacian of Psi in the (kx, y) domain (left by a
+  // finite-difference step for the next; anything else that writes Psi, or
+  // uses G, clears it)
+  bool fd_lap = false;
   std::vector<float> hkx, hky;
   // the k-grids and twiddles of both axes, one upload; kx, ky, twx, twy point
   // into it

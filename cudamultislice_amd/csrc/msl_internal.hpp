@@ -12,9 +12,11 @@ namespace msl {
 // Row pass: one transform along x (contiguous) per (wave, row) line.
 enum RowMode { ROW_FWD = 0, ROW_INV = 1, ROW_INV_MUL_FWD = 2, ROW_INV_FD_FWD = 3 };
 // ROW_INV_FD_FWD: the finite-difference step of one row (finiteDifferenceKernel,
-// U.cu:995-1023) between the transforms: IFFT_x of the Laplacian spectrum
-// (src), psi+ from it, psi- (fd_pm), psi (fd_p0) and V (t, real part, slot
-// indexing as RM_T), then FFT_x of psi+ into dst.
+// U.cu:995-1023) between the transforms: IFFT_x of the band-limited V (t, in
+// the (kx, y) domain, slot indexing as RM_T; its real part is used) and of the
+// Laplacian spectrum (src), psi+ from them, psi- (fd_pm) and psi (fd_p0), then
+// FFT_x of psi+ into dst.  prune_out also says that V's columns outside the
+// band were not written.
 // pointwise factor applied between the (optional) inverse and forward
 // transforms: none, a stored transmission t, or (RM_SEED, with ROW_FWD) twice
 // a real array in the wave's own layout: the gradient 2 dL/dI psi of an
@@ -46,6 +48,7 @@ enum RowMul { RM_NONE = 0, RM_T = 1, RM_SEED = 2 };
   const float2 G* fd_pm;                                                                                 \
   const float2 G* fd_p0;                                                                                 \
   float fd_dz, fd_wavel;                                                                                 \
+  int fd_vreal;              /* t holds the band-limited V in real space instead */                      \
   const float G* seed;       /* RM_SEED: real factor per element, src indexing */                        \
   int alone;                 /* 1: the caller's batch never varies (variant rules, launch_row) */
 struct RowArgs {
@@ -53,20 +56,26 @@ struct RowArgs {
 };
 
 // Column pass: one transform along y (stride nx) per (wave, column).
-enum ColMode { COL_FWD = 0, COL_INV = 1, COL_FWD_MUL_INV = 2, COL_FWD_MUL = 3, COL_FWD_DETECT = 4, COL_MUL_INV = 5 };
+enum ColMode { COL_FWD = 0, COL_INV = 1, COL_FWD_MUL_INV = 2, COL_FWD_MUL = 3, COL_FWD_DETECT = 4, COL_MUL_INV = 5,
+               // forward, then both filters of a finite-difference step and their inverses: band
+               // limit into dst, band limit times Laplacian into dst2 (CM_BAND)
+               COL_FD = 6 };
 // k-space factor: none (scale only), Fresnel propagator with strict
 // |k| < kmax, band limit |k| <= kmax, spectral Laplacian, conjugate propagator
 enum ColMul { CM_SCALE = 0, CM_PROP = 1, CM_BAND = 2, CM_GRAD = 3, CM_PROPCONJ = 4, CM_BANDGRAD = 5,
               // CM_PROP / CM_PROPCONJ where rows ny/4 .. 3ny/4 - 1 lie outside the band for every
               // column (ColArgs::zb_rows): the inverse transform skips their zeros.  Chosen by
               // launch_col from zb_rows; callers pass CM_PROP / CM_PROPCONJ.
-              CM_PROP_ZB = 6, CM_PROPCONJ_ZB = 7 };
+              CM_PROP_ZB = 6, CM_PROPCONJ_ZB = 7,
+              // COL_FD where rows ny/4 .. 3ny/4 - 1 fail |k| <= kmax (ColArgs::zb_rows; by launch_col)
+              CM_BAND_ZB = 8 };
 // CM_BANDGRAD: band limit and spectral Laplacian in one factor (the Laplacian
 // of a band-limited wave, from the spectrum before the band limit)
 
 #define MSL_COL_ARGS(G)                                                                                   \
   const float2 G* src;                                                                                   \
   float2 G* dst;                                                                                         \
+  float2 G* dst2;            /* COL_FD */                                                                \
   long long src_bstride, dst_bstride;                                                                    \
   int nx, ny, nbatch;                                                                                    \
   const float G* kx;         /* FP32 spatial frequencies (1/A) */                                        \
@@ -87,7 +96,8 @@ enum ColMul { CM_SCALE = 0, CM_PROP = 1, CM_BAND = 2, CM_GRAD = 3, CM_PROPCONJ =
   /* > 0: launch only the tiles_lo column tiles at each end of kx (band-limited data); */                \
   /* COL_FWD_DETECT partials are then indexed by launched tile */                                        \
   int tiles_lo;                                                                                          \
-  /* 1: rows ny/4 .. 3ny/4 - 1 are outside |k| < kmax for every column (prop_rows_quarter) */            \
+  /* 1: rows ny/4 .. 3ny/4 - 1 are outside |k| < kmax for every column (prop_rows_quarter; COL_FD:        \
+     outside |k| <= kmax, band_rows_quarter) */                                                          \
   int zb_rows;
 struct ColArgs {
   MSL_COL_ARGS()
@@ -101,6 +111,8 @@ int col_tile(int ny);  // columns per column-pass workgroup (detector layout)
 // every column: the row ny/4 fails it at kx = 0 (the FP32 test of
 // k_prop_rows; |ky| only grows towards ny/2 and |k| >= |ky|)
 bool prop_rows_quarter(const float* hky, int ny, float kmax);
+// the same of the band limit's test |k| <= kmax
+bool band_rows_quarter(const float* hky, int ny, float kmax);
 int band_tiles_lo(int nx);  // column tiles per end covering x < N/4, x >= 3N/4 (0: no pruning)
 // pass layout variants per length (kind 0 row, 1 column), see k_pass.hip
 int pass_variant(int kind, int n);

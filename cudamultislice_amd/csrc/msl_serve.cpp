@@ -84,9 +84,7 @@ class Runner {
     np_ = (long long)n_ * n_;
     ntiles_ = n_ / col_tile(n_);
     prune_ = !fd && cs->prune_tiles > 0;
-    fd_prune_ = fd && cs->prune_tiles > 0;
-    for (int x = n_ / 4; x < 3 * n_ / 4 && fd_prune_; ++x)
-      if (std::sqrt(cs->hkx[x] * cs->hkx[x] + 0.0f) <= cs->kmax) fd_prune_ = false;
+    fd_prune_ = fd && cs->fd_prune;
   }
 
   // jobs of one class, sharing the tables of cs
@@ -98,7 +96,7 @@ class Runner {
     if (probes) probe_norm();
     else scratch_.ensure(np_);
     const long long budget = p_.budget_bytes > 0 ? p_.budget_bytes : (32LL << 30);
-    const long long wave_b = np_ * 8 * (fd ? (fd_prune_ ? 6 : 5) : 1), slot_b = np_ * 8 * (fd ? 2 : 1);
+    const long long wave_b = np_ * 8 * (fd ? 5 : 1), slot_b = np_ * 8 * (fd ? 2 : 1);
     const long long maxw = std::max<long long>(1, (budget - slot_b) / (wave_b + slot_b));
     std::vector<Item> items;
     for (int j : ids) {
@@ -299,7 +297,6 @@ class Runner {
   msl_sim* cs_ = nullptr;
   bool fd_ = false, prune_ = false;
   bool fd_prune_ = false;  // finite differences: band limit |k| <= kmax leaves N/4 <= x < 3N/4 empty
-  DBuf<float2> Z1_;
   int n_ = 0, ntiles_ = 0;
   long long np_ = 0;
   float norm_ = 1.f;
@@ -494,7 +491,6 @@ class Runner {
     DBuf<float2> Pm, P0, Pp, G, Bt, V, Vt;
     DBuf<float> partial, adf;
     Pm.ensure(wn); P0.ensure(wn); Pp.ensure(wn); G.ensure(wn); Bt.ensure(wn);
-    if (fd_prune_) Z1_.ensure(wn);
     V.ensure((size_t)J * np_); Vt.ensure((size_t)J * np_);
     partial.ensure((size_t)L.nw * ntiles_);
     adf.ensure(L.nw);
@@ -522,14 +518,14 @@ class Runner {
     xform(pm, p0, p0, L.nw, CM_PROP);
     const double t0 = now_ms();
     const float dzfd = cs_->dzFD;
-    // Band-limited grids: the step runs fused.  Y holds the Laplacian of psi
-    // in the (kx, y) domain.  Per step: one row pass (IF_x of Y, the
-    // finite-difference update, F_x of psi+ into Z), two column passes over the
-    // in-band columns of Z (band limit -> Z1, band limit times Laplacian -> Y
-    // for the next step) and one row pass IF_x(Z1) -> band-limited psi+: four
-    // passes instead of the three transforms and the update of U.cu:2040-2083.
+    // Band-limited grids: the step runs fused, as the single handle's
+    // (fd_step_passes): Y holds the Laplacian of psi in the (kx, y) domain.
+    // Per step: V's rows and columns for the running jobs, one row pass (IF_x of Y, the finite-difference update, F_x of psi+ into
+    // Z), one column pass over the in-band columns of Z (band limit back into
+    // Z, band limit times Laplacian into Y for the next step) and one row pass
+    // IF_x(Z) -> band-limited psi+.
     if (fd_prune_) {
-      float2 *Y = G.p, *Z = Bt.p, *Z1 = Z1_.p;
+      float2 *Y = G.p, *Z = Bt.p;
       row(cs_, ROW_FWD, RM_NONE, row_args(cs_, p0, Y, L.nw, np_));
       {
         ColArgs c = col_args(cs_, Y, Y, L.nw, np_);
@@ -544,10 +540,28 @@ class Runner {
           const float zc = (jb.s->MaxZ - jb.s->MinZ) - dzfd * (float)it;
           potential(jb.s.get(), 2, 0, 1, 1.0f, zc, 1, V.p + (size_t)jb.slot * np_, np_);
         }
-        xform(V.p, Vt.p, V.p, Ja, CM_BAND);  // band-limited V
+        // band-limited V in the (kx, y) domain
+        RowArgs rv = row_args(cs_, V.p, Vt.p, Ja, np_);
+        rv.prune_out = 1;
+        row(cs_, ROW_FWD, RM_NONE, rv);
+        ColArgs cv = col_args(cs_, Vt.p, Vt.p, Ja, np_);
+        cv.scale = nf2;
+        cv.tiles_lo = cs_->prune_tiles;
+        col(cs_, COL_FWD_MUL_INV, CM_BAND, cv);
+        // its last transform once per job where several waves read it (in the
+        // row pass of every wave 1.4 times that pass's time at 1024), in the
+        // row pass otherwise
+        const bool vreal = A >= 2 * Ja;
+        if (vreal) {
+          RowArgs ri = row_args(cs_, Vt.p, V.p, Ja, np_);
+          ri.prune_in = 1;
+          row(cs_, ROW_INV, RM_NONE, ri);
+          st_.launches += 1;
+        }
         RowArgs r = row_args(cs_, Y, Z, A, np_);
         r.prune_in = r.prune_out = 1;
-        r.t = V.p;
+        r.t = vreal ? V.p : Vt.p;
+        r.fd_vreal = vreal ? 1 : 0;
         r.t_index = L.tidx.p;
         r.t_bstride = np_;
         r.fd_pm = pm;
@@ -556,16 +570,16 @@ class Runner {
         r.fd_wavel = cs_->wavel;
         r.sigma = cs_->sigma2;
         row(cs_, ROW_INV_FD_FWD, RM_T, r);
-        ColArgs c = col_args(cs_, Z, Z1, A, np_);
+        ColArgs c = col_args(cs_, Z, Z, A, np_);
+        c.dst2 = Y;
         c.scale = nf2;
         c.tiles_lo = cs_->prune_tiles;
-        col(cs_, COL_FWD_MUL_INV, CM_BAND, c);
-        c.dst = Y;
-        col(cs_, COL_FWD_MUL_INV, CM_BANDGRAD, c);
-        RowArgs ri = row_args(cs_, Z1, pp, A, np_);
+        c.zb_rows = cs_->fd_zb ? 1 : 0;
+        col(cs_, COL_FD, CM_BAND, c);
+        RowArgs ri = row_args(cs_, Z, pp, A, np_);
         ri.prune_in = 1;
         row(cs_, ROW_INV, RM_NONE, ri);
-        st_.launches += 4;
+        st_.launches += 5;
         std::swap(pm, p0);
         std::swap(p0, pp);
         st_.wave_slices += A;
