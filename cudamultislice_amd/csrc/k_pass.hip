@@ -219,7 +219,9 @@ template <int N, int RV> struct RowCfg {
 // T_SLOTS (row loop only): each wave reads the transmission of its own slot
 // (RowArgs::t_index or b / t_group) instead of one shared by the launch
 // V_REAL (ROW_INV_FD_FWD): the potential comes in real space
-enum { PRUNE_IN = 1, PRUNE_OUT = 2, STORE_AUX = 4, T_SLOTS = 8, V_REAL = 16 };
+// STORE_INT (ROW_INV): |wave|^2 into inten, the wave itself only where dst is
+// given (a pass of its own read and wrote the exit waves once more)
+enum { PRUNE_IN = 1, PRUNE_OUT = 2, STORE_AUX = 4, T_SLOTS = 8, V_REAL = 16, STORE_INT = 32 };
 // a workgroup's N table entries, requested when this is made and written to
 // LDS (and waited for by the workgroup) by store()
 template <int N, int NT> struct TwStage {
@@ -393,6 +395,13 @@ __device__ __forceinline__ void row_block(const A& a, long long blk, float2* lds
   }
   if constexpr (MODE == ROW_FWD) fft_line<P, N, -1, S, LL, ZIN>(v, t, stw, L);
   if constexpr (MODE == ROW_INV_MUL_FWD || MODE == ROW_INV_FD_FWD) fft_line<P, N, -1, S>(v, t, stw, L);
+  if constexpr ((FL & STORE_INT) != 0) {
+    if (!ok) return;
+    float* in = a.inten + roff(a.dst_bstride);
+#pragma unroll
+    for (int c = 0; c < E; ++c) in[t + c * T] = v[c].x * v[c].x + v[c].y * v[c].y;
+    if (!a.dst) return;
+  }
   if (ok) {
     float2* row = a.dst + roff(a.dst_bstride);
 #pragma unroll
@@ -1031,7 +1040,7 @@ static hipError_t row_nv(int mode, int mul, const RowArgs& a, hipStream_t s) {
   if (nlines <= 0) return hipSuccess;
   dim3 grid((unsigned)((nlines + LINES - 1) / LINES)), block(LINES * T);
   const int fl = (a.prune_in ? PRUNE_IN : 0) | (a.prune_out ? PRUNE_OUT : 0) | (a.aux ? STORE_AUX : 0) |
-                 (a.fd_vreal ? V_REAL : 0);
+                 (a.fd_vreal ? V_REAL : 0) | (a.inten ? STORE_INT : 0);
   if (a.aux && mode != ROW_INV_MUL_FWD) return hipErrorInvalidValue;
   if (mode == ROW_INV_FD_FWD && (!a.fd_pm || !a.fd_p0 || !a.t)) return hipErrorInvalidValue;
   if (mul == RM_SEED && (mode != ROW_FWD || !a.seed)) return hipErrorInvalidValue;
@@ -1044,6 +1053,9 @@ static hipError_t row_nv(int mode, int mul, const RowArgs& a, hipStream_t s) {
   else if (mode == ROW_FWD && mul == RM_SEED && fl == PRUNE_OUT) MSL_ROW(ROW_FWD, RM_SEED, PRUNE_OUT);
   else if (mode == ROW_INV && mul == RM_NONE && fl == 0) MSL_ROW(ROW_INV, RM_NONE, 0);
   else if (mode == ROW_INV && mul == RM_NONE && fl == PRUNE_IN) MSL_ROW(ROW_INV, RM_NONE, PRUNE_IN);
+  else if (mode == ROW_INV && mul == RM_NONE && fl == STORE_INT) MSL_ROW(ROW_INV, RM_NONE, STORE_INT);
+  else if (mode == ROW_INV && mul == RM_NONE && fl == (PRUNE_IN | STORE_INT))
+    MSL_ROW(ROW_INV, RM_NONE, PRUNE_IN | STORE_INT);
   else if (mode == ROW_INV_MUL_FWD && mul == RM_T && fl == 0) MSL_ROW(ROW_INV_MUL_FWD, RM_T, 0);
   else if (mode == ROW_INV_MUL_FWD && mul == RM_T && fl == PRUNE_OUT) MSL_ROW(ROW_INV_MUL_FWD, RM_T, PRUNE_OUT);
   else if (mode == ROW_INV_MUL_FWD && mul == RM_T && fl == (PRUNE_IN | PRUNE_OUT))

@@ -122,13 +122,10 @@ float2* tslot(msl_diff* d, int i) { return d->tall.p + (size_t)(i - 1) * d->np()
 
 // slice i (1-based) forward: z_{i-1} (psi0 in real space for i = 1) -> z_i
 // at dst, through W (dst may be W: both passes work in place).  With wout
-// the row pass also stores w_i = IF_x(z_{i-1}) there.  With make_t the
-// slice's transmission exp(i sigma V_i) is evaluated once into its slot and
-// read by the row pass for every probe (evaluated per line, the same sincosf
-// would run once per probe); the backward's recomputation and adjoint passes
-// read the slots the forward wrote.
-void fwd_slice(msl_diff* d, int i, const float2* zprev, float2* dst, float2* wout, bool make_t, hipStream_t s) {
-  if (make_t) HC(launch_transmission(d->V + (size_t)(i - 1) * d->np(), tslot(d, i), d->np(), d->sigma, s));
+// the row pass also stores w_i = IF_x(z_{i-1}) there.  The row pass reads the
+// slice's transmission exp(i sigma V_i) from its slot for every probe
+// (evaluated per line, the same sincosf would run once per probe).
+void fwd_slice(msl_diff* d, int i, const float2* zprev, float2* dst, float2* wout, hipStream_t s) {
   RowArgs r = rargs(d, zprev, d->W.p, i > 1, true);
   r.t = tslot(d, i);
   r.t_group = d->B;
@@ -299,13 +296,18 @@ msl_status diff_forward(msl_diff* d, const float* V, const void* psi0, float* in
     const int last_base = (d->S - 1) * d->K;
     const float2* zprev = d->psi0;
     d->have_forward = false;
+    // every slice's transmission in one launch (the backward's recomputation
+    // and adjoint passes read them too)
+    HC(launch_transmission(d->V, d->tall.p, (long long)d->ns * d->np(), d->sigma, s));
     for (int i = 1; i <= d->ns; ++i) {
       float2* dst = (keep && i % d->K == 0 && i < d->ns) ? ckpt_slot(d, i) : d->W.p;
-      fwd_slice(d, i, zprev, dst, keep && i > last_base ? wslot(d, i, last_base) : nullptr, true, s);
+      fwd_slice(d, i, zprev, dst, keep && i > last_base ? wslot(d, i, last_base) : nullptr, s);
       zprev = dst;
     }
-    HC(launch_row(ROW_INV, RM_NONE, rargs(d, zprev, d->exitw.p, true, false), s));
-    HC(launch_intensity(d->exitw.p, inten, (long long)d->B * d->np(), 1.0f, s));
+    // exit waves (kept for the backward's seed) and their intensities
+    RowArgs re = rargs(d, zprev, keep ? d->exitw.p : nullptr, true, false);
+    re.inten = inten;
+    HC(launch_row(ROW_INV, RM_NONE, re, s));
     d->have_forward = keep;
   } catch (const DErr& e) {
     d->err = e.what();
@@ -342,7 +344,7 @@ msl_status msl_diff_backward(msl_diff* d, const float* dLdI, float* gradV, void*
       if (!kept) {
         // recompute z_{base+1} .. z_{top-1} from the checkpoint, storing w_i
         for (int j = base + 1; j < top; ++j) {
-          fwd_slice(d, j, ztop, d->W.p, wslot(d, j, base), false, s);
+          fwd_slice(d, j, ztop, d->W.p, wslot(d, j, base), s);
           ztop = d->W.p;
         }
       }
