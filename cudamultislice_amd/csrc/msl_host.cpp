@@ -240,7 +240,7 @@ void propagate(msl_sim* s, float2* src, float2* dst, float dz) {
 }
 
 void ensure_vtab(msl_sim* s) {
-  if (s->vtab.p) return;
+  if (s->vtab_ext || s->vtab.p) return;
   DBuf<float> fp;
   fp.ensure(s->fparams.size());
   DBuf<float4> tab;
@@ -300,22 +300,28 @@ void bin_atoms(msl_sim* s, const float* dx, const float* dy, const float* dz) {
   int nslab = (int)std::ceil((s->MaxZ - s->MinZ) / 1.0f);
   nslab += (nslab == 0);
   const int nb = nslab * 2500;
-  s->in.ensure(up.size());
-  s->bx.ensure(n); s->by.ensure(n); s->bz.ensure(n); s->bZ.ensure(n);
-  s->key.ensure(n); s->perm.ensure(n);
-  s->zeroed.ensure(2 * (size_t)nb + 2); s->start.ensure(nb + 1);
-  s->scan_tmp.ensure((nb + 1 + 1023) / 1024 + 1);
+  BinScratch& w = *s->bin;
+  w.in.ensure(up.size());
+  w.key.ensure(n); w.perm.ensure(n);
+  w.zeroed.ensure(2 * (size_t)nb + 2);
+  w.scan_tmp.ensure((nb + 1 + 1023) / 1024 + 1);
+  s->binmem.ensure(4 * (size_t)n + nb + 1);
+  s->bx.p = s->binmem.p;
+  s->by.p = s->bx.p + n;
+  s->bz.p = s->by.p + n;
+  s->bZ.p = reinterpret_cast<int*>(s->bz.p + n);
+  s->start.p = s->bZ.p + n;
   hipStream_t st = s->stream;
-  HIPC(hipMemcpyAsync(s->in.p, up.data(), up.size() * sizeof(float), hipMemcpyHostToDevice, st));
-  HIPC(hipMemsetAsync(s->zeroed.p, 0, (2 * (size_t)nb + 2) * sizeof(int), st));
-  int* flag = s->zeroed.p + 2 * (size_t)nb + 1;
+  HIPC(hipMemcpyAsync(w.in.p, up.data(), up.size() * sizeof(float), hipMemcpyHostToDevice, st));
+  HIPC(hipMemsetAsync(w.zeroed.p, 0, (2 * (size_t)nb + 2) * sizeof(int), st));
+  int* flag = w.zeroed.p + 2 * (size_t)nb + 1;
   BinArgs a{};
-  a.x = s->in.p; a.y = s->in.p + n; a.z = s->in.p + 2 * (size_t)n;
-  a.Z = reinterpret_cast<const int*>(s->in.p + 3 * (size_t)n); a.n = n;
+  a.x = w.in.p; a.y = w.in.p + n; a.z = w.in.p + 2 * (size_t)n;
+  a.Z = reinterpret_cast<const int*>(w.in.p + 3 * (size_t)n); a.n = n;
   a.MaxX = s->MaxX; a.MinX = s->MinX; a.MaxY = s->MaxY; a.MinY = s->MinY; a.MaxZ = s->MaxZ; a.MinZ = s->MinZ;
   a.nslab = nslab;
-  a.key = s->key.p; a.count = s->zeroed.p; a.fill = s->zeroed.p + nb + 1; a.start = s->start.p; a.perm = s->perm.p;
-  a.bx = s->bx.p; a.by = s->by.p; a.bz = s->bz.p; a.bZ = s->bZ.p; a.bad = flag; a.scan_tmp = s->scan_tmp.p;
+  a.key = w.key.p; a.count = w.zeroed.p; a.fill = w.zeroed.p + nb + 1; a.start = s->start.p; a.perm = w.perm.p;
+  a.bx = s->bx.p; a.by = s->by.p; a.bz = s->bz.p; a.bZ = s->bZ.p; a.bad = flag; a.scan_tmp = w.scan_tmp.p;
   HIPC(launch_bin(a, st));
   int bad = 0;
   HIPC(hipMemcpyAsync(&bad, flag, sizeof(int), hipMemcpyDeviceToHost, st));
@@ -456,7 +462,7 @@ PotArgs pot_args(msl_sim* s, int mode, int first, int nslices, float dz, float z
   ensure_vtab(s);
   PotArgs p{};
   p.bx = s->bx.p; p.by = s->by.p; p.bz = s->bz.p; p.bZ = s->bZ.p; p.start = s->start.p; p.nslab = s->nslab;
-  p.vtab = s->vtab.p;
+  p.vtab = s->vtab_ext ? s->vtab_ext : s->vtab.p;
   p.nspec = s->nspec;
   std::copy(s->spec, s->spec + 4, p.spec);
   p.MaxX = s->MaxX; p.MinX = s->MinX; p.MaxY = s->MaxY; p.MinY = s->MinY; p.MaxZ = s->MaxZ; p.MinZ = s->MinZ;
@@ -1243,7 +1249,7 @@ msl_status msl_get_bins(const msl_sim* cs, int* keys) {
   msl_sim* s = const_cast<msl_sim*>(cs);
   API_BEGIN(s)
   require(s->binned && keys, MSL_ERR_STATE, "not binned");
-  d2h(s, keys, s->key.p, s->nbinned * sizeof(int));
+  d2h(s, keys, s->bin->key.p, s->nbinned * sizeof(int));
   API_END(s)
 }
 
@@ -1473,21 +1479,35 @@ extern "C" msl_status msl_stem_batched(msl_sim* s, const msl_stem_batch_desc* d)
   const int nslices = d->nslices > 0 ? d->nslices : (int)std::ceil((s->MaxZ - s->MinZ) / d->dz);
   const int nconf = std::max(1, d->nconfig);
   const bool displace = d->sigma > 0.f;
-  // probes per launch: the tuned width for this grid (msl_autotune_batch), else
-  // all of them when they fit in ~16 GiB of waves
-  const int auto_b = (s->tuned_batch > 0 && s->tuned_batch_n == nx)
-                         ? s->tuned_batch
-                         : (int)std::min<long long>(d->nprobe, (16LL << 30) / (np * 8));
+  // Probes per launch: the tuned width for this grid (msl_autotune_batch), else
+  // as many as keep what a slice's two passes hand over (the columns in the
+  // band) within the 256 MB Infinity Cache, in launches of equal size.  Us per
+  // probe-slice at 512^2: 128 1.79, 256 1.68, 288 1.77, 512 1.86, 1024 1.89; at
+  // 1024^2 32 7.10, 64 6.95, 96 7.42, 256 7.37; at 256^2 512 0.41, 1024 0.39,
+  // 2048 0.43; at 128^2 1024 0.107, 2048 0.098, 4096 0.112.
+  int auto_b = s->tuned_batch;
+  if (!(s->tuned_batch > 0 && s->tuned_batch_n == nx)) {
+    const long long wave_b = s->prune_tiles > 0 ? np * 4 : np * 8;
+    const long long most = std::max<long long>(1, std::min<long long>(2048, (256LL << 20) / wave_b));
+    const long long launches = (d->nprobe + most - 1) / most;
+    auto_b = (int)((d->nprobe + launches - 1) / launches);
+  }
   int B = d->batch > 0 ? d->batch : auto_b;
   B = std::max(1, std::min(std::min(B, d->nprobe), 65535));  // grid.y limit of the column pass
   const int C = col_tile(ny), ntiles = nx / C;
   alloc_waves(s);
   ensure_vtab(s);
   ensure_prop(s, d->dz);
-  DBuf<float2> tall, W;
-  DBuf<float> partial, adf;
-  DBuf<int> pos;
-  DBuf<float> inten, pacbed;
+  StemBuffers& ws = s->stem;
+  struct Trim {
+    StemBuffers& b;
+    ~Trim() { b.trim(); }
+  } trim{ws};
+  auto &tall = ws.tall, &W = ws.W;
+  auto &partial = ws.partial, &adf = ws.adf, &inten = ws.inten, &pacbed = ws.pacbed;
+  auto& pos = ws.pos;
+  for (auto& e : s->tev)
+    if (!e) HIPC(hipEventCreate(&e));
   tall.ensure((size_t)nslices * np);
   W.ensure((size_t)B * np);
   partial.ensure((size_t)B * ntiles);
@@ -1595,7 +1615,7 @@ extern "C" msl_status msl_stem_batched(msl_sim* s, const msl_stem_batch_desc* d)
       nb = -1;
     }
     ~Graph() { reset(); }
-  } graph;
+  } graphs[2];  // one for the chunk size of all but the last chunk, one for the last's
   double tb = 0, tp = 0, tprop = 0;
   // displacements of the configuration being binned, and the next
   // configuration's, drawn on the host while this one propagates (the GPU
@@ -1604,7 +1624,7 @@ extern "C" msl_status msl_stem_batched(msl_sim* s, const msl_stem_batch_desc* d)
   bool have_next = false;
   for (int cfg = 0; cfg < nconf; ++cfg) {
     require(s->cancel == 0, MSL_ERR_CANCELLED, "cancelled");
-    double a0 = now_ms();
+    HIPC(hipEventRecord(s->tev[0], s->stream));
     if (displace) {
       const int n = (int)s->x.size();
       if (have_next) {
@@ -1618,23 +1638,20 @@ extern "C" msl_status msl_stem_batched(msl_sim* s, const msl_stem_batch_desc* d)
     } else if (cfg == 0 || !s->binned) {
       bin_atoms(s, nullptr, nullptr, nullptr);
     }
-    HIPC(hipStreamSynchronize(s->stream));
-    double a1 = now_ms();
+    HIPC(hipEventRecord(s->tev[1], s->stream));
     KTimer kt(s);
     kt.begin(3);
     potential(s, s->potmode, 1, nslices, d->dz, 0.f, 0, tall.p, np);
     kt.end();
     kt.flush();
-    HIPC(hipStreamSynchronize(s->stream));
-    double a2 = now_ms();
-    tb += a1 - a0;
-    tp += a2 - a1;
+    HIPC(hipEventRecord(s->tev[2], s->stream));
     for (int p0 = 0; p0 < d->nprobe; p0 += B) {
       require(s->cancel == 0, MSL_ERR_CANCELLED, "cancelled");
       const int nb = std::min(B, d->nprobe - p0);
       HIPC(hipMemcpyAsync(pos.p, d->posx + p0, nb * sizeof(int), hipMemcpyHostToDevice, s->stream));
       HIPC(hipMemcpyAsync(pos.p + B, d->posy + p0, nb * sizeof(int), hipMemcpyHostToDevice, s->stream));
       if (graph_mode) {
+        Graph& graph = graphs[nb == B ? 0 : 1];
         if (graph.nb != nb) {
           graph.reset();
           HIPC(hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal));
@@ -1680,17 +1697,21 @@ extern "C" msl_status msl_stem_batched(msl_sim* s, const msl_stem_batch_desc* d)
         if (d->pacbed_out) HIPC(launch_sum_maps(inten.p, nb, np, pacbed.p, 1, s->stream));
       }
     }
+    HIPC(hipEventRecord(s->tev[3], s->stream));
     HIPC(hipStreamSynchronize(s->stream));
-    tprop += now_ms() - a2;
+    float ms[3] = {0, 0, 0};
+    for (int k = 0; k < 3; ++k) HIPC(hipEventElapsedTime(&ms[k], s->tev[k], s->tev[k + 1]));
+    tb += ms[0];
+    tp += ms[1];
+    tprop += ms[2];
   }
   std::vector<float> h(d->nprobe);
   d2h(s, h.data(), adf.p, d->nprobe * sizeof(float));
   for (int i = 0; i < d->nprobe; ++i) d->adf_out[i] = h[i] / (float)nconf;
   if (d->pacbed_out) {
-    std::vector<float> pc(np);
-    d2h(s, pc.data(), pacbed.p, np * sizeof(float));
+    d2h(s, d->pacbed_out, pacbed.p, np * sizeof(float));
     const float sc = 1.0f / ((float)nconf * (float)d->nprobe);
-    for (long long i = 0; i < np; ++i) d->pacbed_out[i] = pc[i] * sc;
+    for (long long i = 0; i < np; ++i) d->pacbed_out[i] *= sc;
   }
   s->timings[0] = (float)tb;
   s->timings[1] = (float)tp;

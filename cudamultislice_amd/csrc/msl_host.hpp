@@ -58,6 +58,27 @@ template <class T> struct Ptr {
   T* p = nullptr;
 };
 
+// what binning needs only while it runs: the uploaded x, y, z and Z, bin
+// keys, counts, fills and the range flag (zeroed), the permutation
+struct BinScratch {
+  DBuf<float> in;
+  DBuf<int> key, zeroed, perm, scan_tmp;
+};
+
+// device buffers of a batched STEM run, kept by the handle between runs up to
+// kKeep (allocating and freeing them cost 0.1 ms of a 0.55 ms line scan, more
+// for larger waves) and given back with it
+struct StemBuffers {
+  static constexpr size_t kKeep = (size_t)1 << 30;
+  DBuf<float2> tall, W;
+  DBuf<float> partial, adf, inten, pacbed;
+  DBuf<int> pos;
+  void trim() {
+    if ((tall.n + W.n) * sizeof(float2) + (partial.n + adf.n + inten.n + pacbed.n + pos.n) * 4 <= kKeep) return;
+    tall.release(); W.release(); partial.release(); adf.release(); inten.release(); pacbed.release(); pos.release();
+  }
+};
+
 }  // namespace mslh
 
 // ------------------------------------------------------------------ handle
@@ -85,10 +106,14 @@ struct msl_sim {
   std::vector<float> fparams = std::vector<float>(kFparams, kFparams + 103 * 12);
   bool have_params = false;
   mslh::DBuf<float4> vtab;  // radial potential tables of the parameters
+  const float4* vtab_ext = nullptr;  // another handle's of the same parameters (serving)
 
   // binned atoms on the device
-  mslh::DBuf<float> in, bx, by, bz;   // in: x, y, z and Z as uploaded
-  mslh::DBuf<int> bZ, key, zeroed, start, perm, scan_tmp;  // zeroed: counts, fills and the range flag
+  mslh::DBuf<float> binmem;  // bx, by, bz, bZ and start point into it
+  mslh::Ptr<float> bx, by, bz;
+  mslh::Ptr<int> bZ, start;
+  mslh::BinScratch bin_own;
+  mslh::BinScratch* bin = &bin_own;  // or one that several handles share (serving)
   int nslab = 0, nbinned = 0;
   bool binned = false;
   uint64_t tds_seed = 0x4D534CULL;
@@ -150,6 +175,8 @@ struct msl_sim {
   bool have_tds = false, have_image = false;
   float maxposIm = 0, maxposEW = 0, minposEW = 0, minposIm = 0, imagecontrast = 0;
   float timings[4] = {0, 0, 0, 0};
+  mslh::StemBuffers stem;
+  hipEvent_t tev[4] = {nullptr, nullptr, nullptr, nullptr};  // stage times of batched runs
   int tuned_batch = 0;  // probes per launch chosen by msl_autotune_batch (0: not tuned)
   int tuned_batch_n = 0;  // grid size it was tuned for
   // per-kernel HIP-event timing of batched runs: [row ms, row n, col ms,
@@ -161,6 +188,8 @@ struct msl_sim {
   size_t npix() const { return (size_t)resX * resY; }
   ~msl_sim() {
     for (auto e : events) (void)hipEventDestroy(e);
+    for (auto e : tev)
+      if (e) (void)hipEventDestroy(e);
   }
 };
 
