@@ -3,6 +3,7 @@
 // "GUI Simulation/UnmanagedGUISimulation.cu" (U.cu).
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 #include "msl_fft.hpp"
 #include "msl_internal.hpp"
@@ -237,12 +238,15 @@ hipError_t launch_vatom_table(const float* fparams, float4* tab, hipStream_t s) 
   return hipGetLastError();
 }
 
-// the table's value at r2; base: the species' first entry less VT_FIRST
+// the table's value at r2; base: byte offset of the species' first entry, less
+// that of the interval of 0
+constexpr int VT_ZERO = VT_FIRST * (int)sizeof(float4);
 template <class T> __device__ __forceinline__ float vt_at(T tab, int base, float r2) {
   const float x = __builtin_amdgcn_fmed3f(r2, VT_LO, VT_HI);
-  const unsigned b = __float_as_uint(x);
-  const float4 c = tab[base + (int)(b >> VT_SHIFT)];
-  const float t = x - __uint_as_float(b & ~((1u << VT_SHIFT) - 1u));
+  // the interval's lower end; its number times 16 are the same bits further down
+  const unsigned k = __float_as_uint(x) & ~((1u << VT_SHIFT) - 1u);
+  const float4 c = *(T)((const char*)tab + (int)((k >> (VT_SHIFT - 4)) + (unsigned)base));
+  const float t = x - __uint_as_float(k);
   return fmaf(t, fmaf(t, fmaf(t, c.w, c.z), c.y), c.x);
 }
 
@@ -319,12 +323,12 @@ __device__ __forceinline__ float readlane_f(float v, int l) {
 // the patch and find the samples each can reach, and only those atoms and
 // samples are summed, with the atom in scalar registers.  Lanes out of an
 // atom's reach read the table's zero interval, so there is no divergence.
-// Bound by VALU issue at large grids (13 instructions and a 16-byte LDS read
+// Bound by VALU issue at large grids (11 instructions and a 16-byte LDS read
 // per sample), by those three loads and the launch at small ones.  Per slice,
 // before (slab after slab, transcendentals, a divergent loop per pixel) and
-// now: Si 1024^2 of 0.074 A 114.6 -> 39.9 us, SrTiO3 512^2 of 0.078 A 51.0 ->
-// 19.2, Si 256^2 of 0.085 A 27.9 -> 9.1, 64^2 of 0.2 A 27.2 -> 6.8; one plane
-// of Si at 256^2 16.0 -> 5.6.
+// now: Si 1024^2 of 0.074 A 114.6 -> 34.5 us, SrTiO3 512^2 of 0.078 A 51.0 ->
+// 17.2, Si 256^2 of 0.085 A 27.9 -> 8.5, 64^2 of 0.2 A 27.2 -> 6.7; one plane
+// of Si at 256^2 16.0 -> 5.5.
 template <int TX, int TY, int SPLIT, int KIND, class A>
 __device__ __forceinline__ void potential_tile(const A& a, int tx, int ty, int slice, float4* tabs) {
   static_assert(TX * TY * SPLIT == 256, "256-thread workgroups");
@@ -426,7 +430,7 @@ __device__ __forceinline__ void potential_tile(const A& a, int tx, int ty, int s
           base = 0;
           for (int sp = 1; sp < a.nspec; ++sp) base = Z == a.spec[sp] ? sp * VT_N : base;
         }
-        sa[q] = make_float4(a.bx[src], a.by[src], a.bz[src], __int_as_float(base - VT_FIRST));
+        sa[q] = make_float4(a.bx[src], a.by[src], a.bz[src], __int_as_float(base * (int)sizeof(float4) - VT_ZERO));
       }
       __syncthreads();
       auto atoms = [&](auto tab) {
@@ -441,11 +445,11 @@ __device__ __forceinline__ void potential_tile(const A& a, int tx, int ty, int s
             float room = kReach2 - (ex * ex + ey * ey);
             hit = room > 0.f;
             if constexpr (KIND == POT_SAMPLES) {
-              // samples with |zf - m hs - z| within the patch's reach, one
-              // more on each side
+              // samples with |zf - m hs - z| within the patch's reach (0.011 A
+              // more than any pixel's, which covers the rounding of positions)
               const float hz = __builtin_amdgcn_sqrtf(fmaxf(room, 0.f)), zc = zf - at.z;
-              mlo = max(1, (int)fmaxf(floorf((zc - hz) * us), -1.f) - 1);
-              mhi = min(nsamp, (int)fminf(ceilf((zc + hz) * us), 64.f) + 1);
+              mlo = max(1, (int)fmaxf(ceilf((zc - hz) * us), 0.f));
+              mhi = min(nsamp, (int)fminf(floorf((zc + hz) * us), 64.f));
               hit = hit && mlo <= mhi;
             } else if constexpr (KIND == POT_PLANE) {
               room -= (zf - at.z) * (zf - at.z);
@@ -468,18 +472,25 @@ __device__ __forceinline__ void potential_tile(const A& a, int tx, int ty, int s
               const int m0 = __builtin_amdgcn_readlane(mlo, l), m1 = __builtin_amdgcn_readlane(mhi, l);
               const float dl = zl - az;
               float s = 0.f;
-              // four samples at a time (their table reads in flight
-              // together); a sample past m1 adds an exact zero
-              for (int m = m0; m <= m1; m += 4) {
-                float v[4];
+              // four samples at a time, their table reads in flight together
+              auto samples = [&](int m, auto count) {
+                constexpr int C = decltype(count)::value;
+                float v[C];
 #pragma unroll
-                for (int u = 0; u < 4; ++u) {
+                for (int u = 0; u < C; ++u) {
                   const float dd = readlane_f(dl, m + u);
                   v[u] = vt_at(tab, base, fmaf(dd, dd, rxy));
                 }
 #pragma unroll
-                for (int u = 0; u < 4; ++u) s += v[u];
+                for (int u = 0; u < C; ++u) s += v[u];
+              };
+              int m = m0;
+              for (; m + 3 <= m1; m += 4) samples(m, std::integral_constant<int, 4>{});
+              if (m + 1 <= m1) {
+                samples(m, std::integral_constant<int, 2>{});
+                m += 2;
               }
+              if (m <= m1) samples(m, std::integral_constant<int, 1>{});
               sum = fmaf(hs, s, sum);
             }
           }
