@@ -658,6 +658,46 @@ hipError_t launch_probe_kspace(const ProbeArgs& a, hipStream_t s) {
   return hipSuccess;
 }
 
+// ============================================================== tables
+// k-grids (PreCalculateFrequencies, U.cu:1877-1964; the FP32 division the host
+// takes too) and twiddles exp(-2 pi i k / n) of both axes, and the separable
+// Fresnel factors exp(-i pi dz lambda k^2) of CreatePropsKernel
+// (U.cu:399-428), evaluated in FP64.  Made where they are used: uploads from
+// host memory cost a run of 64^2 five waits and 70 us of 440.
+__global__ void k_ktables(float* kx, float* ky, float2* twx, float2* twy, int nx, int ny, float ksx, float ksy) {
+  const int g = blockIdx.x * blockDim.x + threadIdx.x;
+  if (g >= nx + ny) return;
+  const bool isx = g < nx;
+  const int i = isx ? g : g - nx, n = isx ? nx : ny;
+  const float ks = isx ? ksx : ksy;
+  (isx ? kx : ky)[i] = i > n / 2 ? (float)(i - n) / ks : (float)i / ks;
+  float2* tw = isx ? twx : twy;
+  if (tw) {
+    double sn, cs;
+    sincospi(-2.0 * (double)i / (double)n, &sn, &cs);
+    tw[i] = make_float2((float)cs, (float)sn);
+  }
+}
+hipError_t launch_ktables(float* kx, float* ky, float2* twx, float2* twy, int nx, int ny, float ksx, float ksy,
+                          hipStream_t s) {
+  hipLaunchKernelGGL(k_ktables, dim3(nblk(nx + ny, 64)), dim3(64), 0, s, kx, ky, twx, twy, nx, ny, ksx, ksy);
+  return hipGetLastError();
+}
+__global__ void k_prop_factors(const float* kx, const float* ky, float2* px, float2* py, int nx, int ny, float dz,
+                               float wavel) {
+#pragma clang fp contract(off)
+  const int g = blockIdx.x * blockDim.x + threadIdx.x;
+  if (g >= nx + ny) return;
+  const double k = g < nx ? kx[g] : ky[g - nx];
+  const double a = 3.14159265 * (double)dz * (double)wavel * k * k;
+  (g < nx ? px : py)[g < nx ? g : g - nx] = make_float2((float)cos(a), (float)-sin(a));
+}
+hipError_t launch_prop_factors(const float* kx, const float* ky, float2* px, float2* py, int nx, int ny, float dz,
+                               float wavel, hipStream_t s) {
+  hipLaunchKernelGGL(k_prop_factors, dim3(nblk(nx + ny, 64)), dim3(64), 0, s, kx, ky, px, py, nx, ny, dz, wavel);
+  return hipGetLastError();
+}
+
 // ============================================================== reductions
 constexpr int RB = 256;
 

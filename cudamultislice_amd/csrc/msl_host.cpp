@@ -163,20 +163,9 @@ void col(msl_sim* s, int mode, int mul, const ColArgs& a) { HIPC(launch_col(mode
 // U.cu:399-428: cos / -sin of pi dz lambda (kx^2 + ky^2))
 void ensure_prop(msl_sim* s, float dz) {
   if (s->prop_dz == dz && s->px.p) return;
-  auto tab = [&](const std::vector<float>& k) {
-    std::vector<float2> t(k.size());
-    for (size_t i = 0; i < k.size(); ++i) {
-      const double a = 3.14159265 * (double)dz * (double)s->wavel * (double)k[i] * (double)k[i];
-      t[i] = make_float2((float)std::cos(a), (float)-std::sin(a));
-    }
-    return t;
-  };
-  auto tx = tab(s->hkx), ty = tab(s->hky);
-  s->px.ensure(tx.size());
-  s->py.ensure(ty.size());
-  HIPC(hipMemcpyAsync(s->px.p, tx.data(), tx.size() * sizeof(float2), hipMemcpyHostToDevice, s->stream));
-  HIPC(hipMemcpyAsync(s->py.p, ty.data(), ty.size() * sizeof(float2), hipMemcpyHostToDevice, s->stream));
-  HIPC(hipStreamSynchronize(s->stream));
+  s->px.ensure(s->hkx.size());
+  s->py.ensure(s->hky.size());
+  HIPC(launch_prop_factors(s->kx.p, s->ky.p, s->px.p, s->py.p, s->resX, s->resY, dz, s->wavel, s->stream));
   s->prop_dz = dz;
 }
 
@@ -290,11 +279,17 @@ void bin_atoms(msl_sim* s, const float* dx, const float* dy, const float* dz) {
   require(s->have_atoms, MSL_ERR_STATE, "no atoms loaded");
   const int n = (int)s->x.size();
   // x, y, z and Z in one upload
-  std::vector<float> up(4 * (size_t)n);
+  if (s->up_busy) HIPC(hipStreamSynchronize(s->stream));
+  s->up_busy = false;
+  std::vector<float>& up = s->up;
+  up.resize(4 * (size_t)n);
+  bool far = false;
   for (int i = 0; i < n; ++i) {
-    up[i] = s->x[i] + (dx ? dx[i] : 0.0f);
-    up[n + i] = s->y[i] + (dy ? dy[i] : 0.0f);
-    up[2 * (size_t)n + i] = s->z[i] + (dz ? dz[i] : 0.0f);
+    const float x = s->x[i] + (dx ? dx[i] : 0.0f), y = s->y[i] + (dy ? dy[i] : 0.0f), z = s->z[i] + (dz ? dz[i] : 0.0f);
+    up[i] = x;
+    up[n + i] = y;
+    up[2 * (size_t)n + i] = z;
+    far |= !(std::fabs(x) < 1e5f && std::fabs(y) < 1e5f && std::fabs(z) < 1e5f);
   }
   std::memcpy(up.data() + 3 * (size_t)n, s->Z.data(), n * sizeof(int));
   int nslab = (int)std::ceil((s->MaxZ - s->MinZ) / 1.0f);
@@ -322,11 +317,18 @@ void bin_atoms(msl_sim* s, const float* dx, const float* dy, const float* dz) {
   a.nslab = nslab;
   a.key = w.key.p; a.count = w.zeroed.p; a.fill = w.zeroed.p + nb + 1; a.start = s->start.p; a.perm = w.perm.p;
   a.bx = s->bx.p; a.by = s->by.p; a.bz = s->bz.p; a.bZ = s->bZ.p; a.bad = flag; a.scan_tmp = w.scan_tmp.p;
+  s->up_busy = true;
   HIPC(launch_bin(a, st));
-  int bad = 0;
-  HIPC(hipMemcpyAsync(&bad, flag, sizeof(int), hipMemcpyDeviceToHost, st));
-  HIPC(hipStreamSynchronize(st));
-  require(!bad, MSL_ERR_RANGE, "an atom lies outside the 50x50 bin grid (displacement larger than the 2 A margin?)");
+  // Undisplaced atoms lie 2 A inside their extents (LoadAtomFile's margins),
+  // so at positions that FP32 resolves they are inside the bin grid: nothing
+  // to wait for
+  if (dx || dy || dz || far) {
+    int bad = 0;
+    HIPC(hipMemcpyAsync(&bad, flag, sizeof(int), hipMemcpyDeviceToHost, st));
+    HIPC(hipStreamSynchronize(st));
+    s->up_busy = false;
+    require(!bad, MSL_ERR_RANGE, "an atom lies outside the 50x50 bin grid (displacement larger than the 2 A margin?)");
+  }
   s->nslab = nslab;
   s->nbinned = n;
   s->binned = true;
@@ -419,24 +421,16 @@ void precalc(msl_sim* s) {
     s->gly = GenLen{ry, (int)wy.size(), s->gtwy.p, cy.empty() ? nullptr : s->gchy.p, cy.empty() ? nullptr : s->gfiy.p};
   }
   // k-grids, and the twiddles of the power-of-two passes
-  std::vector<float> kt(s->hkx);
-  kt.insert(kt.end(), s->hky.begin(), s->hky.end());
-  kt.resize(kt.size() + kt.size() % 2);
-  const size_t o = kt.size();
-  if (!s->generic) {
-    const auto tx = twiddles(rx), ty = twiddles(ry);
-    kt.resize(o + 2 * (size_t)(rx + ry));
-    std::memcpy(kt.data() + o, tx.data(), rx * sizeof(float2));
-    std::memcpy(kt.data() + o + 2 * (size_t)rx, ty.data(), ry * sizeof(float2));
-  }
-  upload(s->ktab, kt);
+  const size_t o = (size_t)(rx + ry) + (rx + ry) % 2;
+  s->ktab.ensure(o + (s->generic ? 0 : 2 * (size_t)(rx + ry)));
   s->kx.p = s->ktab.p;
   s->ky.p = s->ktab.p + rx;
   s->twx.p = s->generic ? nullptr : reinterpret_cast<float2*>(s->ktab.p + o);
   s->twy.p = s->generic ? nullptr : reinterpret_cast<float2*>(s->ktab.p + o) + rx;
+  HIPC(launch_ktables(s->kx.p, s->ky.p, s->twx.p, s->twy.p, rx, ry, s->ksizex, s->ksizey, s->stream));
   s->prow.ensure(rx);
   HIPC(launch_prop_rows(s->kx.p, s->ky.p, rx, ry, s->kmax, s->prow.p, s->stream));
-  HIPC(hipStreamSynchronize(s->stream));
+  if (!wx.empty()) HIPC(hipStreamSynchronize(s->stream));  // the generic tables come from host memory
   s->prop_dz = std::nanf("");
   s->fd_lap = false;
   s->have_freqs = true;

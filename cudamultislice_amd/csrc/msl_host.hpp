@@ -114,6 +114,8 @@ struct msl_sim {
   mslh::Ptr<int> bZ, start;
   mslh::BinScratch bin_own;
   mslh::BinScratch* bin = &bin_own;  // or one that several handles share (serving)
+  std::vector<float> up;  // the positions being uploaded (alive until the stream has read them)
+  bool up_busy = false;
   int nslab = 0, nbinned = 0;
   bool binned = false;
   uint64_t tds_seed = 0x4D534CULL;
@@ -144,8 +146,7 @@ struct msl_sim {
   // uses G, clears it)
   bool fd_lap = false;
   std::vector<float> hkx, hky;
-  // the k-grids and twiddles of both axes, one upload; kx, ky, twx, twy point
-  // into it
+  // the k-grids and twiddles of both axes; kx, ky, twx, twy point into it
   mslh::DBuf<float> ktab;
   mslh::Ptr<float> kx, ky;
   mslh::Ptr<float2> twx, twy;

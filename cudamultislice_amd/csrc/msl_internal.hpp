@@ -269,6 +269,13 @@ struct ProbeArgs {
 };
 hipError_t launch_probe_kspace(const ProbeArgs& a, hipStream_t s);
 
+// k-grids of both axes (kx, ky; ks the side in A) and their twiddles (twx, twy;
+// may be null), and the Fresnel factors of slice thickness dz
+hipError_t launch_ktables(float* kx, float* ky, float2* twx, float2* twy, int nx, int ny, float ksx, float ksy,
+                          hipStream_t s);
+hipError_t launch_prop_factors(const float* kx, const float* ky, float2* px, float2* py, int nx, int ny, float dz,
+                               float wavel, hipStream_t s);
+
 // sum |w| over n elements per wave (deterministic), then w /= sum.
 hipError_t launch_l1_normalise(float2* w, long long n, int nbatch, long long bstride, float* scratch, hipStream_t s);
 // as launch_l1_normalise, dividing by sqrt(sum |w|^2) when l2 != 0; the
