@@ -281,7 +281,8 @@ template <int M, bool BLUE> __global__ void __launch_bounds__(GenRow<M>::THREADS
     const int i = t + c * T;
     if (i >= n) continue;
     const float2 r = make_float2((float)v[c].x, (float)v[c].y);
-    a.dst[o + i] = r;
+    if (a.inten) a.inten[o + i] = r.x * r.x + r.y * r.y;
+    if (a.dst) a.dst[o + i] = r;
     if (a.dst2) a.dst2[o + i] = r;
   }
 }
@@ -440,7 +441,7 @@ void gen_tables(int n, std::vector<double2>& tw, std::vector<double2>& chirp, st
   return hipErrorInvalidValue
 
 hipError_t launch_gen_row(const GenRowArgs& a, hipStream_t s) {
-  if (!a.src || !a.dst || a.ny < 1 || a.nbatch < 0 || !len_ok(a.len, a.nx)) return hipErrorInvalidValue;
+  if (!a.src || !(a.dst || a.inten) || a.ny < 1 || a.nbatch < 0 || !len_ok(a.len, a.nx)) return hipErrorInvalidValue;
   if (a.nbatch == 0) return hipSuccess;
   MSL_GEN_LEN(gen_row_m, a, s);
 }

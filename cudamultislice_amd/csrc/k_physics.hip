@@ -845,15 +845,6 @@ hipError_t launch_abs(const float2* w, float* o, long long n, hipStream_t s) {
   return hipGetLastError();
 }
 
-__global__ void k_intensity(const float2* w, float* o, long long n, float f) {
-  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) o[i] = (w[i].x * w[i].x + w[i].y * w[i].y) * f;
-}
-hipError_t launch_intensity(const float2* w, float* o, long long n, float f, hipStream_t s) {
-  hipLaunchKernelGGL(k_intensity, dim3(nblk(n, 256)), dim3(256), 0, s, w, o, n, f);
-  return hipGetLastError();
-}
-
 // ============================================================== real-space multislice
 // One term of MultisliceStepRS's series (RSMS with DifferentialXKernel /
 // DifferentialYKernel, U.cu:798-877): out = w + i pre (Lx w + Ly w + V w)

@@ -170,11 +170,11 @@ void ensure_prop(msl_sim* s, float dz) {
 }
 
 // generic rows: dst = (src t) transformed along x (t optional; dst2 an
-// optional second copy)
+// optional second copy; inten |dst|^2, dst may then be null)
 void gen_row(msl_sim* s, const float2* src, float2* dst, int nbatch, bool inverse, const float2* t = nullptr,
-             float2* dst2 = nullptr) {
+             float2* dst2 = nullptr, float* inten = nullptr) {
   GenRowArgs a{};
-  a.src = src; a.dst = dst; a.dst2 = dst2; a.t = t;
+  a.src = src; a.dst = dst; a.dst2 = dst2; a.t = t; a.inten = inten;
   a.nx = s->resX; a.ny = s->resY; a.nbatch = nbatch; a.inverse = inverse ? 1 : 0;
   a.len = s->glx;
   HIPC(launch_gen_row(a, s->stream));
@@ -1050,13 +1050,26 @@ msl_status msl_get_tds(msl_sim* s, float* out) {
 }
 
 namespace {
+// gives the image buffers back where they are too large to keep
+struct ImageTrim {
+  ImageBuffers& b;
+  ~ImageTrim() { b.trim(); }
+};
+
 // CTF image(s) of the current wave, U.cu:2322-2343 with imagingKernel2
 void ctf_images(msl_sim* s, int ndf, const float* dfs, float* d_out, const float* css = nullptr) {
   const long long n = (long long)s->npix();
-  HIPC(hipMemcpyAsync(s->B.p, s->Psi.p, n * sizeof(float2), hipMemcpyDeviceToDevice, s->stream));
-  fft2(s, s->B.p, 1, false, s->nfd);
-  DBuf<float2> K;
-  DBuf<float> dd, dc;
+  if (s->generic) {
+    gen_row(s, s->Psi.p, s->B.p, 1, false);
+    gen_col(s, s->B.p, 1, COL_FWD, CM_SCALE, s->nfd);
+  } else {
+    row(s, ROW_FWD, RM_NONE, row_args(s, s->Psi.p, s->B.p, 1, n));
+    ColArgs c = col_args(s, s->B.p, s->B.p, 1, n);
+    c.scale = s->nf;
+    col(s, COL_FWD, CM_SCALE, c);
+  }
+  DBuf<float2>& K = s->images.K;
+  DBuf<float>&dd = s->images.dfs, &dc = s->images.css;
   K.ensure((size_t)ndf * n);
   dd.ensure(ndf);
   HIPC(hipMemcpyAsync(dd.p, dfs, ndf * sizeof(float), hipMemcpyHostToDevice, s->stream));
@@ -1069,8 +1082,19 @@ void ctf_images(msl_sim* s, int ndf, const float* dfs, float* d_out, const float
   c.dfs = dd.p; c.css = css ? dc.p : nullptr; c.Cs = s->Cs; c.A1 = s->A1; c.A1phi = s->A1phi; c.A2 = s->A2; c.A2phi = s->A2phi; c.obj = s->obj;
   c.wavel = s->wavel; c.beta = s->beta / 1000.f; c.delta = s->delta; c.scale = 1.0f;
   HIPC(launch_ctf(c, s->stream));
-  fft2(s, K.p, ndf, true, s->nfd);
-  HIPC(launch_intensity(K.p, d_out, n * ndf, 1.0f, s->stream));
+  // the images from the last row pass (a pass of its own read the waves again)
+  if (s->generic) {
+    gen_col(s, K.p, ndf, COL_INV, CM_SCALE, s->nfd);
+    gen_row(s, K.p, nullptr, ndf, true, nullptr, nullptr, d_out);
+  } else {
+    ColArgs ci = col_args(s, K.p, K.p, ndf, n);
+    ci.scale = s->nf;
+    col(s, COL_INV, CM_SCALE, ci);
+    RowArgs ri = row_args(s, K.p, nullptr, ndf, n);
+    ri.inten = d_out;
+    row(s, ROW_INV, RM_NONE, ri);
+  }
+  // the caller's lists have to be read before it returns
   HIPC(hipStreamSynchronize(s->stream));
 }
 
@@ -1104,6 +1128,7 @@ void detector_image(msl_sim* s, float dose) {
 msl_status msl_simulate_image(msl_sim* s, float dose) {
   API_BEGIN(s)
   require(s->have_waves, MSL_ERR_STATE, "no wave");
+  ImageTrim trim{s->images};
   s->image.ensure(s->npix());
   const float df = s->df;
   ctf_images(s, 1, &df, s->image.p);
@@ -1164,7 +1189,8 @@ msl_status msl_ctf_sweep(msl_sim* s, int ndf, const float* dfs, float* out) {
   API_BEGIN(s)
   require(s->have_waves, MSL_ERR_STATE, "no wave");
   require(ndf > 0 && dfs && out, MSL_ERR_ARG, "bad defocus list");
-  DBuf<float> d;
+  ImageTrim trim{s->images};
+  DBuf<float>& d = s->images.out;
   d.ensure((size_t)ndf * s->npix());
   ctf_images(s, ndf, dfs, d.p);
   d2h(s, out, d.p, (size_t)ndf * s->npix() * sizeof(float));
@@ -1188,7 +1214,8 @@ msl_status msl_cs_df_sweep(msl_sim* s, float cs0, float cs1, int ncs, float df0,
       cs.push_back(val(cs0, cs1, ncs, i));
       df.push_back(val(df0, df1, ndf, j));
     }
-  DBuf<float> d;
+  ImageTrim trim{s->images};
+  DBuf<float>& d = s->images.out;
   d.ensure((size_t)std::min(total, chunk) * np);
   for (int k0 = 0; k0 < total; k0 += chunk) {
     const int m = std::min(chunk, total - k0);

@@ -79,6 +79,16 @@ struct StemBuffers {
   }
 };
 
+// the same for CTF images: spectra, images of a sweep, its defoci and Cs
+struct ImageBuffers {
+  DBuf<float2> K;
+  DBuf<float> out, dfs, css;
+  void trim() {
+    if (K.n * sizeof(float2) + (out.n + dfs.n + css.n) * 4 <= StemBuffers::kKeep) return;
+    K.release(); out.release(); dfs.release(); css.release();
+  }
+};
+
 }  // namespace mslh
 
 // ------------------------------------------------------------------ handle
@@ -177,6 +187,7 @@ struct msl_sim {
   float maxposIm = 0, maxposEW = 0, minposEW = 0, minposIm = 0, imagecontrast = 0;
   float timings[4] = {0, 0, 0, 0};
   mslh::StemBuffers stem;
+  mslh::ImageBuffers images;
   hipEvent_t tev[4] = {nullptr, nullptr, nullptr, nullptr};  // stage times of batched runs
   int tuned_batch = 0;  // probes per launch chosen by msl_autotune_batch (0: not tuned)
   int tuned_batch_n = 0;  // grid size it was tuned for

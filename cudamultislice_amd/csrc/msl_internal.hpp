@@ -134,6 +134,7 @@ struct GenRowArgs {
   const float2* src;
   float2* dst;
   float2* dst2;     // optional second copy of the result
+  float* inten;     // optional |result|^2 (dst may then be null)
   const float2* t;  // optional [ny][nx] factor of every wave, before the transform
   int nx, ny, nbatch, inverse;
   GenLen len;  // of nx
@@ -312,7 +313,6 @@ hipError_t launch_detector_filter(float2* F, int nx, int ny, const float* tab, i
 hipError_t launch_shot_noise(const float2* z, float2* out, long long n, float zscale, float dose,
                              unsigned long long seed, hipStream_t s);
 hipError_t launch_real_to_complex(const float* in, float2* out, long long n, hipStream_t s);
-hipError_t launch_intensity(const float2* w, float* out, long long n, float s, hipStream_t st);
 // t[i] = exp(i sigma V[i])
 hipError_t launch_transmission(const float* V, float2* t, long long n, float sigma, hipStream_t s);
 
