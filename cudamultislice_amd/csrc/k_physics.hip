@@ -398,7 +398,101 @@ __device__ __forceinline__ void potential_tile(const A& a, int tx, int ty, int s
   constexpr float kReach2 = 5.05f;
   float sum = 0.f;
   int seen = 0;  // atoms of the patch so far (SPLIT: atom n goes to wave n % SPLIT)
-  for (int rb = 0; rb < runs; rb += 256) {
+  // the atoms of a chunk, in sa[0 .. cn - 1]
+  auto stage = [&](int q, int src) {
+    const int Z = a.bZ[src];
+    int base = (Z - 1) * VT_N + kPart;
+    if (in_lds) {
+      base = 0;
+      for (int sp = 1; sp < a.nspec; ++sp) base = Z == a.spec[sp] ? sp * VT_N : base;
+    }
+    sa[q] = make_float4(a.bx[src], a.by[src], a.bz[src], __int_as_float(base * (int)sizeof(float4) - VT_ZERO));
+  };
+  auto sum_chunk = [&](int cn) {
+    auto atoms = [&](auto tab) {
+      for (int b0 = 0; b0 < cn; b0 += 64) {
+        float4 at = make_float4(0.f, 0.f, 0.f, 0.f);
+        bool hit = false;
+        int mlo = 1, mhi = 0;
+        if (b0 + lane < cn) {
+          at = sa[b0 + lane];
+          const float ex = fmaxf(fmaxf(bx0 - at.x, at.x - bx1), 0.f);
+          const float ey = fmaxf(fmaxf(by0 - at.y, at.y - by1), 0.f);
+          float room = kReach2 - (ex * ex + ey * ey);
+          hit = room > 0.f;
+          if constexpr (KIND == POT_SAMPLES) {
+            // samples with |zf - m hs - z| within the patch's reach (0.011 A
+            // more than any pixel's, which covers the rounding of positions)
+            const float hz = __builtin_amdgcn_sqrtf(fmaxf(room, 0.f)), zc = zf - at.z;
+            mlo = max(1, (int)fmaxf(ceilf((zc - hz) * us), 0.f));
+            mhi = min(nsamp, (int)fminf(floorf((zc + hz) * us), 64.f));
+            hit = hit && mlo <= mhi;
+          } else if constexpr (KIND == POT_PLANE) {
+            room -= (zf - at.z) * (zf - at.z);
+            hit = room > 0.f;
+          }
+        }
+        unsigned long long mask = __ballot(hit);
+        while (mask) {
+          const int l = __builtin_ctzll(mask);
+          mask &= mask - 1;
+          if (SPLIT > 1 && (seen++ % SPLIT) != wv) continue;
+          const float ax = readlane_f(at.x, l), ay = readlane_f(at.y, l), az = readlane_f(at.z, l);
+          const int base = __builtin_amdgcn_readlane(__float_as_int(at.w), l);
+          const float rxy = dist2_xy(px, py, ax, ay);
+          if constexpr (KIND == POT_PROJECTED) {
+            sum += vt_at(tab, base, rxy);
+          } else if constexpr (KIND == POT_PLANE) {
+            sum += vt_at(tab, base, dist2_z(rxy, zf, az));
+          } else {
+            const int m0 = __builtin_amdgcn_readlane(mlo, l), m1 = __builtin_amdgcn_readlane(mhi, l);
+            const float dl = zl - az;
+            float s = 0.f;
+            // four samples at a time, their table reads in flight together
+            auto samples = [&](int m, auto count) {
+              constexpr int C = decltype(count)::value;
+              float v[C];
+#pragma unroll
+              for (int u = 0; u < C; ++u) {
+                const float dd = readlane_f(dl, m + u);
+                v[u] = vt_at(tab, base, fmaf(dd, dd, rxy));
+              }
+#pragma unroll
+              for (int u = 0; u < C; ++u) s += v[u];
+            };
+            int m = m0;
+            for (; m + 3 <= m1; m += 4) samples(m, std::integral_constant<int, 4>{});
+            if (m + 1 <= m1) {
+              samples(m, std::integral_constant<int, 2>{});
+              m += 2;
+            }
+            if (m <= m1) samples(m, std::integral_constant<int, 1>{});
+            sum = fmaf(hs, s, sum);
+          }
+        }
+      }
+    };
+    if (in_lds) atoms((const float4*)tabs);
+    else atoms(a.vtab);
+  };
+  // Small launches: where the window's slabs hold no more than a chunk of atoms
+  // (one run of the CSR), they are taken as they come and the patch test culls
+  // them, 64 at a time, without the bin rows' scan and their expansion (256^2:
+  // 8.5 -> 7.9 us, 64^2 6.7 -> 5.8, a plane 5.5 -> 4.9).  Full launches, whose
+  // windows seldom qualify, lose 2 to 5 % to the registers it takes.
+  bool all = false;
+  if constexpr (SPLIT > 1) {
+    if (runs > 0) {
+      const int s0 = a.start[k0 * 2500], n = a.start[(k1 + 1) * 2500] - s0;
+      all = n <= ACAP;
+      if (all) {
+        for (int q = tid; q < n; q += 256) stage(q, s0 + q);
+        __syncthreads();
+        sum_chunk(n);
+      }
+    }
+  }
+  for (int rb = all ? runs : 0; rb < runs; rb += 256) {
     int len = 0, r0 = 0;
     if (rb + tid < runs) {
       const int k = (rb + tid) / nj, j = (rb + tid) - k * nj;
@@ -423,81 +517,9 @@ __device__ __forceinline__ void potential_tile(const A& a, int tx, int ty, int s
       const int cn = min(ACAP, tot - c0);
       for (int j = max(0, c0 - off); j < len && off + j < c0 + cn; ++j) si[off + j - c0] = r0 + j;
       __syncthreads();
-      for (int q = tid; q < cn; q += 256) {
-        const int src = si[q], Z = a.bZ[src];
-        int base = (Z - 1) * VT_N + kPart;
-        if (in_lds) {
-          base = 0;
-          for (int sp = 1; sp < a.nspec; ++sp) base = Z == a.spec[sp] ? sp * VT_N : base;
-        }
-        sa[q] = make_float4(a.bx[src], a.by[src], a.bz[src], __int_as_float(base * (int)sizeof(float4) - VT_ZERO));
-      }
+      for (int q = tid; q < cn; q += 256) stage(q, si[q]);
       __syncthreads();
-      auto atoms = [&](auto tab) {
-        for (int b0 = 0; b0 < cn; b0 += 64) {
-          float4 at = make_float4(0.f, 0.f, 0.f, 0.f);
-          bool hit = false;
-          int mlo = 1, mhi = 0;
-          if (b0 + lane < cn) {
-            at = sa[b0 + lane];
-            const float ex = fmaxf(fmaxf(bx0 - at.x, at.x - bx1), 0.f);
-            const float ey = fmaxf(fmaxf(by0 - at.y, at.y - by1), 0.f);
-            float room = kReach2 - (ex * ex + ey * ey);
-            hit = room > 0.f;
-            if constexpr (KIND == POT_SAMPLES) {
-              // samples with |zf - m hs - z| within the patch's reach (0.011 A
-              // more than any pixel's, which covers the rounding of positions)
-              const float hz = __builtin_amdgcn_sqrtf(fmaxf(room, 0.f)), zc = zf - at.z;
-              mlo = max(1, (int)fmaxf(ceilf((zc - hz) * us), 0.f));
-              mhi = min(nsamp, (int)fminf(floorf((zc + hz) * us), 64.f));
-              hit = hit && mlo <= mhi;
-            } else if constexpr (KIND == POT_PLANE) {
-              room -= (zf - at.z) * (zf - at.z);
-              hit = room > 0.f;
-            }
-          }
-          unsigned long long mask = __ballot(hit);
-          while (mask) {
-            const int l = __builtin_ctzll(mask);
-            mask &= mask - 1;
-            if (SPLIT > 1 && (seen++ % SPLIT) != wv) continue;
-            const float ax = readlane_f(at.x, l), ay = readlane_f(at.y, l), az = readlane_f(at.z, l);
-            const int base = __builtin_amdgcn_readlane(__float_as_int(at.w), l);
-            const float rxy = dist2_xy(px, py, ax, ay);
-            if constexpr (KIND == POT_PROJECTED) {
-              sum += vt_at(tab, base, rxy);
-            } else if constexpr (KIND == POT_PLANE) {
-              sum += vt_at(tab, base, dist2_z(rxy, zf, az));
-            } else {
-              const int m0 = __builtin_amdgcn_readlane(mlo, l), m1 = __builtin_amdgcn_readlane(mhi, l);
-              const float dl = zl - az;
-              float s = 0.f;
-              // four samples at a time, their table reads in flight together
-              auto samples = [&](int m, auto count) {
-                constexpr int C = decltype(count)::value;
-                float v[C];
-#pragma unroll
-                for (int u = 0; u < C; ++u) {
-                  const float dd = readlane_f(dl, m + u);
-                  v[u] = vt_at(tab, base, fmaf(dd, dd, rxy));
-                }
-#pragma unroll
-                for (int u = 0; u < C; ++u) s += v[u];
-              };
-              int m = m0;
-              for (; m + 3 <= m1; m += 4) samples(m, std::integral_constant<int, 4>{});
-              if (m + 1 <= m1) {
-                samples(m, std::integral_constant<int, 2>{});
-                m += 2;
-              }
-              if (m <= m1) samples(m, std::integral_constant<int, 1>{});
-              sum = fmaf(hs, s, sum);
-            }
-          }
-        }
-      };
-      if (in_lds) atoms((const float4*)tabs);
-      else atoms(a.vtab);
+      sum_chunk(cn);
       __syncthreads();  // si / sa are rewritten by the next chunk
     }
     __syncthreads();  // wsum is rewritten by the next runs
