@@ -40,6 +40,11 @@ static int lg2(int n) {
   return l;
 }
 
+// layouts of small launches, chosen by auto_row and auto_col only (not by
+// number through msl_set_pass_variant)
+constexpr int kSmallRow = 5;  // as row 1 with SmallPlan (64 to 256)
+constexpr int kSmallCol = 8;  // as column 0 with SmallPlan and tiles of four columns (64 to 512)
+
 // ------------------------------------------------------------------ variants
 // row:    0 workgroup barriers, unpadded LDS
 //         1 wave-local exchanges (lines never straddle a wave), LDS pad 1/16
@@ -101,48 +106,61 @@ void set_pass_variant(int kind, int n, int v) {
 // line, or fewer lines per workgroup); above, the layouts of the defaults.
 // Between variants of one plan (0, 1, 3; at 1024 and 2048 also 4) a line's
 // bits are the same, so the choice may follow the batch; a change of plan
-// (2; 4 at 512) is for callers whose batch never varies (RowArgs::alone), so
-// that a wave's result does not depend on how a run is cut into batches.
-// Us per launch of IFFT -> t -> FFT at 1 / 4 / 16 waves of n x n (variant:time):
-//   128  1: 4.4 / 4.5 / 4.6, 2: 3.7 / 3.8 / 3.8 (from 37 waves on 1)
-//   256  1: 4.7 / 4.8 / 5.3, 2: 3.8 / 3.9 / 5.3
+// (2, small; 4 at 512) is for callers whose batch never varies
+// (RowArgs::alone), so that a wave's result does not depend on how a run is
+// cut into batches.
+// Us per launch of IFFT -> t -> FFT (variant:time; s the small layout):
+//    64  0: 3.3 at 1 wave of n x n, 3.5 at 16; 1: 3.0, 3.2; s: 2.7, 2.9
+//   128  1: 4.4, 4.6; 2: 3.7, 3.9; s: 3.2, 3.4 (from 37 waves on 1)
+//   256  1: 4.7 at 1, 5.0 at 8, 5.1 at 12; 2: 3.8, 4.1, 5.2; s: 3.3, 4.2, 5.2
 //   512  1: 4.2 at 1 wave (2: 5.8); at 24 waves 3: 15.7, 4: 18.2; at 64 3: 40.2, 4: 38.1
 //  1024  1: 6.5 at 1 wave (3: 7.9); at 8 waves 3: 23.9, 4: 25.4; at 16 3: 44.5, 4: 42.6
 static int auto_row(int n, long long lines, bool alone) {
   switch (n) {
+    case 64:
     case 128:
-    case 256: return alone && lines <= 3072 ? 2 : 1;
+    case 256: return alone && lines <= 3072 ? kSmallRow : kRowDefault[lg2(n)];
     case 512: return !alone || lines > 20480 ? 4 : lines <= 1024 ? 1 : 3;
     case 1024: return lines <= 2048 ? 1 : lines <= 12288 ? 3 : 4;
   }
   return kRowDefault[lg2(n)];
 }
 
-// The variant of a launch of `cols` columns: half-width tiles (twice the
-// workgroups, the same bits as 0) while the full ones leave CUs idle, and at
-// 512 always.  Us per launch of the propagation pass, variants 0 and 3:
-//   64   3.3, 2.9 at 16 waves of n x n
-//  256   5.2, 4.4 at 1 wave; 5.5, 4.9 at 16; 8.1, 8.2 at 64
-//  512   8.1, 5.3 at 1; 16.3, 11.0 at 24; 128, 72.1 at 256 (variant 7: 6.2, 11.7, 73.1)
-//  1024  8.5, 7.8 at 1; 16.1, 19.1 at 8
-static int auto_col(int n, long long cols) {
+// The variant of a launch of `cols` columns: the small layout (ColArgs::alone
+// as above; at 512 its plan and so its bits are those of 0) while most CUs
+// have a tile or two, half-width tiles (twice the workgroups, the same bits
+// as 0) while the full ones leave CUs idle, and at 512 always.  Us per
+// launch of the propagation pass, variants 0, 3 and small:
+//   64   3.0, 3.0, 3.1 at 1 wave of n x n; 3.3, 2.9, 2.7 at 16
+//  128   4.0, 4.3, 3.6 at 1; 4.3, 4.0, 3.4 at 16
+//  256   5.2, 4.4, 3.7 at 1; 5.4, 4.8, 4.7 at 12; 8.1, 8.2, - at 64
+//  512   8.1, 5.3, 4.7 at 1; 8.1, 5.5, 5.0 at 2; 8.4, 5.6, 5.6 at 4; 16.3, 11.0, - at 24;
+//        128, 72.1, - at 256 (variant 7: 6.2, 6.3, 6.5, 11.7, 73.1)
+//  1024  8.5, 7.8, 7.9 at 1; 8.9, 8.8, 10.3 at 2; 16.1, 19.1, - at 8
+static int auto_col(int n, long long cols, bool alone) {
+  if (n == 512 ? cols <= 1024 : (n >= 64 && n <= 256 && alone && cols <= 3072)) return kSmallCol;
   const int half = n == 64 ? 4096 : n == 256 ? 8192 : n == 1024 ? 1024 : 0;
   return cols <= half ? 3 : kColDefault[lg2(n)];
 }
 int num_pass_variants(int kind) { return kind == 0 ? 5 : 8; }
 #endif
 
+template <int N, bool SMALL, bool ALT> struct PassPlan { using P = SmallPlan<N>; };
+template <int N> struct PassPlan<N, false, true> { using P = AltPlan<N>; };
+template <int N> struct PassPlan<N, false, false> { using P = Plan<N>; };
+
 template <int N> struct ColTile0 { static constexpr int C = (N >= 2048) ? 4 : (N >= 1024 ? 8 : 16); };
 
 template <int N, int CV> struct ColCfg {
-  using P = typename std::conditional<CV == 2 || CV == 6 || CV == 7, AltPlan<N>, Plan<N>>::type;
+  using P = typename PassPlan<N, CV == kSmallCol, CV == 2 || CV == 6 || CV == 7>::P;
   // variant 6: consecutive threads of a wave hold one column (T <= 64), so the
   // exchanges synchronise the wave only; loads take C / (64 / T) columns'
   // worth of each row per instruction instead of the whole tile row
   static constexpr bool WAVECOL = CV == 6 && P::T <= 64 && 64 % P::T == 0;
   static constexpr bool INTERLEAVED = CV != 1 && !WAVECOL;
   static constexpr int T = P::T;
-  static constexpr int C = (CV == 3 || CV == 6 || CV == 7) ? ColTile0<N>::C / 2 : ColTile0<N>::C;
+  static constexpr int C = CV == kSmallCol ? 4
+                           : (CV == 3 || CV == 6 || CV == 7) ? ColTile0<N>::C / 2 : ColTile0<N>::C;
   static constexpr int SH = INTERLEAVED ? 0 : 4;
   // [col][row] line stride in float2: span + padding so consecutive columns
   // start two banks apart (stride = 2 mod 32 float2)
@@ -197,7 +215,7 @@ __device__ __forceinline__ long long xcd_remap(long long id, long long total) {
 
 // ------------------------------------------------------------------ rows
 template <int N, int RV> struct RowCfg {
-  using P = typename std::conditional<RV == 2, AltPlan<N>, Plan<N>>::type;
+  using P = typename PassPlan<N, RV == kSmallRow, RV == 2>::P;
   static constexpr int T = P::T;
   static constexpr bool WAVE = RV >= 1 && T <= 64;
   static constexpr int SH = RV >= 1 ? 4 : 0;
@@ -1121,6 +1139,8 @@ static hipError_t row_pl(int mode, int mul, const RowArgs& a, hipStream_t s) {
 
 template <int N>
 static hipError_t row_n(int mode, int mul, const RowArgs& a, hipStream_t s, int var) {
+  if constexpr (N >= 64 && N <= 256)
+    if (var == kSmallRow) return row_nv<N, kSmallRow>(mode, mul, a, s);
   if (var == 4) return row_pl<N>(mode, mul, a, s);
   if (var == 3) return row_nv<N, 3>(mode, mul, a, s);
   if (var == 2) return row_nv<N, 2>(mode, mul, a, s);
@@ -1153,7 +1173,7 @@ static hipError_t col_nv(int mode, int mul, const ColArgs& a, hipStream_t s) {
     else if (mode == COL_FWD_MUL_INV && mul == CM_BAND) MSL_COL(COL_FWD_MUL_INV, CM_BAND);
     else if (mode == COL_FWD_MUL_INV && mul == CM_GRAD) MSL_COL(COL_FWD_MUL_INV, CM_GRAD);
     else if (mode == COL_FD) {
-      if constexpr (CV == 0 || CV == 3) {  // col_n sends it to no other
+      if constexpr (CV == 0 || CV == 3 || CV == kSmallCol) {  // col_n sends it to no other
         if (!a.dst2) return hipErrorInvalidValue;
         if (mul == CM_BAND) MSL_COL(COL_FD, CM_BAND);
         else if (mul == CM_BAND_ZB) MSL_COL(COL_FD, CM_BAND_ZB);
@@ -1208,6 +1228,8 @@ static hipError_t col_n(int mode, int mul, const ColArgs& a, hipStream_t s, int 
     return var == 2 ? col_nv<N, 2>(mode, mul, a, s) : col_nv<N, 0>(mode, mul, a, s);
   }
   // the two filters of a finite-difference step: full or half-width tiles
+  if constexpr (N >= 64 && N <= 512)
+    if (var == kSmallCol) return col_nv<N, kSmallCol>(mode, mul, a, s);
   if (mode == COL_FD) return var == 3 ? col_nv<N, 3>(mode, mul, a, s) : col_nv<N, 0>(mode, mul, a, s);
   if (var == 6) {
     if constexpr (ColCfg<N, 6>::WAVECOL) return col_nv<N, 6>(mode, mul, a, s);
@@ -1318,7 +1340,7 @@ hipError_t launch_row(int mode, int mul, const RowArgs& a, hipStream_t s) {
 }
 hipError_t launch_col(int mode, int mul, const ColArgs& a, hipStream_t s) {
   const int v = fft_size_supported(a.ny) ? g_col_var[lg2(a.ny)] : 0;
-  return launch_col_v(mode, mul, a, s, v >= 0 ? v : auto_col(a.ny, (long long)a.nbatch * a.nx));
+  return launch_col_v(mode, mul, a, s, v >= 0 ? v : auto_col(a.ny, (long long)a.nbatch * a.nx, a.alone != 0));
 }
 
 #endif

@@ -90,6 +90,7 @@ ColArgs cargs(msl_diff* d, const float2* src, float2* dst, float scale) {
   a.kmax = d->kmax; a.scale = scale; a.tw = d->twy.p; a.prop_rows = d->prow.p;
   a.tiles_lo = d->prune_tiles;
   a.zb_rows = d->zb_rows ? 1 : 0;
+  a.alone = 1;
   return a;
 }
 

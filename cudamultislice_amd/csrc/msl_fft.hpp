@@ -153,6 +153,19 @@ template <> struct AltPlan<512> { static constexpr int T = 32, R1 = 16, R2 = 8, 
 template <> struct AltPlan<1024> { static constexpr int T = 32, R1 = 16, R2 = 8, R3 = 8; };
 template <> struct AltPlan<2048> { static constexpr int T = 64, R1 = 16, R2 = 16, R3 = 8; };
 
+// Plans for launches of a few waves, where the chip is not full and a pass
+// takes as long as the chain of one line's own operations: four values per
+// thread, up to four stages.
+template <int N> struct SmallPlan;
+template <> struct SmallPlan<64> { static constexpr int T = 16, R1 = 4, R2 = 4, R3 = 4, R4 = 1; };
+template <> struct SmallPlan<128> { static constexpr int T = 32, R1 = 4, R2 = 4, R3 = 4, R4 = 2; };
+template <> struct SmallPlan<256> { static constexpr int T = 64, R1 = 4, R2 = 4, R3 = 4, R4 = 4; };
+template <> struct SmallPlan<512> : Plan<512> {};
+
+// radix of the fourth stage (1 for the plans of up to three)
+template <class P, class = void> struct FourthRadix { static constexpr int R = 1; };
+template <class P> struct FourthRadix<P, decltype((void)P::R4)> { static constexpr int R = P::R4; };
+
 // Exchange synchronisation: a whole workgroup, or one wavefront when every
 // line lives inside a single wave (LDS traffic of one wave is processed in
 // order; the fences keep the compiler from moving accesses across).
@@ -262,8 +275,14 @@ __device__ __forceinline__ void stockham_stage(float2 (&v)[N / T], int t, const 
 // ZIN: the line is band-limited, v[c] = 0 for E/4 <= c < 3E/4 (E = N / T).
 template <class P, int N, int DIR, class S = BlockSync, class LL = LdsLine<0>, bool ZIN = false>
 __device__ __forceinline__ void fft_line(float2 (&v)[N / P::T], int t, const float2* __restrict__ tw, const LL& lds) {
-  constexpr int T = P::T;
-  if constexpr (P::R3 > 1) {  // two exchanges: copies 0, 1 in every transform
+  constexpr int T = P::T, R4 = FourthRadix<P>::R;
+  if constexpr (R4 > 1) {
+    static_assert(!LL::kDual, "three exchanges need a barrier after each");
+    stockham_stage<N, T, P::R1, 1, DIR, false, S, 0, LL, ZIN>(v, t, tw, lds);
+    stockham_stage<N, T, P::R2, P::R1, DIR, false, S, 0>(v, t, tw, lds);
+    stockham_stage<N, T, P::R3, P::R1 * P::R2, DIR, false, S, 0>(v, t, tw, lds);
+    stockham_stage<N, T, R4, P::R1 * P::R2 * P::R3, DIR, true, S, 0>(v, t, tw, lds);
+  } else if constexpr (P::R3 > 1) {  // two exchanges: copies 0, 1 in every transform
     stockham_stage<N, T, P::R1, 1, DIR, false, S, 0, LL, ZIN>(v, t, tw, lds);
     stockham_stage<N, T, P::R2, P::R1, DIR, false, S, 1>(v, t, tw, lds);
     stockham_stage<N, T, P::R3, P::R1 * P::R2, DIR, true, S, 0>(v, t, tw, lds);

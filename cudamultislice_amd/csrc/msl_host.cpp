@@ -157,6 +157,10 @@ void row1(msl_sim* s, int mode, int mul, RowArgs a) {
   a.alone = 1;
   row(s, mode, mul, a);
 }
+void col1(msl_sim* s, int mode, int mul, ColArgs a) {
+  a.alone = 1;
+  col(s, mode, mul, a);
+}
 void col(msl_sim* s, int mode, int mul, const ColArgs& a) { HIPC(launch_col(mode, mul, a, s->stream)); }
 
 // separable Fresnel factors exp(-i pi dz lambda k^2) per axis (CreatePropsKernel,
@@ -224,7 +228,7 @@ void propagate(msl_sim* s, float2* src, float2* dst, float dz) {
   row1(s, ROW_FWD, RM_NONE, row_args(s, src, dst, 1, bs));
   ColArgs c = col_args(s, dst, dst, 1, bs);
   c.scale = s->nf * s->nf;
-  col(s, COL_FWD_MUL_INV, CM_PROP, c);
+  col1(s, COL_FWD_MUL_INV, CM_PROP, c);
   row1(s, ROW_INV, RM_NONE, row_args(s, dst, dst, 1, bs));
 }
 
@@ -578,14 +582,14 @@ void fd_step_passes(msl_sim* s) {
   ColArgs c = col_args(s, s->B.p, s->B.p, 1, bs);
   c.scale = s->nf * s->nf;
   c.tiles_lo = tiles;
-  col(s, COL_FWD_MUL_INV, CM_BAND, c);
+  col1(s, COL_FWD_MUL_INV, CM_BAND, c);
   // spectral Laplacian of psi: FFT, * nf (-4 pi^2 k^2), IFFT_y, * nf
   const bool had_lap = s->fd_lap;
   if (!had_lap) {
     row1(s, ROW_FWD, RM_NONE, row_args(s, s->Psi.p, s->G.p, 1, bs));
     c = col_args(s, s->G.p, s->G.p, 1, bs);
     c.scale = s->nf * s->nf;
-    col(s, COL_FWD_MUL_INV, CM_GRAD, c);
+    col1(s, COL_FWD_MUL_INV, CM_GRAD, c);
   }
   s->fd_lap = false;
   RowArgs r = row_args(s, s->G.p, s->V.p, 1, bs);
@@ -603,7 +607,7 @@ void fd_step_passes(msl_sim* s) {
   c.scale = s->nf * s->nf;
   c.tiles_lo = tiles;
   c.zb_rows = s->fd_zb ? 1 : 0;
-  col(s, COL_FD, CM_BAND, c);
+  col1(s, COL_FD, CM_BAND, c);
   RowArgs ri = row_args(s, s->V.p, s->PsiPlus.p, 1, bs);
   ri.prune_in = s->fd_prune;
   row1(s, ROW_INV, RM_NONE, ri);
@@ -899,7 +903,7 @@ msl_status msl_multislice_step_conv(msl_sim* s, int it) {
     ColArgs c = col_args(s, s->PsiPlus.p, s->PsiPlus.p, 1, bs);
     c.scale = s->nf * s->nf;
     c.tiles_lo = s->prune_tiles;
-    col(s, COL_FWD_MUL_INV, CM_PROP, c);
+    col1(s, COL_FWD_MUL_INV, CM_PROP, c);
     RowArgs ri = row_args(s, s->PsiPlus.p, s->Psi.p, 1, bs);
     ri.prune_in = prune;
     row1(s, ROW_INV, RM_NONE, ri);

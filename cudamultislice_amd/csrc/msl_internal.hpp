@@ -99,7 +99,8 @@ enum ColMul { CM_SCALE = 0, CM_PROP = 1, CM_BAND = 2, CM_GRAD = 3, CM_PROPCONJ =
   int tiles_lo;                                                                                          \
   /* 1: rows ny/4 .. 3ny/4 - 1 are outside |k| < kmax for every column (prop_rows_quarter; COL_FD:        \
      outside |k| <= kmax, band_rows_quarter) */                                                          \
-  int zb_rows;
+  int zb_rows;                                                                                           \
+  int alone;                 /* as RowArgs::alone */
 struct ColArgs {
   MSL_COL_ARGS()
 };
