@@ -682,7 +682,7 @@ hipError_t launch_probe_kspace(const ProbeArgs& a, hipStream_t s) {
 
 // ============================================================== tables
 // k-grids (PreCalculateFrequencies, U.cu:1877-1964; the FP32 division the host
-// takes too) and twiddles exp(-2 pi i k / n) of both axes, and the separable
+// takes too) and twiddles of both axes, and the separable
 // Fresnel factors exp(-i pi dz lambda k^2) of CreatePropsKernel
 // (U.cu:399-428), evaluated in FP64.  Made where they are used: uploads from
 // host memory cost a run of 64^2 five waits and 70 us of 440.
@@ -697,7 +697,7 @@ __global__ void k_ktables(float* kx, float* ky, float2* twx, float2* twy, int nx
   if (tw) {
     double sn, cs;
     sincospi(-2.0 * (double)i / (double)n, &sn, &cs);
-    tw[i] = make_float2((float)cs, (float)sn);
+    tw[i] = twiddle(cs, sn, i, n);
   }
 }
 hipError_t launch_ktables(float* kx, float* ky, float2* twx, float2* twy, int nx, int ny, float ksx, float ksy,

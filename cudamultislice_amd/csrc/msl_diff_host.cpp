@@ -193,7 +193,7 @@ msl_status msl_diff_create(msl_diff** out, int device, int nx, int ny, float ps,
       std::vector<float2> t(n);
       for (int k = 0; k < n; ++k) {
         const double a = -2.0 * M_PI * k / n;
-        t[k] = make_float2((float)std::cos(a), (float)std::sin(a));
+        t[k] = twiddle(std::cos(a), std::sin(a), k, n);
       }
       return t;
     };

@@ -67,57 +67,86 @@ __host__ __device__ __forceinline__ void dft4(float2& a0, float2& a1, float2& a2
   a3 = csub(t1, t3);
 }
 
+// Butterflies on fused multiply-adds.  The row passes are bound by VALU issue
+// first (82 % of the cycles at 512 points), and a factor multiplied onto a
+// value before it is added and subtracted costs four instructions of its own.
+// With the factor as c (1 + i t) the bracket takes two, and c goes into the
+// sums: a, b <- a + w b, a - w b in six instructions instead of eight, with
+// one rounding less (512 points: 9.9e-8 rms against 1.02e-7; six instructions
+// by way of 2 a - (a + w b) give 1.12e-7).  256 waves of 512^2: rows 60.0 to
+// 54.6 million vector instructions, 134 to 131 us; columns 35.0 to 32.5, 84 to
+// 81 us.
+__host__ __device__ __forceinline__ void bfly_p(float2& a, float2& b, float2 p, float c) {
+  b = make_float2(fmaf(-c, p.x, a.x), fmaf(-c, p.y, a.y));
+  a = make_float2(fmaf(c, p.x, a.x), fmaf(c, p.y, a.y));
+}
+// constant factors c (1 + DIR i t) and c (t + DIR i)
+template <int DIR> __host__ __device__ __forceinline__ void bfly_c(float2& a, float2& b, float c, float t) {
+  const float d = DIR < 0 ? -t : t;
+  bfly_p(a, b, make_float2(fmaf(-d, b.y, b.x), fmaf(d, b.x, b.y)), c);
+}
+template <int DIR> __host__ __device__ __forceinline__ void bfly_s(float2& a, float2& b, float c, float t) {
+  const float2 r = rot4<DIR>(b);
+  bfly_p(a, b, make_float2(fmaf(t, b.x, r.x), fmaf(t, b.y, r.y)), c);
+}
+// w = (c, t) from a table of forward factors (twiddle)
+template <int DIR> __host__ __device__ __forceinline__ void bfly(float2& a, float2& b, float2 w) {
+  bfly_c<DIR>(a, b, w.x, -w.y);
+}
+// the same for w W4, with W4 = exp(DIR 2 pi i / 4)
+template <int DIR> __host__ __device__ __forceinline__ void bfly_r(float2& a, float2& b, float2 w) {
+  b = rot4<DIR>(b);
+  bfly<DIR>(a, b, w);
+}
+// as bfly_c and bfly_s for the factors h (+-1 + DIR i), h = sqrt(1/2)
+template <int DIR, int SG> __host__ __device__ __forceinline__ void bfly_h(float2& a, float2& b) {
+  const float2 r = rot4<DIR>(b);
+  bfly_p(a, b, SG > 0 ? cadd(b, r) : csub(r, b), 0.70710678118654752f);
+}
+
+// Transforms of R values in place, natural order in and out.  Even and odd
+// members each give a transform of R/2; member k of the odd one joins with
+// the factor exp(DIR 2 pi i k / R).
 // Z: a[2..5] = 0 on entry
 template <int DIR, bool Z = false> __host__ __device__ __forceinline__ void dft8(float2 (&a)[8]) {
-  constexpr float h = 0.70710678118654752f;
   float2 e0 = a[0], e1 = a[2], e2 = a[4], e3 = a[6];
   float2 o0 = a[1], o1 = a[3], o2 = a[5], o3 = a[7];
   dft4<DIR, Z>(e0, e1, e2, e3);
   dft4<DIR, Z>(o0, o1, o2, o3);
-  // o1 *= W8^1, o2 *= W8^2, o3 *= W8^3 with W8 = exp(DIR 2 pi i / 8)
-  if (DIR < 0) {
-    o1 = make_float2(h * (o1.x + o1.y), h * (o1.y - o1.x));
-    o3 = make_float2(h * (o3.y - o3.x), -h * (o3.x + o3.y));
-  } else {
-    o1 = make_float2(h * (o1.x - o1.y), h * (o1.x + o1.y));
-    o3 = make_float2(-h * (o3.x + o3.y), h * (o3.x - o3.y));
-  }
   o2 = rot4<DIR>(o2);
+  bfly_h<DIR, 1>(e1, o1);
+  bfly_h<DIR, -1>(e3, o3);
   a[0] = cadd(e0, o0); a[4] = csub(e0, o0);
-  a[1] = cadd(e1, o1); a[5] = csub(e1, o1);
   a[2] = cadd(e2, o2); a[6] = csub(e2, o2);
-  a[3] = cadd(e3, o3); a[7] = csub(e3, o3);
+  a[1] = e1; a[5] = o1;
+  a[3] = e3; a[7] = o3;
 }
 
 // Z: a[4..11] = 0 on entry
 template <int DIR, bool Z = false> __host__ __device__ __forceinline__ void dft16(float2 (&a)[16]) {
-  // 16 = 4 x 4: DFT4 over n1 (stride 4), twiddle W16^(n2 k1), DFT4 over n2
-  constexpr float c1 = 0.92387953251128674f, s1 = 0.38268343236508977f, h = 0.70710678118654752f;
+  constexpr float c1 = 0.92387953251128674f, t1 = 0.41421356237309505f;  // cos, tan of pi / 8
+  float2 e[8], o[8];
 #pragma unroll
-  for (int n2 = 0; n2 < 4; ++n2) dft4<DIR, Z>(a[n2], a[n2 + 4], a[n2 + 8], a[n2 + 12]);
-  // now a[n2 + 4 k1] = B[n2][k1]; apply W16^(n2*k1), W16 = exp(DIR 2 pi i/16)
-  const float sg = DIR < 0 ? -1.f : 1.f;
-  const float2 w1 = make_float2(c1, sg * s1), w2 = make_float2(h, sg * h), w3 = make_float2(s1, sg * c1);
-  const float2 w6 = make_float2(-h, sg * h), w9 = make_float2(-c1, -sg * s1);
-  a[1 + 4] = cmul(a[1 + 4], w1);
-  a[1 + 8] = cmul(a[1 + 8], w2);
-  a[1 + 12] = cmul(a[1 + 12], w3);
-  a[2 + 4] = cmul(a[2 + 4], w2);
-  a[2 + 8] = rot4<DIR>(a[2 + 8]);
-  a[2 + 12] = cmul(a[2 + 12], w6);
-  a[3 + 4] = cmul(a[3 + 4], w3);
-  a[3 + 8] = cmul(a[3 + 8], w6);
-  a[3 + 12] = cmul(a[3 + 12], w9);
+  for (int i = 0; i < 8; ++i) {
+    e[i] = a[2 * i];
+    o[i] = a[2 * i + 1];
+  }
+  dft8<DIR, Z>(e);
+  dft8<DIR, Z>(o);
+  dft2<DIR>(e[0], o[0]);
+  bfly_c<DIR>(e[1], o[1], c1, t1);
+  bfly_h<DIR, 1>(e[2], o[2]);
+  bfly_s<DIR>(e[3], o[3], c1, t1);
+  o[4] = rot4<DIR>(o[4]);
+  dft2<DIR>(e[4], o[4]);
+  bfly_s<DIR>(e[5], o[5], c1, -t1);
+  bfly_h<DIR, -1>(e[6], o[6]);
+  bfly_c<DIR>(e[7], o[7], -c1, -t1);
 #pragma unroll
-  for (int k1 = 0; k1 < 4; ++k1) dft4<DIR>(a[4 * k1 + 0], a[4 * k1 + 1], a[4 * k1 + 2], a[4 * k1 + 3]);
-  // a[4 k1 + k2] holds X[k1 + 4 k2]; transpose into natural order
-  float2 o[16];
-#pragma unroll
-  for (int k1 = 0; k1 < 4; ++k1)
-#pragma unroll
-    for (int k2 = 0; k2 < 4; ++k2) o[k1 + 4 * k2] = a[4 * k1 + k2];
-#pragma unroll
-  for (int i = 0; i < 16; ++i) a[i] = o[i];
+  for (int i = 0; i < 8; ++i) {
+    a[i] = e[i];
+    a[i + 8] = o[i];
+  }
 }
 
 // Z: a[R/4 .. 3R/4 - 1] = 0 on entry (R >= 4)
@@ -127,6 +156,37 @@ template <int R, int DIR, bool Z = false> __host__ __device__ __forceinline__ vo
   else if constexpr (R == 4) dft4<DIR, Z>(a[0], a[1], a[2], a[3]);
   else if constexpr (R == 8) dft8<DIR, Z>(a);
   else if constexpr (R == 16) dft16<DIR, Z>(a);
+}
+
+// The same with member m multiplied by w^m, w = tw[k] of a table of N: the
+// powers of w go with the factors of the joins, so only w, w^2, w^4, ... and
+// the first join's products are read, half of the R - 1 powers.
+template <int R, int N, int DIR, class TW>
+__host__ __device__ __forceinline__ void dft_tw(float2 (&a)[R], const TW tw, int k) {
+  if constexpr (R == 2) {
+    bfly<DIR>(a[0], a[1], tw[k]);
+  } else {
+    constexpr int H = R / 2;
+    float2 e[H], o[H];
+#pragma unroll
+    for (int i = 0; i < H; ++i) {
+      e[i] = a[2 * i];
+      o[i] = a[2 * i + 1];
+    }
+    dft_tw<H, N, DIR>(e, tw, 2 * k);
+    dft_tw<H, N, DIR>(o, tw, 2 * k);
+#pragma unroll
+    for (int i = 0; i < (H + 1) / 2; ++i) {
+      const float2 w = tw[k + i * (N / R)];
+      bfly<DIR>(e[i], o[i], w);
+      if constexpr (H > 1) bfly_r<DIR>(e[i + H / 2], o[i + H / 2], w);
+    }
+#pragma unroll
+    for (int i = 0; i < H; ++i) {
+      a[i] = e[i];
+      a[i + H] = o[i];
+    }
+  }
 }
 
 // Per-length plan: T threads per line, radices of up to three stages.
@@ -232,16 +292,8 @@ __device__ __forceinline__ void stockham_stage(float2 (&v)[N / T], int t, const 
     float2 a[R];
 #pragma unroll
     for (int m = 0; m < R; ++m) a[m] = v[b + m * NB];
-    if constexpr (L > 1) {
-      constexpr int step = N / (L * R);
-#pragma unroll
-      for (int m = 1; m < R; ++m) {
-        float2 w = tw[m * k * step];
-        if (DIR > 0) w.y = -w.y;
-        a[m] = cmul(a[m], w);
-      }
-    }
-    dftR<R, DIR, ZIN>(a);
+    if constexpr (L > 1) dft_tw<R, N, DIR>(a, tw, k * (N / (L * R)));
+    else dftR<R, DIR, ZIN>(a);
     if constexpr (LAST) {
 #pragma unroll
       for (int m = 0; m < R; ++m) out[b + m * NB] = a[m];
@@ -270,7 +322,7 @@ __device__ __forceinline__ void stockham_stage(float2 (&v)[N / T], int t, const 
 }
 
 // Full transform of one line with plan P (T threads, radices R1 R2 R3).
-// tw points at the N-entry table exp(-2 pi i k / N).  Every thread that
+// tw points at the N-entry table exp(-2 pi i k / N) (twiddle).  Every thread that
 // shares the synchronisation scope must call this together.
 // ZIN: the line is band-limited, v[c] = 0 for E/4 <= c < 3E/4 (E = N / T).
 template <class P, int N, int DIR, class S = BlockSync, class LL = LdsLine<0>, bool ZIN = false>

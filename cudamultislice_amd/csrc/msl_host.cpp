@@ -94,7 +94,7 @@ std::vector<float2> twiddles(int n) {
   std::vector<float2> t(n);
   for (int k = 0; k < n; ++k) {
     const double a = -2.0 * M_PI * (double)k / (double)n;
-    t[k] = make_float2((float)std::cos(a), (float)std::sin(a));
+    t[k] = twiddle(std::cos(a), std::sin(a), k, n);
   }
   return t;
 }

@@ -8,6 +8,16 @@
 
 namespace msl {
 
+// Entry k of the passes' table exp(-2 pi i k / n) = cs + i sn: (c, t) with
+// the factor c (1 + i t), the form that the butterflies take.  t is the sine
+// over the rounded c, so that c t has one rounding; where the cosine is zero
+// c is 2^-40 and c t exact.
+__host__ __device__ inline float2 twiddle(double cs, double sn, int k, int n) {
+  if (4 * k == n || 4 * k == 3 * n) return make_float2(0x1p-40f, sn < 0 ? -0x1p40f : 0x1p40f);
+  const float c = (float)cs;
+  return make_float2(c, (float)(sn / (double)c));
+}
+
 // ------------------------------------------------------------------ passes
 // Row pass: one transform along x (contiguous) per (wave, row) line.
 enum RowMode { ROW_FWD = 0, ROW_INV = 1, ROW_INV_MUL_FWD = 2, ROW_INV_FD_FWD = 3 };
@@ -40,7 +50,7 @@ enum RowMul { RM_NONE = 0, RM_T = 1, RM_SEED = 2 };
   float sigma;                                                                                           \
   float scale;               /* applied with the pointwise factor */                                     \
   int prune_in, prune_out;   /* band-limited input / output (only x < N/4, x >= 3N/4) */                 \
-  const float2 G* tw;        /* twiddles for length nx */                                                \
+  const float2 G* tw;        /* twiddle() for length nx */                                               \
   const int G* t_index;      /* optional per-wave transmission slot (device) */                          \
   /* ROW_INV_MUL_FWD: also store the real-space wave (before the multiply) here, same indexing as dst */ \
   float2 G* aux;                                                                                         \
@@ -88,7 +98,7 @@ enum ColMul { CM_SCALE = 0, CM_PROP = 1, CM_BAND = 2, CM_GRAD = 3, CM_PROPCONJ =
   const int2 G* prop_rows;                                                                               \
   float kmax;                                                                                            \
   float scale;                                                                                           \
-  const float2 G* tw;        /* twiddles for length ny */                                                \
+  const float2 G* tw;        /* twiddle() for length ny */                                               \
   /* COL_FWD_DETECT: annular sum of |v|^2 over kin <= |k| < kout, times det_scale, into */              \
   /* partial[b * (nx / C) + tile]; optional per-wave |v|^2 map (fftshifted) into inten */                \
   float kin, kout, det_scale;                                                                            \

@@ -45,13 +45,13 @@ hipError_t scratch_ptr(float2** out) {
   return hipSuccess;
 }
 
-// tw[k] = exp(-2 pi i k / n), k < n, in double then rounded to float (the
+// twiddle() of exp(-2 pi i k / n), k < n, from double (the
 // host tables of msl_fft2_device are computed the same way)
 __global__ void k_twiddles(float2* tw, int n) {
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= n) return;
   const double a = -2.0 * M_PI * (double)k / (double)n;
-  tw[k] = make_float2((float)cos(a), (float)sin(a));
+  tw[k] = twiddle(cos(a), sin(a), k, n);
 }
 
 }  // namespace

@@ -45,7 +45,7 @@ struct Bench {
       const double a = 3.14159265 * 2.0 * 0.0197 * (double)kk[i] * kk[i];
       p[i] = make_float2((float)std::cos(a), (float)-std::sin(a));
       const double b = -2.0 * M_PI * i / n;
-      w[i] = make_float2((float)std::cos(b), (float)std::sin(b));
+      w[i] = twiddle(std::cos(b), std::sin(b), i, n);
     }
     hipError_t e;
     if ((e = hipMemcpyAsync(k.p, kk.data(), n * 4, hipMemcpyHostToDevice, s)) != hipSuccess) return e;
