@@ -50,15 +50,16 @@ __global__ void __launch_bounds__((AdjCfg<N, REAL_Z>::L * Plan<N>::T)) k_row_adj
   constexpr int T = Plan<N>::T, E = N / T, LINES = Cfg::L, LS = Cfg::LS, NT = LINES * T;
   static_assert(LS * 2 >= N, "the reduction reuses the line buffers");
   __shared__ float2 lds[LINES * LS];
-  __shared__ float2 stw[N];  // twiddles staged in LDS
+  __shared__ float2 stw[N / 2];  // twiddles staged in LDS
   const int tid = threadIdx.x, t = tid % T, ln = tid / T;
   const int y = blockIdx.x, g = blockIdx.y;
   // the first probe's gradient row is requested with the twiddles and the
   // transmissions: one wait before the first transform
-  float2 twr[(N + NT - 1) / NT];
+  constexpr int NTW = (N / 2 + NT - 1) / NT;
+  float2 twr[NTW];
 #pragma unroll
-  for (int k = 0; k < (N + NT - 1) / NT; ++k)
-    if (tid + k * NT < N) twr[k] = a.tw[tid + k * NT];
+  for (int k = 0; k < NTW; ++k)
+    if (tid + k * NT < N / 2) twr[k] = a.tw[tid + k * NT];
   float2 tr[E];
   {
     const float2* trow = a.t + (long long)y * N;
@@ -99,8 +100,8 @@ __global__ void __launch_bounds__((AdjCfg<N, REAL_Z>::L * Plan<N>::T)) k_row_adj
   float2 gn[E];
   if constexpr (PIPE) load_g(gn, row_of(0));
 #pragma unroll
-  for (int k = 0; k < (N + NT - 1) / NT; ++k)
-    if (tid + k * NT < N) stw[tid + k * NT] = twr[k];
+  for (int k = 0; k < NTW; ++k)
+    if (tid + k * NT < N / 2) stw[tid + k * NT] = twr[k];
   __syncthreads();
   // band-limited inputs (PRUNE): the first butterflies skip the zero blocks
   constexpr bool ZIN = PRUNE && E % 4 == 0 && Plan<N>::R1 % 4 == 0;

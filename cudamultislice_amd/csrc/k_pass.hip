@@ -271,7 +271,7 @@ template <int E> struct BandBlocks {
 };
 
 // The row pass body: the LINES lines of workgroup-sized block blk; lds holds
-// LINES * LS elements, tw the N twiddles staged in LDS.  k_row (one length
+// LINES * LS elements, stw the first N / 2 twiddles staged in LDS.  k_row (one length
 // per launch, arguments in kernel registers) and k_row_group (several
 // lengths per launch, arguments read from a table in device memory) both
 // expand this one body.
@@ -450,9 +450,9 @@ __device__ __forceinline__ long long row_order(long long h, long long total, int
 template <int N, int MODE, int MUL, int FL, int RV>
 __global__ void __launch_bounds__((RowCfg<N, RV>::LINES * RowCfg<N, RV>::T)) k_row(RowArgs a) {
   __shared__ float2 lds[RowCfg<N, RV>::LINES * RowCfg<N, RV>::LS];
-  __shared__ float2 stw[N];  // twiddles staged in LDS: no global loads inside the transforms
+  __shared__ float2 stw[N / 2];  // twiddles staged in LDS: no global loads inside the transforms
   constexpr int NT = RowCfg<N, RV>::LINES * RowCfg<N, RV>::T;
-  const TwStage<N, NT> tws(a.tw);
+  const TwStage<N / 2, NT> tws(a.tw);
   long long blk = blockIdx.x;
   // wave-interleaved, XCD-aware order where a shared slice outgrows the L2
   // (measured slower than the plain order at 1024 and below, where the slice
@@ -488,9 +488,9 @@ __global__ void __launch_bounds__((RowPL<N>::LINES * RowPL<N>::T)) k_row_pl(RowA
   using LL = LdsLine<Cfg::SH>;
   constexpr int T = Cfg::T, E = N / T, LINES = Cfg::LINES, LS = Cfg::LS, NT = LINES * T;
   __shared__ float2 lds[LINES * LS];
-  __shared__ float2 stw[N];
+  __shared__ float2 stw[N / 2];
   const int tid = threadIdx.x, t = tid % T, ln = tid / T;
-  for (int i = tid; i < N; i += NT) stw[i] = a.tw[i];
+  for (int i = tid; i < N / 2; i += NT) stw[i] = a.tw[i];
   const int y = blockIdx.x, g = blockIdx.y;
   // lines past the batch read wave 0 and store nothing
   auto wave_of = [&](int q) { return (g * per_line + q) * LINES + ln; };
@@ -670,7 +670,7 @@ __device__ __forceinline__ void col_body(float2 (&v)[N / P::T], int t, int x, co
 // variants 0, 1: the C columns of a tile spread over the workgroup, thread
 // (col, t) holds rows t + c T of column col; workgroup barriers
 // launched tile bx (of nbx per wave) of wave b; lds holds Cfg::LDS elements,
-// stw the twiddles of length N
+// stw the first half of the twiddles of length N
 // (staged() as in row_block; py the propagator's row factors, ky the rows'
 // frequencies)
 template <int N, int MODE, int MUL, class Cfg, class A, class PY, class KY, class F>
@@ -770,13 +770,13 @@ template <int N, int MODE, int MUL, int CV>
 __global__ void __launch_bounds__((ColCfg<N, CV>::THREADS), (ColCfg<N, CV>::MIN_WAVES)) k_col(ColArgs a) {
   using Cfg = ColCfg<N, CV>;
   __shared__ float2 lds[Cfg::LDS];
-  __shared__ float2 stw[N];  // twiddles staged in LDS
+  __shared__ float2 stw[N / 2];  // twiddles staged in LDS
   // and the propagator's row factors: read between the transforms, where a
   // load from memory would stall the workgroup
   constexpr bool ROWS = needs_rows<MODE, MUL>(), FREQ = needs_k<MODE, MUL>();
   __shared__ float2 spy[ROWS ? N : 1];
   __shared__ float sky[FREQ ? N : 1];
-  const TwStage<N, Cfg::THREADS> tws(a.tw);
+  const TwStage<N / 2, Cfg::THREADS> tws(a.tw);
   const TwStage<ROWS ? N : 1, Cfg::THREADS> pys(ROWS ? a.py : a.tw);
   if constexpr (FREQ)
     for (int i = threadIdx.x; i < N; i += Cfg::THREADS) sky[i] = a.ky[i];
@@ -806,8 +806,8 @@ __global__ void __launch_bounds__((ColCfg<N, ColPL<N>::CV>::THREADS), 4) k_col_p
   using LL = LdsLine<Cfg::SH>;
   constexpr int T = Cfg::T, E = N / T, C = Cfg::C;
   __shared__ float2 lds[Cfg::LDS];
-  __shared__ float2 stw[N];
-  for (int i = threadIdx.x; i < N; i += Cfg::THREADS) stw[i] = a.tw[i];
+  __shared__ float2 stw[N / 2];
+  for (int i = threadIdx.x; i < N / 2; i += Cfg::THREADS) stw[i] = a.tw[i];
   const long long gid = xcd_remap((long long)blockIdx.y * gridDim.x + blockIdx.x, (long long)gridDim.x * gridDim.y);
   const int bx = (int)(gid % gridDim.x), g = (int)(gid / gridDim.x);
   const int col = threadIdx.x % C, t = threadIdx.x / C;
@@ -874,7 +874,7 @@ template <int N> constexpr int group_row_lds() { return RowCfg<N, GroupRow<N>::R
 constexpr int kGroupRowLds = cmax(cmax(group_row_lds<256>(), group_row_lds<512>()),
                                   cmax(group_row_lds<1024>(), group_row_lds<2048>()));
 constexpr int kGroupColLds = cmax(cmax(GroupCol<256>::LDS, GroupCol<512>::LDS), cmax(GroupCol<1024>::LDS, GroupCol<2048>::LDS));
-constexpr int kGroupTw = 2048;
+constexpr int kGroupTw = 1024;  // twiddles staged: half of the longest line's
 
 // Segment boundaries and lengths as plain kernel arguments: the segment of a
 // workgroup and its length come from scalar compares and selects, and only
@@ -903,7 +903,7 @@ __global__ void __launch_bounds__(256) k_row_group(const PassGroup<RowArgs>* g, 
   const long long blk = it - pick4<long long>(s, 0, h.b1, h.b2, h.b3);
   const int n = pick4(s, h.n0, h.n1, h.n2, h.n3);
   const RowArgsG& a = reinterpret_cast<const RowArgsG*>(g->a)[s];
-  for (int i = threadIdx.x; i < n; i += 256) stw[i] = a.tw[i];
+  for (int i = threadIdx.x; i < n / 2; i += 256) stw[i] = a.tw[i];
   __syncthreads();
   switch (n) {
     case 256: row_block<256, MODE, MUL, FL, GroupRow<256>::RV>(a, blk, lds, stw, [] {}); break;
@@ -930,7 +930,7 @@ __global__ void __launch_bounds__(512) k_col_group(const PassGroup<ColArgs>* g, 
   const int n = pick4(s, h.n0, h.n1, h.n2, h.n3), nbx = pick4(s, h.x0, h.x1, h.x2, h.x3);
   const int b = (int)(blk / nbx), bx = (int)(blk - (long long)b * nbx);
   const ColArgsG& a = reinterpret_cast<const ColArgsG*>(g->a)[s];
-  for (int i = threadIdx.x; i < n; i += 512) stw[i] = a.tw[i];
+  for (int i = threadIdx.x; i < n / 2; i += 512) stw[i] = a.tw[i];
   __syncthreads();
   switch (n) {
     case 256: col_block<256, MODE, MUL, GroupCol<256>>(a, bx, b, nbx, lds, stw, a.py, a.ky, [] {}); break;

@@ -160,7 +160,9 @@ template <int R, int DIR, bool Z = false> __host__ __device__ __forceinline__ vo
 
 // The same with member m multiplied by w^m, w = tw[k] of a table of N: the
 // powers of w go with the factors of the joins, so only w, w^2, w^4, ... and
-// the first join's products are read, half of the R - 1 powers.
+// the first join's products are read, half of the R - 1 powers, and of the
+// table the first half (k < N / R: a join of R reads below N / 4, of two
+// below N / 2).
 template <int R, int N, int DIR, class TW>
 __host__ __device__ __forceinline__ void dft_tw(float2 (&a)[R], const TW tw, int k) {
   if constexpr (R == 2) {
@@ -322,7 +324,7 @@ __device__ __forceinline__ void stockham_stage(float2 (&v)[N / T], int t, const 
 }
 
 // Full transform of one line with plan P (T threads, radices R1 R2 R3).
-// tw points at the N-entry table exp(-2 pi i k / N) (twiddle).  Every thread that
+// tw points at the first N / 2 entries of the table exp(-2 pi i k / N) (twiddle).  Every thread that
 // shares the synchronisation scope must call this together.
 // ZIN: the line is band-limited, v[c] = 0 for E/4 <= c < 3E/4 (E = N / T).
 template <class P, int N, int DIR, class S = BlockSync, class LL = LdsLine<0>, bool ZIN = false>
