@@ -114,14 +114,15 @@ void set_pass_variant(int kind, int n, int v) {
 //   128  1: 4.4, 4.6; 2: 3.7, 3.9; s: 3.2, 3.4 (from 37 waves on 1)
 //   256  1: 4.7 at 1, 5.0 at 8, 5.1 at 12; 2: 3.8, 4.1, 5.2; s: 3.3, 4.2, 5.2
 //   512  1: 4.2 at 1 wave (2: 5.8); at 24 waves 3: 15.7, 4: 18.2; at 64 3: 40.2, 4: 38.1
-//  1024  1: 6.5 at 1 wave (3: 7.9); at 8 waves 3: 23.9, 4: 25.4; at 16 3: 44.5, 4: 42.6
+//  1024  1: 6.6 at 1 wave (3: 8.0); at 8 waves 1: 21.7, 3: 22.0, 4: 23.5; at 16 38.9, 40.8, 39.0;
+//        at 32 75.9, 76.9, 70.6
 static int auto_row(int n, long long lines, bool alone) {
   switch (n) {
     case 64:
     case 128:
     case 256: return alone && lines <= 3072 ? kSmallRow : kRowDefault[lg2(n)];
     case 512: return !alone || lines > 20480 ? 4 : lines <= 1024 ? 1 : 3;
-    case 1024: return lines <= 2048 ? 1 : lines <= 12288 ? 3 : 4;
+    case 1024: return lines <= 16384 ? 1 : 4;
   }
   return kRowDefault[lg2(n)];
 }
@@ -1093,7 +1094,7 @@ static hipError_t row_nv(int mode, int mul, const RowArgs& a, hipStream_t s) {
 }
 
 // variant 4 where its layout applies (see k_row_pl); elsewhere the best of
-// the other layouts for the length (2 at 512, 3 at 1024, 1 otherwise)
+// the other layouts for the length (2 at 512, 1 otherwise)
 template <int N>
 static hipError_t row_pl(int mode, int mul, const RowArgs& a, hipStream_t s) {
   const bool shared_t = a.t && !a.t_index && a.t_group >= a.nbatch;
@@ -1106,7 +1107,6 @@ static hipError_t row_pl(int mode, int mul, const RowArgs& a, hipStream_t s) {
   if (mode != ROW_INV_MUL_FWD || mul != RM_T || !(shared_t || slots) || a.ny > 65535 ||
       a.nbatch < 2 * RowPL<N>::LINES) {
     if constexpr (N == 512) return row_nv<N, 2>(mode, mul, a, s);
-    else if constexpr (N == 1024) return row_nv<N, 3>(mode, mul, a, s);
     else return row_nv<N, 1>(mode, mul, a, s);
   }
   if (a.nbatch <= 0) return hipSuccess;
