@@ -205,7 +205,8 @@ typedef struct {
   float dz;               /* slice thickness (A) */
   int nslices;            /* 0: ceil((MaxZ - MinZ) / dz) */
   float adf_inner, adf_outer; /* mrad */
-  int batch;              /* probes per launch, 0: automatic */
+  int batch;              /* probes per launch, 0: the tuned width, else as many as keep their
+                             in-band waves in the Infinity Cache (256 MB) */
   int use_graph;          /* capture one chunk (probe synthesis, slice loop, detector) in a
                              hipGraph per chunk size and replay it for every chunk and
                              configuration; ignored with exit_out or while per-kernel
