@@ -71,20 +71,13 @@ constexpr int kSmallCol = 8;  // as column 0 with SmallPlan and tiles of four co
 //         7 as 2 with half as many columns per workgroup
 // (a staged column layout with one wavefront per column and an LDS pad of
 // 1/8 were measured slower or equal on MI355X and were removed)
-// defaults from msl_autotune_passes on MI355X (band-pruned passes, 1-4 GiB
-// of waves): rows of 512 take the alternative plan (0.67 vs 0.71 ms per 1024
-// waves for 1), rows of 1024 the 512-thread workgroups (0.81 vs 0.91 ms per
-// 256 waves); rows of 512 and 1024 then went to variant 4 (one workgroup per
-// row looping over waves; 512: 0.58 vs 0.69 ms per 1024 waves for 2, 1024:
-// 0.78 vs 0.85 ms per 256 waves for 3; 1.131 vs 1.080e6 probe-slice/s on the
-// 512^2 STEM workload).  Columns: 512 half-width tiles (with the row factors
-// in LDS 72.1 us per 256 waves against 73.1 on the alternative plan, which
-// was ahead before); 256, 1024 and 2048 variant 0 (1024: 0.54 vs 0.62 ms per
-// 256 waves for the half-width tiles once the inverse skipped the
-// propagator's zero rows).  At 2048 the
-// loops over waves won once they existed: rows variant 4 (0.447-0.469 vs
-// 0.525-0.531 ms per 32 waves for variant 1), columns variant 5 (0.376-0.378
-// vs 0.440-0.447 ms for variant 0); at 256 variants 1 and 0 stay fastest.
+// Defaults of large launches, us per launch of band-pruned passes on MI355X.
+// Rows: 512 and 1024 the workgroup per row (512, 256 waves: 4 124, 2 132, 1
+// 143, 3 142; 1024, 32 waves: 4 70, 1 76, 3 78; 2048, 32 waves: 4 363, 3 367, 2
+// 372, 1 379); 256 and below variant 1.  Columns: 512 half-width tiles (with
+// the row factors in LDS 68.0 per 256 waves, 69.2 on the alternative plan, 78
+// full width); 2048 the loop over waves (32 waves: 5 338, 0 420); 1024 full
+// width (32 waves: 0 49.2, 3 50.8, 5 52.6); 256 and below variant 0.
 #ifndef MSL_PASS_LEN
 static const int kRowDefault[12] = {0, 0, 0, 0, 1, 1, 1, 1, 1, 4, 4, 4};
 static const int kColDefault[12] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 3, 0, 5};
@@ -110,17 +103,16 @@ void set_pass_variant(int kind, int n, int v) {
 // (RowArgs::alone), so that a wave's result does not depend on how a run is
 // cut into batches.
 // Us per launch of IFFT -> t -> FFT (variant:time; s the small layout):
-//    64  0: 3.3 at 1 wave of n x n, 3.5 at 16; 1: 3.0, 3.2; s: 2.7, 2.9
-//   128  1: 4.4, 4.6; 2: 3.7, 3.9; s: 3.2, 3.4 (from 37 waves on 1)
-//   256  1: 4.7 at 1, 5.0 at 8, 5.1 at 12; 2: 3.8, 4.1, 5.2; s: 3.3, 4.2, 5.2
-//   512  1: 4.2 at 1 wave (2: 5.8); at 24 waves 3: 15.7, 4: 18.2; at 64 3: 40.2, 4: 38.1
-//  1024  1: 6.6 at 1 wave (3: 8.0); at 8 waves 1: 21.7, 3: 22.0, 4: 23.5; at 16 38.9, 40.8, 39.0;
-//        at 32 75.9, 76.9, 70.6
+//    64  0: 3.3 at 1 wave of n x n, 3.5 at 16; 1: 3.0, 3.2; s: 2.7, 2.8
+//   128  1: 4.2 at 1, 4.4 at 16, 4.6 at 37; 2: 3.6, 3.7, 4.6; s: 3.1, 3.3, 4.6
+//   256  1: 4.5 at 1, 4.7 at 8, 4.8 at 12; 2: 3.7, 3.9, 4.9; s: 3.2, 3.9, 4.9
+//   512  1: 4.1 at 1 (2: 5.5, 3: 4.6), 5.1 at 4 (3: 5.0); at 24 3: 15.4, 4: 17.2; at 64 3: 37.0, 4: 34.8
+//  1024  1: 6.1 at 1, 21.8 at 8, 39.4 at 16, 75.6 at 32; 3: 7.4, 21.9, 41.5, 77.7; 4: -, 23.6, 39.3, 69.9
 static int auto_row(int n, long long lines, bool alone) {
   switch (n) {
     case 64:
     case 128:
-    case 256: return alone && lines <= 3072 ? kSmallRow : kRowDefault[lg2(n)];
+    case 256: return alone && lines <= 2048 ? kSmallRow : kRowDefault[lg2(n)];
     case 512: return !alone || lines > 20480 ? 4 : lines <= 1024 ? 1 : 3;
     case 1024: return lines <= 16384 ? 1 : 4;
   }
@@ -132,14 +124,16 @@ static int auto_row(int n, long long lines, bool alone) {
 // have a tile or two, half-width tiles (twice the workgroups, the same bits
 // as 0) while the full ones leave CUs idle, and at 512 always.  Us per
 // launch of the propagation pass, variants 0, 3 and small:
-//   64   3.0, 3.0, 3.1 at 1 wave of n x n; 3.3, 2.9, 2.7 at 16
-//  128   4.0, 4.3, 3.6 at 1; 4.3, 4.0, 3.4 at 16
-//  256   5.2, 4.4, 3.7 at 1; 5.4, 4.8, 4.7 at 12; 8.1, 8.2, - at 64
-//  512   8.1, 5.3, 4.7 at 1; 8.1, 5.5, 5.0 at 2; 8.4, 5.6, 5.6 at 4; 16.3, 11.0, - at 24;
-//        128, 72.1, - at 256 (variant 7: 6.2, 6.3, 6.5, 11.7, 73.1)
-//  1024  8.5, 7.8, 7.9 at 1; 8.9, 8.8, 10.3 at 2; 16.1, 19.1, - at 8
+//   64   3.0, 3.2, 3.4 at 1 wave of n x n; 3.1, 3.2, 3.0 at 2; 3.3, 3.1, 3.0 at 16
+//  128   4.2, 4.1, 3.8 at 1; 4.5, 3.9, 3.6 at 16
+//  256   5.3, 4.2, 4.0 at 1; 5.4, 4.4, 4.4 at 8; 5.5, 4.5, 4.9 at 12; 7.8, 7.9, 10.2 at 64
+//  512   7.8, 5.5, 4.5 at 1; 7.9, 5.6, 4.8 at 2; 8.0, 5.8, 5.4 at 4; 12.5, 10.9, 12.3 at 24;
+//        78, 68, 78 at 256 (variant 7: 6.0, 6.1, 6.4, 11.3, 69)
+//  1024  8.2, 7.6, - at 1; 8.7, 8.7, - at 2; 15.6, 19.0, - at 8
 static int auto_col(int n, long long cols, bool alone) {
-  if (n == 512 ? cols <= 1024 : (n >= 64 && n <= 256 && alone && cols <= 3072)) return kSmallCol;
+  if (n == 64 && cols <= 64) return 0;
+  if (n == 512 ? cols <= 2048 : n == 256 ? alone && cols <= 1024 : n >= 64 && n <= 128 && alone && cols <= 2048)
+    return kSmallCol;
   const int half = n == 64 ? 4096 : n == 256 ? 8192 : n == 1024 ? 1024 : 0;
   return cols <= half ? 3 : kColDefault[lg2(n)];
 }
