@@ -214,9 +214,7 @@ template <int N, int RV> struct RowCfg {
   static constexpr int T = P::T;
   static constexpr bool WAVE = RV >= 1 && T <= 64;
   static constexpr int SH = RV >= 1 ? 4 : 0;
-  // variant 3: 512-thread workgroups (eight one-wave lines at 512 and 1024:
-  // two workgroups, sixteen waves per CU at 1024, where four-line
-  // workgroups of 43 KB of LDS fit three)
+  // variant 3: 512-thread workgroups (eight one-wave lines at 512 and 1024)
   static constexpr int LINES = ((RV == 3 ? 512 : 256) / T) > 0 ? (RV == 3 ? 512 : 256) / T : 1;
   static constexpr int LS = LdsLine<SH>::span(N) + 1;
 };

@@ -327,8 +327,8 @@ __device__ __forceinline__ float readlane_f(float v, int l) {
 // per sample), by those three loads and the launch at small ones.  Per slice,
 // before (slab after slab, transcendentals, a divergent loop per pixel) and
 // now: Si 1024^2 of 0.074 A 114.6 -> 34.5 us, SrTiO3 512^2 of 0.078 A 51.0 ->
-// 17.2, Si 256^2 of 0.085 A 27.9 -> 8.5, 64^2 of 0.2 A 27.2 -> 6.7; one plane
-// of Si at 256^2 16.0 -> 5.5.
+// 17.2, Si 256^2 of 0.085 A 27.9 -> 7.9, 64^2 of 0.2 A 27.2 -> 5.8; one plane
+// of Si at 256^2 16.0 -> 4.6.
 template <int TX, int TY, int SPLIT, int KIND, class A>
 __device__ __forceinline__ void potential_tile(const A& a, int tx, int ty, int slice, float4* tabs) {
   static_assert(TX * TY * SPLIT == 256, "256-thread workgroups");
