@@ -44,3 +44,24 @@ def test_steps_of_one_wave_match_the_oracle(fp, nx, ny):
     got, want = g.get_wave(), o.wave()
     assert np.linalg.norm(got - want) < 2e-5 * np.linalg.norm(want)
     g.close()
+
+
+@pytest.mark.parametrize("n", [64, 256, 512, 1024])
+def test_a_probe_has_the_same_bits_in_every_batch(n):
+    """Launches of one to nine waves of a batched run cross the rules' sizes;
+    layouts they may choose among share a plan: the same bits."""
+    Z, x, y, z = S.srtio3(2, 2, 2)
+    g = MultisliceSimulation()
+    g.set_atoms(Z, x, y, z)
+    g.GetParameterisation()
+    g.UploadBinnedAtoms()
+    g.ApplyMicroscopeParameters(200.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 15.0)
+    g.STEMSetCalculationVariables(12.0 / n, 0.0, n, n, 1, 1, 1)
+    g.PreCalculateFrequencies()
+    g.STEMInitialiseWavefunctions(n // 2, n // 2)
+    px = np.arange(9, dtype=np.int32) * (n // 16) + 3
+    runs = [g.stem_batched(px, px[::-1].copy(), dz=1.0, nslices=4, adf=(5.0, 40.0), batch=b, exit_waves=True)
+            for b in (9, 1, 2, 5)]
+    for r in runs[1:]:
+        assert np.array_equal(r["exit"], runs[0]["exit"]) and np.array_equal(r["adf"], runs[0]["adf"])
+    g.close()
