@@ -406,7 +406,12 @@ __device__ __forceinline__ void potential_tile(const A& a, int tx, int ty, int s
       base = 0;
       for (int sp = 1; sp < a.nspec; ++sp) base = Z == a.spec[sp] ? sp * VT_N : base;
     }
-    sa[q] = make_float4(a.bx[src], a.by[src], a.bz[src], __int_as_float(base * (int)sizeof(float4) - VT_ZERO));
+    const float x = a.bx[src], y = a.by[src], z = a.bz[src];
+    // a position that is no number is put out of every patch's reach: it is at
+    // no distance below the cutoff (the patch test and the table's clamp would
+    // take it for one at the centre)
+    const bool num = x == x && y == y && (KIND == POT_PROJECTED || z == z);
+    sa[q] = make_float4(num ? x : 1e18f, y, z, __int_as_float(base * (int)sizeof(float4) - VT_ZERO));
   };
   auto sum_chunk = [&](int cn) {
     auto atoms = [&](auto tab) {
