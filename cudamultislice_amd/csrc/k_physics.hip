@@ -170,8 +170,10 @@ constexpr int VT_N = 6 * VT_OCT + VT_OCT / 4 + 1;    // [1/16, 4), [4, 5), zeros
 constexpr int VT_FIRST = 0x3D800000 >> VT_SHIFT;     // 1/16
 constexpr float VT_LO = 0.0625f, VT_HI = 5.0f;
 
-// Abramowitz & Stegun 9.8.1-9.8.6 (the forms of U.cu:41-111)
+// Abramowitz & Stegun 9.8.1-9.8.6 (the forms of U.cu:41-111, with their value
+// at 0: a term that a parameter file leaves out, a = b = 0, adds nothing)
 __device__ double bessk0_f64(double x) {
+  if (!(x > 0.0)) return 1.0e20;
   if (x <= 2.0) {
     double t = x / 3.75, u = x * 0.5;
     t = t * t;
