@@ -124,7 +124,11 @@ template <int DIR, bool Z = false> __host__ __device__ __forceinline__ void dft8
 
 // Z: a[4..11] = 0 on entry
 template <int DIR, bool Z = false> __host__ __device__ __forceinline__ void dft16(float2 (&a)[16]) {
-  constexpr float c1 = 0.92387953251128674f, t1 = 0.41421356237309505f;  // cos, tan of pi / 8
+  // cos and tan of pi / 8, the cosine rounded up (0.92387956, by 3.4e-8; to
+  // nearest it would be 0.9238795, down by 3.1e-8): sqrt(1/2) above is down by
+  // 1.7e-8, and as both act on every line at every slice their errors of |w|
+  // would add up (see twiddle)
+  constexpr float c1 = 0x1.d906bep-1f, t1 = 0.41421356237309505f;
   float2 e[8], o[8];
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
