@@ -11,7 +11,9 @@ namespace msl {
 // Entry k of the passes' table exp(-2 pi i k / n) = cs + i sn: (c, t) with
 // the factor c (1 + i t), the form that the butterflies take.  t is the sine
 // over the rounded c, so that c t has one rounding; where the cosine is zero
-// c is 2^-40 and c t exact.
+// c is 2^-30 and c t exact: off by 9e-10 in the real part, a thirtieth of the
+// other entries' rounding; the bracket b (1 + i t) then holds values up to
+// 2^98 (with 2^-40 it overflowed from 2^88 on).
 //
 // A line takes up to one factor per doubling of its length, and the rounding
 // errors of their moduli are the same at every slice: they add up over a run.
@@ -24,7 +26,7 @@ namespace msl {
 // 512 the one at pi / 8 is enough (252 slices of a plane wave at 1024^2:
 // 3.8e-6, with both 5.2e-6).
 __host__ __device__ inline float2 twiddle(double cs, double sn, int k, int n) {
-  if (4 * k == n || 4 * k == 3 * n) return make_float2(0x1p-40f, sn < 0 ? -0x1p40f : 0x1p40f);
+  if (4 * k == n || 4 * k == 3 * n) return make_float2(0x1p-30f, sn < 0 ? -0x1p30f : 0x1p30f);
   const float c = 32 * k == n && n <= 512 ? 0x1.f6297ep-1f : (float)cs;
   return make_float2(c, (float)(sn / (double)c));
 }

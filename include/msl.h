@@ -349,7 +349,8 @@ msl_status msl_server_run(msl_server* srv, const msl_serve_params* prm, const ms
 
 /* ---- device-array primitives (used by the torch binding and tests) ---- */
 /* batched 2D FFT of nbatch [ny][nx] complex64 device arrays, in place,
- * unnormalised; inverse != 0 for exp(+2 pi i) */
+ * unnormalised; inverse != 0 for exp(+2 pi i).  Partial sums of a line may reach
+ * 2^97 (1.6e29) in modulus; beyond, results are not finite */
 msl_status msl_fft2_device(int nx, int ny, int nbatch, void* data, int inverse, void* stream);
 /* msl_fft2_device without any device allocation, for callers that cannot
  * allocate (code under HIP graph capture, serving loops that forbid
