@@ -1234,12 +1234,22 @@ __global__ void k_transmission(const float* V, float2* t, long long n, float sig
   if (i < n) t[i] = phase_of(V[i], sigma);
 }
 hipError_t launch_transmission(const float* V, float2* t, long long n, float sigma, hipStream_t s) {
-  if (n % 4 == 0 && (uintptr_t)V % 16 == 0 && (uintptr_t)t % 16 == 0)
-    hipLaunchKernelGGL(k_transmission4, dim3(nblk(n / 4, 256)), dim3(256), 0, s, (const float4*)V, (float4*)t, n / 4,
-                       sigma);
-  else
-    hipLaunchKernelGGL(k_transmission, dim3(nblk(n, 256)), dim3(256), 0, s, V, t, n, sigma);
-  return hipGetLastError();
+  // a launch holds fewer than 2^32 threads: 2^31 values each, a multiple of
+  // four (16 GiB of transmissions)
+  constexpr long long kPiece = 1LL << 31;
+  for (long long o = 0; o < n; o += kPiece) {
+    const long long m = std::min(kPiece, n - o);
+    const float* v = V + o;
+    float2* w = t + o;
+    if (m % 4 == 0 && (uintptr_t)v % 16 == 0 && (uintptr_t)w % 16 == 0)
+      hipLaunchKernelGGL(k_transmission4, dim3(nblk(m / 4, 256)), dim3(256), 0, s, (const float4*)v, (float4*)w, m / 4,
+                         sigma);
+    else
+      hipLaunchKernelGGL(k_transmission, dim3(nblk(m, 256)), dim3(256), 0, s, v, w, m, sigma);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
 }
 
 }  // namespace msl
