@@ -410,11 +410,16 @@ void precalc(msl_sim* s) {
     if (!v.empty()) HIPC(hipMemcpyAsync(d.p, v.data(), v.size() * sizeof(v[0]), hipMemcpyHostToDevice, s->stream));
   };
   std::vector<double2> wx, cx, fx, wy, cy, fy;
+  Drain drain{s->stream, false};
   if (s->generic && s->glx.n == rx && s->gly.n == ry) {
     // the tables depend on the sides alone
   } else if (s->generic) {
     gen_tables(rx, wx, cx, fx);
     gen_tables(ry, wy, cy, fy);
+    // no sides have tables until these are up: an upload that fails may have
+    // given the old ones' memory back
+    s->glx = s->gly = GenLen{};
+    drain.on = true;
     upload(s->gtwx, wx);
     upload(s->gchx, cx);
     upload(s->gfix, fx);
@@ -434,7 +439,7 @@ void precalc(msl_sim* s) {
   HIPC(launch_ktables(s->kx.p, s->ky.p, s->twx.p, s->twy.p, rx, ry, s->ksizex, s->ksizey, s->stream));
   s->prow.ensure(rx);
   HIPC(launch_prop_rows(s->kx.p, s->ky.p, rx, ry, s->kmax, s->prow.p, s->stream));
-  if (!wx.empty()) HIPC(hipStreamSynchronize(s->stream));  // the generic tables come from host memory
+  if (drain.on) HIPC(hipStreamSynchronize(s->stream));  // the generic tables come from host memory
   s->prop_dz = std::nanf("");
   s->fd_lap = false;
   s->have_freqs = true;

@@ -53,6 +53,16 @@ template <class T> struct DBuf {
   }
 };
 
+// waits for a stream when a scope is left, by an error too: host memory
+// declared before it outlives the copies that still read it
+struct Drain {
+  hipStream_t s;
+  bool on;
+  ~Drain() {
+    if (on) (void)hipStreamSynchronize(s);
+  }
+};
+
 // a pointer into another buffer
 template <class T> struct Ptr {
   T* p = nullptr;
