@@ -718,6 +718,8 @@ msl_status msl_server_run(msl_server* srv, const msl_serve_params* prm, const ms
     // tables are those of the first job of a class.
     BinScratch scratch;
     std::vector<Job> jobs(njobs);
+    // a job that is refused leaves here with the earlier jobs' uploads under way
+    Drain drain{srv->stream, true};
     std::map<std::tuple<int, int, int>, std::vector<int>> classes;
     for (int i = 0; i < njobs; ++i) {
       const msl_job& d = jd[i];
