@@ -95,7 +95,7 @@ class Runner {
     for (int j : ids) probes = probes || jobs_[j].d->nprobe > 0;
     if (probes) probe_norm();
     else scratch_.ensure(np_);
-    const long long budget = p_.budget_bytes > 0 ? p_.budget_bytes : (32LL << 30);
+    const long long budget = this->budget();
     const long long wave_b = np_ * 8 * (fd ? 5 : 1), slot_b = np_ * 8 * (fd ? 2 : 1);
     const long long maxw = std::max<long long>(1, (budget - slot_b) / (wave_b + slot_b));
     std::vector<Item> items;
@@ -135,7 +135,7 @@ class Runner {
   // class per size; per slice one potential, one row and one column launch
   // cover every running job / wave of every size
   void run_group(const std::vector<std::pair<std::vector<int>, msl_sim*>>& classes) {
-    const long long budget = p_.budget_bytes > 0 ? p_.budget_bytes : (32LL << 30);
+    const long long budget = this->budget();
     std::vector<GItem> items;
     for (size_t c = 0; c < classes.size(); ++c) {
       msl_sim* cs = classes[c].second;
@@ -172,6 +172,7 @@ class Runner {
         ++i1;
       }
       st_.peak = std::max(st_.peak, (double)bytes);
+      buf_.fit(budget - bytes, 0, 0, 0, 0);  // a grouped batch has arrays of its own
       run_group_batch(classes, std::vector<GItem>(items.begin() + i0, items.begin() + i1));
       i0 = i1;
     }
@@ -304,6 +305,7 @@ class Runner {
   DBuf<float> red_;
 
   hipStream_t st() const { return srv_->stream; }
+  long long budget() const { return p_.budget_bytes > 0 ? p_.budget_bytes : (32LL << 30); }
 
   // sum |psi| of the probe at the origin (U.cu:2698-2705); integer shifts keep it
   void probe_norm() {
@@ -337,11 +339,23 @@ class Runner {
     Layout(DBuf<int>& t, DBuf<int>& p) : tidx(t), pos(p) {}
   };
   // device buffers of a batch, kept from one batch of a run to the next
-  // (allocating and freeing them took 14 ms of a 94 ms mix of 16 jobs)
+  // (allocating and freeing them took 14 ms of a 94 ms mix of 16 jobs) while
+  // they stay within the run's budget
   struct Buffers {
     DBuf<float2> wave[5], slot[2];
     DBuf<float> partial, adf;
     DBuf<int> tidx, pos;
+    // makes room for a batch of `waves` arrays of wn values and `slots` of sn:
+    // where those and what earlier batches left would exceed the budget, all
+    // are given back, as after a batch of its own
+    void fit(long long budget, int waves, size_t wn, int slots, size_t sn) {
+      size_t n = 0;
+      for (int i = 0; i < 5; ++i) n += std::max(wave[i].n, i < waves ? wn : 0);
+      for (int i = 0; i < 2; ++i) n += std::max(slot[i].n, i < slots ? sn : 0);
+      if ((long long)(n * sizeof(float2)) <= budget) return;
+      for (auto& b : wave) b.release();
+      for (auto& b : slot) b.release();
+    }
   } buf_;
   // one size inside a grouped batch
   struct Seg {
@@ -425,6 +439,7 @@ class Runner {
     const int J = (int)L.jobs.size();
     DBuf<float2>&W = buf_.wave[0], &T = buf_.slot[0];
     DBuf<float>&partial = buf_.partial, &adf = buf_.adf;
+    buf_.fit(budget(), 1, (size_t)L.nw * np_, 1, (size_t)J * np_);
     W.ensure((size_t)L.nw * np_);
     T.ensure((size_t)J * np_);
     partial.ensure((size_t)L.nw * ntiles_);
@@ -501,6 +516,7 @@ class Runner {
     DBuf<float2>&Pm = buf_.wave[0], &P0 = buf_.wave[1], &Pp = buf_.wave[2], &G = buf_.wave[3], &Bt = buf_.wave[4];
     DBuf<float2>&V = buf_.slot[0], &Vt = buf_.slot[1];
     DBuf<float>&partial = buf_.partial, &adf = buf_.adf;
+    buf_.fit(budget(), 5, wn, 2, (size_t)J * np_);
     Pm.ensure(wn); P0.ensure(wn); Pp.ensure(wn); G.ensure(wn); Bt.ensure(wn);
     V.ensure((size_t)J * np_); Vt.ensure((size_t)J * np_);
     partial.ensure((size_t)L.nw * ntiles_);
