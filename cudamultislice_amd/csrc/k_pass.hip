@@ -81,17 +81,37 @@ constexpr int kSmallCol = 8;  // as column 0 with SmallPlan and tiles of four co
 #ifndef MSL_PASS_LEN
 static const int kRowDefault[12] = {0, 0, 0, 0, 1, 1, 1, 1, 1, 4, 4, 4};
 static const int kColDefault[12] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 3, 0, 5};
-// variants chosen by msl_set_pass_variant or the tuner (-1: by the rules below)
-static int g_row_var[12] = {-1, -1, -1, -1, -1, -1, -1, -1, -1, -1, -1, -1};
-static int g_col_var[12] = {-1, -1, -1, -1, -1, -1, -1, -1, -1, -1, -1, -1};
+// per kind and length, -1 where there is none: the variant pinned for every
+// launch (msl_set_pass_variant) and the tuner's, which was timed on a full
+// batch and stands in for the default only where the rules below take that.
+// The default's number is no pin: it stands for the rules, so that reading a
+// variant and setting it again changes nothing.
+struct PassChoice {
+  int pin = -1, tuned = -1;
+};
+static PassChoice g_choice[2][12];
 
+static int default_variant(int kind, int l) { return kind == 0 ? kRowDefault[l] : kColDefault[l]; }
 int pass_variant(int kind, int n) {
-  const int l = lg2(n), v = kind == 0 ? g_row_var[l] : g_col_var[l];
-  return v >= 0 ? v : kind == 0 ? kRowDefault[l] : kColDefault[l];
+  const PassChoice& c = g_choice[kind][lg2(n)];
+  return c.pin >= 0 ? c.pin : c.tuned >= 0 ? c.tuned : default_variant(kind, lg2(n));
 }
 void set_pass_variant(int kind, int n, int v) {
-  if (kind == 0) g_row_var[lg2(n)] = v;
-  else g_col_var[lg2(n)] = v;
+  PassChoice& c = g_choice[kind][lg2(n)];
+  if (v == default_variant(kind, lg2(n))) c = PassChoice{};
+  else c.pin = v == c.tuned ? -1 : v;
+}
+void tune_pass_variant(int kind, int n, int v) {
+  g_choice[kind][lg2(n)] = PassChoice{-1, v == default_variant(kind, lg2(n)) ? -1 : v};
+}
+// the variant of a launch that the rules give `rule`.  Launches of one batch
+// among several (not alone) have the tuner's at every size: it may have
+// another plan, and their bits must not follow the batch.
+static int chosen_variant(int kind, int n, int rule, bool alone) {
+  const int l = lg2(n);
+  const PassChoice& c = g_choice[kind][l];
+  if (c.pin >= 0) return c.pin;
+  return c.tuned >= 0 && (!alone || rule == default_variant(kind, l)) ? c.tuned : rule;
 }
 
 // The variant of a launch of `lines` rows.  Below some thousand rows the
@@ -1327,12 +1347,14 @@ hipError_t launch_col_v(int mode, int mul, const ColArgs& a, hipStream_t s, int 
 }
 
 hipError_t launch_row(int mode, int mul, const RowArgs& a, hipStream_t s) {
-  const int v = fft_size_supported(a.nx) ? g_row_var[lg2(a.nx)] : 0;
-  return launch_row_v(mode, mul, a, s, v >= 0 ? v : auto_row(a.nx, (long long)a.nbatch * a.ny, a.alone != 0));
+  if (!fft_size_supported(a.nx)) return hipErrorInvalidValue;
+  const int rule = auto_row(a.nx, (long long)a.nbatch * a.ny, a.alone != 0);
+  return launch_row_v(mode, mul, a, s, chosen_variant(0, a.nx, rule, a.alone != 0));
 }
 hipError_t launch_col(int mode, int mul, const ColArgs& a, hipStream_t s) {
-  const int v = fft_size_supported(a.ny) ? g_col_var[lg2(a.ny)] : 0;
-  return launch_col_v(mode, mul, a, s, v >= 0 ? v : auto_col(a.ny, (long long)a.nbatch * a.nx, a.alone != 0));
+  if (!fft_size_supported(a.ny)) return hipErrorInvalidValue;
+  const int rule = auto_col(a.ny, (long long)a.nbatch * a.nx, a.alone != 0);
+  return launch_col_v(mode, mul, a, s, chosen_variant(1, a.ny, rule, a.alone != 0));
 }
 
 #endif

@@ -142,6 +142,7 @@ int band_tiles_lo(int nx);  // column tiles per end covering x < N/4, x >= 3N/4 
 // pass layout variants per length (kind 0 row, 1 column), see k_pass.hip
 int pass_variant(int kind, int n);
 void set_pass_variant(int kind, int n, int v);
+void tune_pass_variant(int kind, int n, int v);
 int num_pass_variants(int kind);
 hipError_t launch_row_v(int mode, int mul, const RowArgs& a, hipStream_t s, int var);
 hipError_t launch_col_v(int mode, int mul, const ColArgs& a, hipStream_t s, int var);

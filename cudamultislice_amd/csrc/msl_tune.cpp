@@ -181,7 +181,7 @@ msl_status msl_autotune_passes(int n, int nbatch, int reps, int* row_var, int* c
         best[kind] = v;
       }
     }
-    set_pass_variant(kind, n, best[kind]);
+    tune_pass_variant(kind, n, best[kind]);
   }
   if (row_var) *row_var = best[0];
   if (col_var) *col_var = best[1];

@@ -276,7 +276,13 @@ msl_status msl_diff_set_chunk(msl_diff* d, int probes);
  * nbatch waves and, with maxdiff, compares against variant 0;
  * msl_autotune_passes selects the fastest agreeing variant per pass for n
  * (out[16]: [0..7] row and [8..15] column timings in ms per variant, -1 where
- * rejected or absent).  Timings use band-pruned passes where the length allows. */
+ * rejected or absent).  Timings use band-pruned passes where the length allows.
+ * Until a variant is set, launches of a few waves take layouts of their own by
+ * their size and larger ones the length's default, which msl_get_pass_variant
+ * returns.  msl_set_pass_variant puts a variant in the place of all of them;
+ * set to the default's number it goes back to the rules by size, so a variant
+ * read and set again changes nothing.  The tuner's choice, timed on a batch,
+ * replaces the default and leaves the layouts of a handle's single wave. */
 msl_status msl_set_pass_variant(int kind, int n, int variant);
 msl_status msl_get_pass_variant(int kind, int n, int* variant);
 msl_status msl_bench_pass(int kind, int variant, int n, int nbatch, int reps, float* ms, float* maxdiff);
