@@ -119,9 +119,10 @@ static int chosen_variant(int kind, int n, int rule, bool alone) {
 // line, or fewer lines per workgroup); above, the layouts of the defaults.
 // Between variants of one plan (0, 1, 3; at 1024 and 2048 also 4) a line's
 // bits are the same, so the choice may follow the batch; a change of plan
-// (2, small; 4 at 512) is for callers whose batch never varies
-// (RowArgs::alone), so that a wave's result does not depend on how a run is
-// cut into batches.
+// (2, small; 4 at 512) is for runs whose waves are always the same (one
+// handle's, an engine's probes: RowArgs::alone, their number), which the rule
+// then goes by, so that a wave's result does not depend on how its run is cut
+// into batches.
 // Us per launch of IFFT -> t -> FFT (variant:time; s the small layout):
 //    64  0: 3.3 at 1 wave of n x n, 3.5 at 16; 1: 3.0, 3.2; s: 2.7, 2.8
 //   128  1: 4.2 at 1, 4.4 at 16, 4.6 at 37; 2: 3.6, 3.7, 4.6; s: 3.1, 3.3, 4.6
@@ -1348,12 +1349,12 @@ hipError_t launch_col_v(int mode, int mul, const ColArgs& a, hipStream_t s, int 
 
 hipError_t launch_row(int mode, int mul, const RowArgs& a, hipStream_t s) {
   if (!fft_size_supported(a.nx)) return hipErrorInvalidValue;
-  const int rule = auto_row(a.nx, (long long)a.nbatch * a.ny, a.alone != 0);
+  const int rule = auto_row(a.nx, (long long)(a.alone ? a.alone : a.nbatch) * a.ny, a.alone != 0);
   return launch_row_v(mode, mul, a, s, chosen_variant(0, a.nx, rule, a.alone != 0));
 }
 hipError_t launch_col(int mode, int mul, const ColArgs& a, hipStream_t s) {
   if (!fft_size_supported(a.ny)) return hipErrorInvalidValue;
-  const int rule = auto_col(a.ny, (long long)a.nbatch * a.nx, a.alone != 0);
+  const int rule = auto_col(a.ny, (long long)(a.alone ? a.alone : a.nbatch) * a.nx, a.alone != 0);
   return launch_col_v(mode, mul, a, s, chosen_variant(1, a.ny, rule, a.alone != 0));
 }
 

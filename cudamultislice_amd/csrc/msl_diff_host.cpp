@@ -80,7 +80,7 @@ RowArgs rargs(msl_diff* d, const float2* src, float2* dst, bool pin = false, boo
   a.src = src; a.dst = dst; a.src_bstride = a.dst_bstride = d->np();
   a.nx = d->nx; a.ny = d->ny; a.nbatch = d->B; a.t_group = d->B; a.t_bstride = 0; a.scale = 1.f;
   a.tw = d->twx.p; a.sigma = d->sigma;
-  a.alone = 1;
+  a.alone = d->B;
   return a;
 }
 ColArgs cargs(msl_diff* d, const float2* src, float2* dst, float scale) {
@@ -90,7 +90,7 @@ ColArgs cargs(msl_diff* d, const float2* src, float2* dst, float scale) {
   a.kmax = d->kmax; a.scale = scale; a.tw = d->twy.p; a.prop_rows = d->prow.p;
   a.tiles_lo = d->prune_tiles;
   a.zb_rows = d->zb_rows ? 1 : 0;
-  a.alone = 1;
+  a.alone = d->B;
   return a;
 }
 

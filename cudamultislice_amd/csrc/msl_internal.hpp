@@ -74,7 +74,7 @@ enum RowMul { RM_NONE = 0, RM_T = 1, RM_SEED = 2 };
   float G* inten;            /* ROW_INV: optional |wave|^2, dst indexing (dst may then be null) */        \
   int fd_vreal;              /* t holds the band-limited V in real space instead */                      \
   const float G* seed;       /* RM_SEED: real factor per element, src indexing */                        \
-  int alone;                 /* 1: the caller's batch never varies (variant rules, launch_row) */
+  int alone;                 /* waves of a run that never varies, this batch among them; else 0 (launch_row) */
 struct RowArgs {
   MSL_ROW_ARGS()
 };
