@@ -595,11 +595,15 @@ template <int V, int KIND> static hipError_t potential_v(const PotArgs& a, hipSt
   return hipGetLastError();
 }
 
+// one wave per 8 x 8 pixels leaves SIMDs (1024 on the chip) with fewer than
+// four waves each below 4096 patches: four waves then share a patch, and the
+// pixel tiles have no part in it
+bool potential_tiled(int nx, int ny, int nslices) {
+  return (long long)nblk(nx, 8) * nblk(ny, 8) * nslices >= 4096;
+}
+
 template <int KIND> static hipError_t potential_k(const PotArgs& a, hipStream_t s) {
-  // one wave per 8 x 8 pixels leaves SIMDs (1024 on the chip) with fewer than
-  // four waves each below 4096 patches: four waves then share a patch
-  const long long patches = (long long)nblk(a.nx, 8) * nblk(a.ny, 8) * a.nslices;
-  if (patches < 4096) {
+  if (!potential_tiled(a.nx, a.ny, a.nslices)) {
     hipLaunchKernelGGL(k_potential_split<KIND>, dim3(nblk(a.nx, 8), nblk(a.ny, 8), a.nslices), dim3(256),
                        pot_lds<KIND>(a), s, a);
     return hipGetLastError();

@@ -1303,7 +1303,8 @@ msl_status msl_set_potential_tile(msl_sim* s, int variant) {
 
 // Times every pixel-tile shape of the potential kernel on the handle's atoms
 // and grid (nslices slices of thickness dz, its potential mode), keeps the
-// fastest whose potentials equal the 16x16 tile's bit for bit.
+// fastest whose potentials equal the 16x16 tile's bit for bit.  Slices too few
+// for the tiles to have a part in their launch leave the shape as it is.
 msl_status msl_autotune_potential(msl_sim* s, float dz, int nslices, int* best, float* ms_per_variant) {
   API_BEGIN(s)
   require(s->have_freqs, MSL_ERR_STATE, "PreCalculateFrequencies first");
@@ -1346,8 +1347,8 @@ msl_status msl_autotune_potential(msl_sim* s, float dz, int nslices, int* best, 
   }
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
-  s->pot_tile = pick;
-  if (best) *best = pick;
+  s->pot_tile = potential_tiled(s->resX, s->resY, nslices) ? pick : saved;
+  if (best) *best = s->pot_tile;
   API_END(s)
 }
 

@@ -270,6 +270,8 @@ hipError_t launch_potential(const PotArgs& a, hipStream_t s);
 // workgroup of each job, job j owning potential_tiles(nx, ny) workgroups; mode (0 or 1) is every job's
 int potential_tiles(int nx, int ny);
 int potential_tile_variants();
+// whether a launch of nslices slices takes PotArgs::tile (small ones do not)
+bool potential_tiled(int nx, int ny, int nslices);
 hipError_t launch_potential_group(const PotArgs* tab, const long long* blk0, int njobs, long long nblocks, int first,
                                   int mode, hipStream_t s);
 // radial tables of every species from the 103 x 12 parameters (device)

@@ -372,7 +372,9 @@ msl_status msl_fft2_device_noalloc(int nx, int ny, int nbatch, void* data, int i
  * each on the handle's binned atoms and grid (nslices slices of thickness
  * dz from the top) and keeps the fastest whose potentials equal the 16x16
  * tile's; ms_per_variant (optional, 4 floats) gets the times (-1 where
- * rejected). */
+ * rejected).  Launches below 4096 patches of 8 x 8 pixels (all slices of the
+ * launch) share each patch between four waves and take no tile: with so few
+ * slices the tuner leaves the tile as it is. */
 msl_status msl_set_potential_tile(msl_sim* sim, int variant);
 msl_status msl_autotune_potential(msl_sim* sim, float dz, int nslices, int* best, float* ms_per_variant);
 /* bin / potential on device arrays held by a handle (debug access) */
