@@ -287,23 +287,22 @@ template <int M, bool BLUE> __global__ void __launch_bounds__(GenRow<M>::THREADS
   }
 }
 
-// k-space factor of column x, row y (ColMul, scale included): CM_PROP /
-// CM_PROPCONJ the Fresnel propagator px[x] py[y] inside |k| < kmax
-// (CreatePropsKernel, U.cu:419), CM_BAND the band limit |k| <= kmax
-// (BandLimitKernel, U.cu:1037-1040), CM_GRAD -4 pi^2 k^2 (gradKernel,
-// U.cu:959-960, pi = 3.14159f), CM_BANDGRAD both, CM_SCALE the scale only
+// k-space factor of column x, row y (ColMul, scale included): CM_PROP the
+// Fresnel propagator px[x] py[y] inside |k| < kmax (CreatePropsKernel,
+// U.cu:419), CM_BAND the band limit |k| <= kmax (BandLimitKernel,
+// U.cu:1037-1040), CM_GRAD -4 pi^2 k^2 (gradKernel, U.cu:959-960, pi =
+// 3.14159f), CM_SCALE the scale only
 __device__ __forceinline__ double2 gen_factor(const GenColArgs& a, int x, int y) {
   if (a.mul == CM_SCALE) return make_double2(a.scale, 0.0);
   const float kxv = a.kx[x], kyv = a.ky[y];
   const float k = sqrtf(kxv * kxv + kyv * kyv);
-  if (a.mul == CM_PROP || a.mul == CM_PROPCONJ) {
+  if (a.mul == CM_PROP) {
     const double2 p = mul(wide(a.px[x]), wide(a.py[y]));
     const double m = k < a.kmax ? a.scale : 0.0;
-    return make_double2(p.x * m, (a.mul == CM_PROPCONJ ? -p.y : p.y) * m);
+    return make_double2(p.x * m, p.y * m);
   }
-  const float gr = -4.f * 3.14159f * 3.14159f * (kxv * kxv + kyv * kyv);
-  if (a.mul == CM_GRAD) return make_double2(a.scale * gr, 0.0);
-  return make_double2(k <= a.kmax ? (a.mul == CM_BAND ? a.scale : a.scale * gr) : 0.0, 0.0);
+  if (a.mul == CM_GRAD) return make_double2(a.scale * (-4.f * 3.14159f * 3.14159f * (kxv * kxv + kyv * kyv)), 0.0);
+  return make_double2(k <= a.kmax ? a.scale : 0.0, 0.0);
 }
 
 template <int M> struct GenCol {
@@ -449,8 +448,9 @@ hipError_t launch_gen_row(const GenRowArgs& a, hipStream_t s) {
 hipError_t launch_gen_col(const GenColArgs& a, hipStream_t s) {
   if (!a.src || !a.dst || a.nx < 1 || a.nbatch < 0 || !len_ok(a.len, a.ny)) return hipErrorInvalidValue;
   if (a.mode != COL_FWD && a.mode != COL_INV && a.mode != COL_FWD_MUL_INV) return hipErrorInvalidValue;
+  if (a.mul != CM_SCALE && a.mul != CM_PROP && a.mul != CM_BAND && a.mul != CM_GRAD) return hipErrorInvalidValue;
   if (a.mul != CM_SCALE && (!a.kx || !a.ky)) return hipErrorInvalidValue;
-  if ((a.mul == CM_PROP || a.mul == CM_PROPCONJ) && (!a.px || !a.py)) return hipErrorInvalidValue;
+  if (a.mul == CM_PROP && (!a.px || !a.py)) return hipErrorInvalidValue;
   const long long np = (long long)a.nx * a.ny;
   for (int b0 = 0; b0 < a.nbatch; b0 += 65535) {  // waves on grid.y
     GenColArgs c = a;

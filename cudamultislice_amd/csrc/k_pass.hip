@@ -807,10 +807,12 @@ __global__ void __launch_bounds__((ColCfg<N, CV>::THREADS), (ColCfg<N, CV>::MIN_
 // Variant 5, for the propagation pass (FFT_y -> P -> IFFT_y): a workgroup
 // owns one column tile and loops over per_tile waves of the batch; each
 // thread forms its propagator factors once (the other layouts load and form
-// them again for every wave).  Tile, plan and LDS layout of the length's
-// default variant (7 at 512, 0 otherwise), held to four waves per SIMD (112
-// VGPRs at 512).  Requesting the next wave's tile during the transforms as
-// well took 174 VGPRs, two waves per SIMD, and ran slower than variant 7.
+// them again for every wave: rounding of the factors differs, 2.5e-7 of a
+// wave after three slices).  Tile, plan and LDS layout of variant 7 at 512, of
+// 0 otherwise, held to four waves per SIMD (112 VGPRs at 512).  Requesting the
+// next wave's tile during the transforms as well took 174 VGPRs, two waves per
+// SIMD, and ran slower than variant 7.  The default at 2048 alone; a launch of
+// one wave takes variant 0.
 template <int N> struct ColPL { static constexpr int CV = N == 512 ? 7 : 0; };
 
 template <int N, int MUL>
