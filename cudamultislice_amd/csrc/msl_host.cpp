@@ -404,7 +404,7 @@ void precalc(msl_sim* s) {
   s->fd_zb = band_rows_quarter(s->hky.data(), ry, s->kmax);
   // (a grid of 2048 x 512 or less counts more of the band's tiles than its
   // column pass has: its finite differences run unpruned)
-  s->fd_prune = s->prune_tiles > 0 && 2 * s->prune_tiles <= rx / col_tile(ry);
+  s->fd_prune = !s->generic && s->prune_tiles > 0 && 2 * s->prune_tiles <= rx / col_tile(ry);
   for (int x = rx / 4; x < 3 * rx / 4 && s->fd_prune; ++x)
     if (std::sqrt(s->hkx[x] * s->hkx[x] + 0.0f) <= s->kmax) s->fd_prune = false;
   auto upload = [&](auto& d, const auto& v) {

@@ -1,4 +1,5 @@
-"""Finite-difference steps on grids much wider than high."""
+"""Finite-difference steps on grids much wider than high, and of a power of two
+beside another side."""
 import numpy as np
 import pytest
 
@@ -9,7 +10,8 @@ from oracle import oracle as O
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("nx,ny", [(2048, 16), (2048, 512), (2048, 1024), (1024, 16), (16, 1024)])
+@pytest.mark.parametrize("nx,ny", [(2048, 16), (2048, 512), (2048, 1024), (1024, 16), (16, 1024),
+                                   (256, 60), (60, 256)])
 def test_steps_match_the_oracle(fp, nx, ny):
     Z, x, y, z = S.silicon(2, 2, 2)
     with MultisliceSimulation() as g:
