@@ -1582,7 +1582,9 @@ extern "C" msl_status msl_stem_batched(msl_sim* s, const msl_stem_batch_desc* d)
     if (!(std::sqrt(s->hkx[x] * s->hkx[x]) > apert * 1.0001f)) probe_in_band = false;
   const int band_cols = probe_in_band ? nx / 4 : 0;
   // detector tiles per probe: the |Psi|^2 map needs every column written
-  const int det_tiles = (prune && !d->pacbed_out) ? 2 * s->prune_tiles : ntiles;
+  // (the band's tiles in those of the detector pass: prune_tiles counts in the
+  // tiles of a column as long as the rows)
+  const int det_tiles = (prune && !d->pacbed_out) ? 2 * (nx / 4 / C) : ntiles;
   // One chunk of nb probes whose positions are in pos: probe synthesis, the
   // slice loop and the fused detector.  Every pointer it uses is fixed for
   // the whole call, so the sequence can be captured once per chunk size and
