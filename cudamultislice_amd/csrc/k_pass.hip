@@ -76,7 +76,8 @@ constexpr int kSmallCol = 8;  // as column 0 with SmallPlan and tiles of four co
 // 143, 3 142; 1024, 32 waves: 4 70, 1 76, 3 78; 2048, 32 waves: 4 363, 3 367, 2
 // 372, 1 379); 256 and below variant 1.  Columns: 512 half-width tiles (with
 // the row factors in LDS 68.0 per 256 waves, 69.2 on the alternative plan, 78
-// full width); 2048 the loop over waves (32 waves: 5 338, 0 420); 1024 full
+// full width, one launch repeated; in whole runs 80 to 84 and the first two
+// equal); 2048 the loop over waves (32 waves: 5 338, 0 420); 1024 full
 // width (32 waves: 0 49.2, 3 50.8, 5 52.6); 256 and below variant 0.
 #ifndef MSL_PASS_LEN
 static const int kRowDefault[12] = {0, 0, 0, 0, 1, 1, 1, 1, 1, 4, 4, 4};
